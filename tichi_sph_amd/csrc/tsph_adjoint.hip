@@ -39,16 +39,11 @@ __device__ __forceinline__ D2<T> kern_d2(const KP<T>& k, T r2) {
   T u = T(1) - q;
   D2<T> d;
   d.r = r;
-  if (q <= T(0.5)) {
-    d.g = k.wg_a * (T(3) * q - T(2));
-    d.w2 = k.wg_a * (T(6) * q - T(2));
-  } else if (q < T(1)) {
-    d.g = -k.wg_b * (u * u) * rinv;
-    d.w2 = T(2) * k.wg_a * u;
-  } else {
-    d.g = T(0);
-    d.w2 = T(0);
-  }
+  const bool in = q <= T(0.5), out = q < T(1);
+  const T ga = k.wg_a * (T(3) * q - T(2)), gb = -k.wg_b * (u * u) * rinv;
+  const T wa = k.wg_a * (T(6) * q - T(2)), wb = T(2) * k.wg_a * u;
+  d.g = in ? ga : (out ? gb : T(0));
+  d.w2 = in ? wa : (out ? wb : T(0));
   d.hq = (d.w2 - d.g) * (rinv * rinv);
   return d;
 }
@@ -245,11 +240,13 @@ __global__ void __launch_bounds__(kBlock)
   BoundSums<T> bs{};
   if (hb) bs = load_bound_sums(bmom, cap, i);
   T kb = 0, ax = 0, ay = 0, az = 0;
-  auto term = [&](const Rec2<T>& d) {  // a fluid neighbour j
+  auto term = [&](const Rec2<T>& d, bool ok) {  // a fluid neighbour j
     const V4<T>& q = d.a;   // q.w = X_j = m_j
     const V4<T>& uj = d.b;  // xyz = u_j, w = kappa_j
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
+    e.g = ok ? e.g : T(0);
+    e.hq = ok ? e.hq : T(0);
     T rmj = f_rcp(q.w);  // hardware reciprocal in FP32 (the reverse is not a bit-exact sum)
     T mx = wx - uj.x * rmj, my = wy - uj.y * rmj, mz = wz - uj.z * rmj;
     kb += q.w * e.g * (dx * mx + dy * my + dz * mz);
@@ -261,7 +258,7 @@ __global__ void __launch_bounds__(kBlock)
   sweep_lists_coop<kCoopR, T, Rec2<T>>(
       k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0,
       [&](int j) { return Rec2<T>{fpos[j], vbar[j]}; }, [&](int) { return Rec2<T>{}; },
-      term, [&](const Rec2<T>&) {});
+      term, [&](const Rec2<T>&, bool) {});
   kb = group_sum<kCoopR>(kb);
   ax = group_sum<kCoopR>(ax);
   ay = group_sum<kCoopR>(ay);
@@ -316,11 +313,13 @@ __global__ void __launch_bounds__(kBlock)
   BoundSums<T> bs{};
   if (hb) bs = load_bound_sums(bmom, cap, i);
   T vx = 0, vy = 0, vz = 0, ax = 0, ay = 0, az = 0;
-  auto term = [&](const Rec2<T>& d) {
+  auto term = [&](const Rec2<T>& d, bool ok) {
     const V4<T>& q = d.a;   // q.w = X_j
     const V4<T>& vj = d.b;  // xyz = vel_adv_j, w = psib_j
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
+    e.g = ok ? e.g : T(0);
+    e.hq = ok ? e.hq : T(0);
     T c = pbi * q.w + vj.w * Xi;
     T cg = c * e.g;
     vx += cg * dx;
@@ -333,7 +332,7 @@ __global__ void __launch_bounds__(kBlock)
   sweep_lists_coop<kCoopR, T, Rec2<T>>(
       k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0,
       [&](int j) { return Rec2<T>{fpos[j], tvel[j]}; }, [&](int) { return Rec2<T>{}; }, term,
-      [&](const Rec2<T>&) {});
+      [&](const Rec2<T>&, bool) {});
   vx = group_sum<kCoopR>(vx);
   vy = group_sum<kCoopR>(vy);
   vz = group_sum<kCoopR>(vz);
@@ -442,8 +441,8 @@ __global__ void __launch_bounds__(kBlock)
       });
       // cohesion, per in-range neighbour: (x_j, X_j = m_j) as well
       auto loadc = [&](int j) { return Rec3<T>{fpos[j], tnormal[j], brec[j]}; };
-      auto coh = [&](const Rec3<T>& d) {
-        if (!(d.b.w > T(0))) return;
+      auto coh = [&](const Rec3<T>& d, bool ok) {
+        if (!ok || !(d.b.w > T(0))) return;
         const V4<T>& q = d.a;
         const V4<T>& bj = d.c;
         const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
@@ -476,7 +475,7 @@ __global__ void __launch_bounds__(kBlock)
         walk_cells(k, fstart, c, [&](int j) {
           const V4<T> q = fpos[j];
           const T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
-          if (r2 > T(0) && r2 <= k.r2max) coh(loadc(j));
+          if (r2 > T(0) && r2 <= k.r2max) coh(loadc(j), true);
         });
       }
     }
@@ -555,7 +554,7 @@ __global__ void __launch_bounds__(kBlock)
     const T rb0 = rhobar[i], di = dens[i];
     const V4<T> xb = xbar[i];
     T vbx = 0, vby = 0, vbz = 0, xbx = 0, xby = 0, xbz = 0, Vb = 0, ms = 0;
-    auto term = [&](const Rec4<T>& d) {
+    auto term = [&](const Rec4<T>& d, bool ok) {
       const V4<T>& q = d.a;   // position
       const V4<T>& vj = d.b;  // velocity, w = V_j
       const V4<T>& aj = d.c;  // a_bar_j, w = fv_j
@@ -563,6 +562,8 @@ __global__ void __launch_bounds__(kBlock)
       T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       T r2 = dx * dx + dy * dy + dz * dz;
       D2<T> e = kern_d2(k, r2);
+      e.g = ok ? e.g : T(0);
+      e.hq = ok ? e.hq : T(0);
       T den = k.eps + r2;
       T rden = f_rcp(den);
       T w = e.g * rden;
@@ -597,7 +598,7 @@ __global__ void __launch_bounds__(kBlock)
           // tvel.w = V_j; arec = (dt u_j, fv_j)
           return Rec4<T>{fpos[j], tvel[j], arec[j], nbar ? nbar[j] : V4<T>{}};
         },
-        [&](int j) { return Rec4<T>{}; }, term, [&](const Rec4<T>&) {});
+        [&](int j) { return Rec4<T>{}; }, term, [&](const Rec4<T>&, bool) {});
     vbx = group_sum<kCoopR>(vbx);
     vby = group_sum<kCoopR>(vby);
     vbz = group_sum<kCoopR>(vbz);
@@ -684,12 +685,14 @@ __global__ void __launch_bounds__(kBlock)
         return Rec4<T>{q, a1bar[j], extra, V4<T>{}};
       },
       [&](int) { return Rec4<T>{}; },
-      [&](const Rec4<T>& d) {
+      [&](const Rec4<T>& d, bool ok) {
         const V4<T>& q = d.a;
         const V4<T>& abj = d.b;
         const T rbj = d.c.x, mj = d.c.y;
         T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
+        e.g = ok ? e.g : T(0);
+        e.hq = ok ? e.hq : T(0);
         T cd = (rbi * mj + rbj * mi) * e.g;
         T c2 = T(2) * e.g * e.w2 * (abi.w * q.w * q.w * f_rcp(mj) + abj.w * xm_i);
         T s1 = cd + c2;
@@ -699,7 +702,7 @@ __global__ void __launch_bounds__(kBlock)
         add_J(ax, ay, az, e, dx, dy, dz, q.w * abi.x - Xi * abj.x, q.w * abi.y - Xi * abj.y,
               q.w * abi.z - Xi * abj.z);
       },
-      [&](const Rec4<T>&) {});
+      [&](const Rec4<T>&, bool) {});
   ax = group_sum<kCoop>(ax);
   ay = group_sum<kCoop>(ay);
   az = group_sum<kCoop>(az);

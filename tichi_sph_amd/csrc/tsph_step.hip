@@ -459,14 +459,14 @@ __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n
     const T pr = psi_rho[i];
     const T al = alpha[i];
     T sum = 0;  // this lane's share of sum_j X_j (v_i - v_j) . grad W_ij
-    auto term = [&](const Rec2<T>& d) {
+    auto term = [&](const Rec2<T>& d, bool ok) {
       const V4<T>& q = d.a;
       const V4<T>& vj = d.b;
       T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       T r2 = dx * dx + dy * dy + dz * dz, r;
       T g = f_grad(k, r2, &r);
       T dot = (dx * (va.x - vj.x) + dy * (va.y - vj.y) + dz * (va.z - vj.z)) * g;
-      sum += dot * q.w;
+      sum += (ok ? dot : T(0)) * q.w;
     };
     // (f,f) pairs from the list; the (f,b) pairs have v_j = 0 (boundary
     // vel_adv is never written), so their sum is v_i . sum_b X_j grad W_ij,
@@ -474,7 +474,7 @@ __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n
     sweep_lists_coop<kCoop, T, Rec2<T>>(
         k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
         [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
-        [&](int) { return Rec2<T>{}; }, term, [&](const Rec2<T>&) {});
+        [&](int) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
     sum = group_sum<kCoop>(sum);
     if (c != 0) continue;
     sum += va.x * B.x + va.y * B.y + va.z * B.z;
@@ -571,11 +571,11 @@ __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, in
     const V4<T> p = fpos[i];
     const T Xi = p.w;
     T sx = 0, sy = 0, sz = 0;  // this lane's share of sum_j kappa_j grad W_ij
-    auto term = [&](const V4<T>& q) {  // q = (x_j, kappa_j)
+    auto term = [&](const V4<T>& q, bool ok) {  // q = (x_j, kappa_j)
       T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       T r2 = dx * dx + dy * dy + dz * dz, r;
       T g = f_grad(k, r2, &r);
-      T s = q.w * g;
+      T s = ok ? q.w * g : T(0);
       sx += s * dx;
       sy += s * dy;
       sz += s * dz;
@@ -583,7 +583,7 @@ __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, in
     sweep_lists_coop<kCoopU, T, V4<T>>(
         k, cap, i, cl, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
         [&](int j) { return krec[j]; }, [&](int) { return V4<T>{}; }, term,
-        [&](const V4<T>&) {});
+        [&](const V4<T>&, bool) {});
     sx = group_sum<kCoopU>(sx);
     sy = group_sum<kCoopU>(sy);
     sz = group_sum<kCoopU>(sz);
@@ -637,7 +637,7 @@ __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, in
     const V4<T> vi = vadv[i];
     const T fvis = k.two_d2 * mu_of(k, vf, i) / rdens[i];
     T ax = 0, ay = 0, az = 0, nx = 0, ny = 0, nz = 0;  // this lane's share
-    auto term = [&](const Rec2<T>& d) {
+    auto term = [&](const Rec2<T>& d, bool ok) {
       const V4<T>& q = d.a;
       const V4<T>& vj = d.b;
       T Vj = vj.w;  // V_j = X_j / sph_psi_j rides in vel_adv's 4th lane (pass A)
@@ -646,10 +646,11 @@ __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, in
       T g = f_grad(k, r2, &r);
       T Ax = (vi.x - vj.x) * dx + (vi.y - vj.y) * dy + (vi.z - vj.z) * dz;
       T s = fvis * Vj * g * Ax * f_rcp(k.eps + r2);  // W_lap, sph_util.py:40-43 (fast quotient)
+      s = ok ? s : T(0);
       ax += s * dx;
       ay += s * dy;
       az += s * dz;
-      T t = -Vj * g;  // normal, sph.py:149
+      T t = ok ? -Vj * g : T(0);  // normal, sph.py:149
       nx += t * dx;
       ny += t * dy;
       nz += t * dz;
@@ -658,7 +659,7 @@ __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, in
     sweep_lists_coop<kCoop, T, Rec2<T>>(
         k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
         [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
-        [&](int j) { return Rec2<T>{}; }, term, [&](const Rec2<T>&) {});
+        [&](int j) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
     ax = group_sum<kCoop>(ax);
     ay = group_sum<kCoop>(ay);
     az = group_sum<kCoop>(az);
@@ -967,8 +968,8 @@ __global__ void __launch_bounds__(kBlock)
       d.V = vx ? d.x.w : rvol[j];
       return d;
     };
-    auto pair = [&](const FbmRec<T, NP>& d) {
-      if (d.u[0].w < T(0)) return;  // a flagged neighbour
+    auto pair = [&](const FbmRec<T, NP>& d, bool ok) {
+      if (!ok || d.u[0].w < T(0)) return;  // no neighbour, or a flagged one
       const T dx = p.x - d.x.x, dy = p.y - d.x.y, dz = p.z - d.x.z;
       const T r2 = dx * dx + dy * dy + dz * dz;
       T r;
@@ -987,7 +988,7 @@ __global__ void __launch_bounds__(kBlock)
     };
     sweep_lists_coop<kCoop, T, FbmRec<T, NP>>(
         k, cap, i, c, p, fstart, fstart, fpos, fpos, nbr_f, nullptr, nbr_nf[i], 0, load, load,
-        pair, [&](const FbmRec<T, NP>&) {});
+        pair, [&](const FbmRec<T, NP>&, bool) {});
 #pragma unroll
     for (int s = 0; s < NP; ++s) {
       conv[s] = group_sum<kCoop>(conv[s]);
