@@ -218,13 +218,10 @@ __global__ void __launch_bounds__(kBlock)
                 const int* __restrict__ nbr_nf, const V4<T>* __restrict__ bmom,
                 const int* __restrict__ bflag, V4<T>* __restrict__ tvel, T* __restrict__ rhobar,
                 T* __restrict__ alphabar, V4<T>* __restrict__ xbar, const TsphControl* ctrl) {
-  const int base = xcd_block(blockIdx.x, gridDim.x) * kBlock;
+  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  if (i >= n) return;
   const int cl = coop_lane<kCoopR>();
   const T dt = (T)ctrl->dt;
-#pragma unroll 1
-  for (int round = 0; round < kCoopR; ++round) {
-  const int i = coop_particle<kCoopR>(base, round);
-  if (i >= n) break;
   const V4<T> p = fpos[i];
   const T Xi = p.w;
   const V4<T> u = vbar[i];
@@ -263,7 +260,7 @@ __global__ void __launch_bounds__(kBlock)
   ax = group_sum<kCoopR>(ax);
   ay = group_sum<kCoopR>(ay);
   az = group_sum<kCoopR>(az);
-  if (cl != 0) continue;
+  if (cl != 0) return;
   if (hb) {
     kb += bs.dot_A(wx, wy, wz);
     bs.add_M(ax, ay, az, ki * wx, ki * wy, ki * wz);
@@ -275,7 +272,6 @@ __global__ void __launch_bounds__(kBlock)
   rhobar[i] = rb0 + pb;
   alphabar[i] = ab0 + -kb * ki / al;
   xbar[i] = v4(xb.x + s * ax, xb.y + s * ay, xb.z + s * az);
-  }
 }
 
 // Jacobi iteration reverse, half 2: IPPE_adv_psi (sph.py:202-216)
@@ -293,13 +289,10 @@ __global__ void __launch_bounds__(kBlock)
               const int* __restrict__ nbr_f, const int* __restrict__ nbr_nf,
               const V4<T>* __restrict__ bmom, const int* __restrict__ bflag,
               V4<T>* __restrict__ vbar_out, V4<T>* __restrict__ xbar, const TsphControl* ctrl) {
-  const int base = xcd_block(blockIdx.x, gridDim.x) * kBlock;
+  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  if (i >= n) return;
   const int cl = coop_lane<kCoopR>();
   const T dt = (T)ctrl->dt;
-#pragma unroll 1
-  for (int round = 0; round < kCoopR; ++round) {
-  const int i = coop_particle<kCoopR>(base, round);
-  if (i >= n) break;
   const V4<T> p = fpos[i];
   const T Xi = p.w;
   const V4<T> vi = tvel[i];  // w = psi_bar of this particle
@@ -339,7 +332,7 @@ __global__ void __launch_bounds__(kBlock)
   ax = group_sum<kCoopR>(ax);
   ay = group_sum<kCoopR>(ay);
   az = group_sum<kCoopR>(az);
-  if (cl != 0) continue;
+  if (cl != 0) return;
   if (hb) {
     vx += pbi * bs.m0.x;
     vy += pbi * bs.m0.y;
@@ -348,7 +341,6 @@ __global__ void __launch_bounds__(kBlock)
   }
   vbar_out[i] = v4(u.x + dt * vx, u.y + dt * vy, u.z + dt * vz, kn);
   xbar[i] = v4(xb.x + dt * ax, xb.y + dt * ay, xb.z + dt * az);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -532,13 +524,10 @@ __global__ void __launch_bounds__(kBlock)
                     V4<T>* __restrict__ xbar, double* __restrict__ partial,
                     const TsphControl* ctrl) {
   __shared__ double lds[kWaves];
-  const int base = xcd_block(blockIdx.x, gridDim.x) * kBlock;
+  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   const int cl = coop_lane<kCoopR>();
   double msum = 0;
-#pragma unroll 1
-  for (int round = 0; round < kCoopR; ++round) {
-    const int i = coop_particle<kCoopR>(base, round);
-    if (i >= n) break;
+  if (i < n) {
     const T dt = (T)ctrl->dt;
     const V4<T> p = fpos[i];
     const V4<T> vi = tvel[i];
@@ -607,13 +596,14 @@ __global__ void __launch_bounds__(kBlock)
     xbz = group_sum<kCoopR>(xbz);
     Vb = group_sum<kCoopR>(Vb);
     ms = group_sum<kCoopR>(ms);
-    if (cl != 0) continue;
-    vbar_out[i] = v4(ui.x + vbx, ui.y + vby, ui.z + vbz, kn);
-    // V_i = X_i / psi_i enters only pair terms; a particle outside the grid
-    // (psi_i = 0, V_i infinite) has none, so there is nothing to carry back
-    rhobar[i] = di > T(0) ? rb0 + -Vb * Vi / di : rb0;
-    xbar[i] = v4(xb.x + xbx, xb.y + xby, xb.z + xbz);
-    msum += (double)ms;
+    if (cl == 0) {
+      vbar_out[i] = v4(ui.x + vbx, ui.y + vby, ui.z + vbz, kn);
+      // V_i = X_i / psi_i enters only pair terms; a particle outside the grid
+      // (psi_i = 0, V_i infinite) has none, so there is nothing to carry back
+      rhobar[i] = di > T(0) ? rb0 + -Vb * Vi / di : rb0;
+      xbar[i] = v4(xb.x + xbx, xb.y + xby, xb.z + xbz);
+      msum += (double)ms;
+    }
   }
   double s = block_sum(msum, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
@@ -658,12 +648,9 @@ __global__ void __launch_bounds__(kBlock)
                  const int* __restrict__ nbr_f, const int* __restrict__ nbr_nf,
                  const V4<T>* __restrict__ bmom, const int* __restrict__ bflag,
                  V4<T>* __restrict__ xbar) {
-  const int base = xcd_block(blockIdx.x, gridDim.x) * kBlock;
+  const int i = coop_particle<kCoop>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  if (i >= n) return;
   const int cl = coop_lane<kCoop>();
-#pragma unroll 1
-  for (int round = 0; round < kCoop; ++round) {
-  const int i = coop_particle<kCoop>(base, round);
-  if (i >= n) break;
   const V4<T> p = fpos[i];
   const T Xi = p.w, mi = fmass[i];
   const T rbi = rhobar[i];
@@ -706,7 +693,7 @@ __global__ void __launch_bounds__(kBlock)
   ax = group_sum<kCoop>(ax);
   ay = group_sum<kCoop>(ay);
   az = group_sum<kCoop>(az);
-  if (cl != 0) continue;
+  if (cl != 0) return;
   if (hb) {
     ax += rbi * bs.m0.x;
     ay += rbi * bs.m0.y;
@@ -714,7 +701,6 @@ __global__ void __launch_bounds__(kBlock)
     bs.add_M(ax, ay, az, abi.x, abi.y, abi.z);
   }
   xbar[i] = v4(xb.x + ax, xb.y + ay, xb.z + az);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -750,14 +736,15 @@ int adj_solver_iteration(const TsphParams& prm, TsphObject* f, TsphObject* b, Ts
   (void)wsb;
   KP<T> k = make_kp<T>(prm);
   if (f->n == 0) return 0;
-  int nb = blocks_for(f->n);
   (void)b;  // the boundary enters through the boundary sums
-  hipLaunchKernelGGL(k_adj_kappa<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+  hipLaunchKernelGGL(k_adj_kappa<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
+                     f->n, f->capacity,
                      (const V4<T>*)f->pos, (const T*)f->alpha, (const V4<T>*)a->vbar,
                      f->cell_start, f->nbr_f, f->nbr_nf, (const V4<T>*)a->bmom, a->bflag,
                      (V4<T>*)a->tape_vel_adv, (T*)a->rhobar, (T*)a->alphabar, (V4<T>*)a->xbar,
                      ctrl);
-  hipLaunchKernelGGL(k_adj_vel<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+  hipLaunchKernelGGL(k_adj_vel<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
+                     f->n, f->capacity,
                      (const V4<T>*)f->pos, (const V4<T>*)a->tape_vel_adv, (const V4<T>*)a->vbar,
                      (const T*)a->kappa_next, f->cell_start, f->nbr_f, f->nbr_nf,
                      (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->vbar_out, (V4<T>*)a->xbar,
@@ -795,14 +782,16 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
   // (pass A's output for the forward psi sweeps, free during a reverse)
   hipLaunchKernelGGL(k_adj_vis_rec<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                      (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.a1b, ctrl);
-  hipLaunchKernelGGL(k_adj_viscosity<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+  hipLaunchKernelGGL(k_adj_viscosity<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
+                     f->n, f->capacity,
                      (const V4<T>*)f->pos, (const T*)f->sph_density,
                      (const T*)f->rest_density, f->cell_start, (const int*)nullptr,
                      (const V4<T>*)nullptr, f->nbr_f, f->nbr_nf, (const V4<T>*)a->tape_vel,
                      (const V4<T>*)a->nbar, (const V4<T>*)a->vbar, (const V4<T>*)L.a1b,
                      (const T*)a->kappa_next,
                      (V4<T>*)a->vbar_out, (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
-  hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial, nb, a->grad, 0);
+  hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
+                     coop_blocks<kCoopR>(f->n), a->grad, 0);
   TSPH_LAUNCH_CHECK("adj_advect");
   return 0;
 }
@@ -816,7 +805,8 @@ int adj_density_alpha(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphA
   hipLaunchKernelGGL(k_adj_alpha_prep<T>, dim3(nb), dim3(kBlock), 0, st, f->n, (const T*)f->alpha,
                      (const V4<T>*)f->alpha_1, (const T*)f->mass, (const T*)a->alphabar,
                      (V4<T>*)a->a1bar);
-  hipLaunchKernelGGL(k_adj_pass_a<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+  hipLaunchKernelGGL(k_adj_pass_a<T>, dim3(coop_blocks<kCoop>(f->n)), dim3(kBlock), 0, st, k,
+                     f->n, f->capacity,
                      (const V4<T>*)f->pos, (const T*)f->mass, (const T*)a->rhobar,
                      (const V4<T>*)a->a1bar, f->cell_start, f->nbr_f, f->nbr_nf,
                      (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->xbar);

@@ -428,7 +428,7 @@ __global__ void k_solver_begin(KP<T> k, TsphControl* ctrl, int solve, int* signa
 
 // Jacobi half-step P: IPPE_adv_psi_init + IPPE_adv_psi (f,f)(f,b) +
 // IPPE_psi_adv_non_negative (sph.py:196-226) for iteration kk of the solve.
-template <class T>
+template <class T, int R = 1>
 __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n, int cap, int kk, const V4<T>* __restrict__ fpos,
                  const V4<T>* __restrict__ vadv, const T* __restrict__ psi_rho,
                  const T* __restrict__ rdens, const T* __restrict__ alpha,
@@ -440,61 +440,70 @@ __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n
                  V4<T>* __restrict__ tape_v, T* __restrict__ tape_k,
                  const T* __restrict__ clamp_ref,
                  double* __restrict__ partial, TsphControl* ctrl) {
-  __shared__ double lds[kWaves];
+  __shared__ double lds[R][kWaves];
   if (!ctrl->run_u[kk]) return;
-  const int base = xcd_block(blk.b, blk.nb) * kBlock;
   const int c = coop_lane<kCoop>();
   const T dt = (T)ctrl->dt;
-  double err = 0;
 #pragma unroll 1
-  for (int round = 0; round < kCoop; ++round) {
-    const int i = coop_particle<kCoop>(base, round);
-    if (i >= n) break;
-    const V4<T> p = fpos[i];
-    const V4<T> va = vadv[i];
-    // the particle's own fields, requested before the walk so that their
-    // latency hides behind it
-    const V4<T> B = a1b[i];
-    const T rp = rest_psi_of(k, rdens, i);
-    const T pr = psi_rho[i];
-    const T al = alpha[i];
-    T sum = 0;  // this lane's share of sum_j X_j (v_i - v_j) . grad W_ij
-    auto term = [&](const Rec2<T>& d, bool ok) {
-      const V4<T>& q = d.a;
-      const V4<T>& vj = d.b;
-      T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-      T r2 = dx * dx + dy * dy + dz * dz, r;
-      T g = f_grad(k, r2, &r);
-      T dot = (dx * (va.x - vj.x) + dy * (va.y - vj.y) + dz * (va.z - vj.z)) * g;
-      sum += (ok ? dot : T(0)) * q.w;
-    };
-    // (f,f) pairs from the list; the (f,b) pairs have v_j = 0 (boundary
-    // vel_adv is never written), so their sum is v_i . sum_b X_j grad W_ij,
-    // the boundary share of alpha_1 that pass A recorded
-    sweep_lists_coop<kCoop, T, Rec2<T>>(
-        k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
-        [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
-        [&](int) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
-    sum = group_sum<kCoop>(sum);
-    if (c != 0) continue;
-    sum += va.x * B.x + va.y * B.y + va.z * B.z;
-    T psi = (pr - rp) + sum * dt;
-    // IPPE_psi_adv_non_negative (sph.py:219-226); with a clamp reference, the
-    // clamp set of a recorded iteration instead (psi clamped exactly where the
-    // recorded kappa is 0): the path whose derivative the adjoint takes
-    if (clamp_ref ? clamp_ref[i] == T(0) : psi < T(0)) psi = T(0);
-    psi_adv[i] = psi;
-    const T kap = psi / al;
-    kappa[i] = kap;
-    krec[i] = V4<T>{p.x, p.y, p.z, kap};  // the record the update sweep gathers
-    if (tape_v) {  // record the iteration for the adjoint
-      tape_v[i] = va;
-      tape_k[i] = kap;
+  for (int r = 0; r < R; ++r) {
+    const int i = coop_particle<kCoop>(coop_sub<R>(blk, r));
+    double err = 0;
+    if (i < n) {
+      const V4<T> p = fpos[i];
+      const V4<T> va = vadv[i];
+      // the particle's own fields, requested before the walk so that their
+      // latency hides behind it
+      const V4<T> B = a1b[i];
+      const T rp = rest_psi_of(k, rdens, i);
+      const T pr = psi_rho[i];
+      const T al = alpha[i];
+      T sum = 0;  // this lane's share of sum_j X_j (v_i - v_j) . grad W_ij
+      auto term = [&](const Rec2<T>& d, bool ok) {
+        const V4<T>& q = d.a;
+        const V4<T>& vj = d.b;
+        T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        T r2 = dx * dx + dy * dy + dz * dz, r;
+        T g = f_grad(k, r2, &r);
+        T dot = (dx * (va.x - vj.x) + dy * (va.y - vj.y) + dz * (va.z - vj.z)) * g;
+        sum += (ok ? dot : T(0)) * q.w;
+      };
+      // (f,f) pairs from the list; the (f,b) pairs have v_j = 0 (boundary
+      // vel_adv is never written), so their sum is v_i . sum_b X_j grad W_ij,
+      // the boundary share of alpha_1 that pass A recorded
+      sweep_lists_coop<kCoop, T, Rec2<T>>(
+          k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
+          [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
+          [&](int) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
+      sum = group_sum<kCoop>(sum);
+      if (c == 0) {
+        sum += va.x * B.x + va.y * B.y + va.z * B.z;
+        T psi = (pr - rp) + sum * dt;
+        // IPPE_psi_adv_non_negative (sph.py:219-226); with a clamp reference, the
+        // clamp set of a recorded iteration instead (psi clamped exactly where the
+        // recorded kappa is 0): the path whose derivative the adjoint takes
+        if (clamp_ref ? clamp_ref[i] == T(0) : psi < T(0)) psi = T(0);
+        psi_adv[i] = psi;
+        const T kap = psi / al;
+        kappa[i] = kap;
+        krec[i] = V4<T>{p.x, p.y, p.z, kap};  // the record the update sweep gathers
+        if (tape_v) {  // record the iteration for the adjoint
+          tape_v[i] = va;
+          tape_k[i] = kap;
+        }
+        err += (double)(psi / rp);
+      }
     }
-    err += (double)(psi / rp);
+    err = wave_sum(err);
+    if ((threadIdx.x & 63) == 0) lds[r][threadIdx.x >> 6] = err;
   }
-  double s = block_sum(err, lds);
-  if (threadIdx.x == 0) partial[blk.b] = s;
+  // one partial per sub-tile, in storage order
+  __syncthreads();
+  if (threadIdx.x < R) {
+    double s = 0;
+    for (int w = 0; w < kWaves; ++w) s += lds[threadIdx.x][w];
+    partial[coop_sub<R>(blk, threadIdx.x)] = s;
+  }
+  __syncthreads();  // lds is free again for a grid-stride block's next tile
 }
 
 template <class T>
@@ -523,7 +532,7 @@ __global__ void __launch_bounds__(kBlock)
 // alpha_1 = sum_j X_j grad W_ij of pass A (positions and X do not change
 // within the step), so the sweep only visits the fluid list, gathering the
 // one record (x_j, kappa_j) that the psi half-step wrote.
-template <class T>
+template <class T, int R = 1>
 __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, int n, int cap, int kk, const V4<T>* __restrict__ fpos,
                     const T* __restrict__ fmass, const T* __restrict__ kappa,
                     const V4<T>* __restrict__ krec, const V4<T>* __restrict__ alpha_1,
@@ -537,7 +546,7 @@ __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, in
   if (blk.b == 0) {
     // IPPE_psi_adv_non_negative's 0-D reduction (sph.py:221-226) and the loop
     // test of main.py:201-213 / 222-234
-    double tot = sum_partials(partial, blk.nb, lds);
+    double tot = sum_partials(partial, coop_blocks<kCoop>(n), lds);
     if (threadIdx.x == 0) {
       TSPH_STRICT
       T comp = (T)tot / (T)n;
@@ -561,12 +570,11 @@ __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, in
       }
     }
   }
-  const int base = xcd_block(blk.b, blk.nb) * kBlock;
   const int cl = coop_lane<kCoopU>();
   const T dt = (T)ctrl->dt;
 #pragma unroll 1
-  for (int round = 0; round < kCoopU; ++round) {
-    const int i = coop_particle<kCoopU>(base, round);
+  for (int r = 0; r < R; ++r) {
+    const int i = coop_particle<kCoopU>(coop_sub<R>(blk, r));
     if (i >= n) break;
     const V4<T> p = fpos[i];
     const T Xi = p.w;
@@ -619,7 +627,7 @@ __global__ void __launch_bounds__(kBlock)
 // must not write vel_adv: the update vel_adv = vel + dt * acce_adv happens in
 // the next kernel (k_surface_tension).
 // ---------------------------------------------------------------------------
-template <class T>
+template <class T, int R = 1>
 __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, int cap, const V4<T>* __restrict__ fpos, const T* __restrict__ vf,
              const T* __restrict__ rdens, const int* __restrict__ fstart,
              const int* __restrict__ bstart, const V4<T>* __restrict__ bpos,
@@ -627,11 +635,10 @@ __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, in
              V4<T>* __restrict__ vadv, V4<T>* __restrict__ vel, V4<T>* __restrict__ acce_adv,
              V4<T>* __restrict__ normal, const T* __restrict__ fmass,
              const T* __restrict__ psi_rho, V4<T>* __restrict__ strec) {
-  const int base = xcd_block(blk.b, blk.nb) * kBlock;
   const int c = coop_lane<kCoop>();
 #pragma unroll 1
-  for (int round = 0; round < kCoop; ++round) {
-    const int i = coop_particle<kCoop>(base, round);
+  for (int r = 0; r < R; ++r) {
+    const int i = coop_particle<kCoop>(coop_sub<R>(blk, r));
     if (i >= n) break;
     const V4<T> p = fpos[i];
     const V4<T> vi = vadv[i];
@@ -940,69 +947,65 @@ __global__ void __launch_bounds__(kBlock)
                     const int* __restrict__ nbr_nf, T* __restrict__ tmp,
                     const TsphControl* ctrl) {
   if (!ctrl->general_flag) return;
-  const int base = xcd_block(blockIdx.x, gridDim.x) * kBlock;
+  const int i = coop_particle<kCoop>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  if (i >= n) return;
   const int c = coop_lane<kCoop>();
   const T dt = (T)ctrl->dt;
-#pragma unroll 1
-  for (int round = 0; round < kCoop; ++round) {
-    const int i = coop_particle<kCoop>(base, round);
-    if (i >= n) break;
-    if (flag[i] != 0) continue;  // the whole group: one particle
-    const V4<T> p = fpos[i];
-    V4<T> ui[NP];
-    T pi[NP], conv[NP], diff[NP];
+  if (flag[i] != 0) return;  // the whole group: one particle
+  const V4<T> p = fpos[i];
+  V4<T> ui[NP];
+  T pi[NP], conv[NP], diff[NP];
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    ui[s] = drift[(long)i * NP + s];
+    pi[s] = vf[(long)i * NP + s];
+    conv[s] = T(0);
+    diff[s] = T(0);
+  }
+  // VFSPH: the position's alias lane is the rest volume (no extra gather)
+  const bool vx = k.solver == TSPH_VFSPH;
+  auto load = [&](int j) {
+    FbmRec<T, NP> d;
+    d.x = fpos[j];
+#pragma unroll
+    for (int s = 0; s < NP; ++s) d.u[s] = drift[(long)j * NP + s];
+    d.V = vx ? d.x.w : rvol[j];
+    return d;
+  };
+  auto pair = [&](const FbmRec<T, NP>& d, bool ok) {
+    if (!ok || d.u[0].w < T(0)) return;  // no neighbour, or a flagged one
+    const T dx = p.x - d.x.x, dy = p.y - d.x.y, dz = p.z - d.x.z;
+    const T r2 = dx * dx + dy * dy + dz * dz;
+    T r;
+    const T g = f_grad(k, r2, &r);
+    const T gv = g * d.V;
+    const T gd = gv * r2 * f_rcp(r2 + k.eps);
 #pragma unroll
     for (int s = 0; s < NP; ++s) {
-      ui[s] = drift[(long)i * NP + s];
-      pi[s] = vf[(long)i * NP + s];
-      conv[s] = T(0);
-      diff[s] = T(0);
+      const T pj = d.u[s].w;
+      const T fx = pi[s] * ui[s].x + pj * d.u[s].x;
+      const T fy = pi[s] * ui[s].y + pj * d.u[s].y;
+      const T fz = pi[s] * ui[s].z + pj * d.u[s].z;
+      conv[s] += (fx * dx + fy * dy + fz * dz) * gv;
+      diff[s] += (pi[s] - pj) * gd;
     }
-    // VFSPH: the position's alias lane is the rest volume (no extra gather)
-    const bool vx = k.solver == TSPH_VFSPH;
-    auto load = [&](int j) {
-      FbmRec<T, NP> d;
-      d.x = fpos[j];
+  };
+  sweep_lists_coop<kCoop, T, FbmRec<T, NP>>(
+      k, cap, i, c, p, fstart, fstart, fpos, fpos, nbr_f, nullptr, nbr_nf[i], 0, load, load,
+      pair, [&](const FbmRec<T, NP>&, bool) {});
 #pragma unroll
-      for (int s = 0; s < NP; ++s) d.u[s] = drift[(long)j * NP + s];
-      d.V = vx ? d.x.w : rvol[j];
-      return d;
-    };
-    auto pair = [&](const FbmRec<T, NP>& d, bool ok) {
-      if (!ok || d.u[0].w < T(0)) return;  // no neighbour, or a flagged one
-      const T dx = p.x - d.x.x, dy = p.y - d.x.y, dz = p.z - d.x.z;
-      const T r2 = dx * dx + dy * dy + dz * dz;
-      T r;
-      const T g = f_grad(k, r2, &r);
-      const T gv = g * d.V;
-      const T gd = gv * r2 * f_rcp(r2 + k.eps);
+  for (int s = 0; s < NP; ++s) {
+    conv[s] = group_sum<kCoop>(conv[s]);
+    diff[s] = group_sum<kCoop>(diff[s]);
+  }
+  if (c != 0) return;
+  const T pre_c = k.fbmC * dt, pre_d = dt * k.fbmD;
 #pragma unroll
-      for (int s = 0; s < NP; ++s) {
-        const T pj = d.u[s].w;
-        const T fx = pi[s] * ui[s].x + pj * d.u[s].x;
-        const T fy = pi[s] * ui[s].y + pj * d.u[s].y;
-        const T fz = pi[s] * ui[s].z + pj * d.u[s].z;
-        conv[s] += (fx * dx + fy * dy + fz * dz) * gv;
-        diff[s] += (pi[s] - pj) * gd;
-      }
-    };
-    sweep_lists_coop<kCoop, T, FbmRec<T, NP>>(
-        k, cap, i, c, p, fstart, fstart, fpos, fpos, nbr_f, nullptr, nbr_nf[i], 0, load, load,
-        pair, [&](const FbmRec<T, NP>&, bool) {});
-#pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      conv[s] = group_sum<kCoop>(conv[s]);
-      diff[s] = group_sum<kCoop>(diff[s]);
-    }
-    if (c != 0) continue;
-    const T pre_c = k.fbmC * dt, pre_d = dt * k.fbmD;
-#pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      T a = tmp[(long)i * NP + s];
-      a = a - pre_c * conv[s];
-      a = a + pre_d * diff[s];
-      tmp[(long)i * NP + s] = a;
-    }
+  for (int s = 0; s < NP; ++s) {
+    T a = tmp[(long)i * NP + s];
+    a = a - pre_c * conv[s];
+    a = a + pre_d * diff[s];
+    tmp[(long)i * NP + s] = a;
   }
 }
 
@@ -1219,19 +1222,18 @@ int solver_half(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl
   // With no fluid particles one block still runs the stop rule: the mean of
   // an empty sum is 0/0 = NaN, as in the reference (sph.py:221-226), so the
   // solve runs its minimum iteration count.
-  int nb = blocks_for(f->n > 0 ? f->n : 1);
   const T* psi = (const T*)(prm.solver_type == TSPH_VFSPH ? f->sph_compression : f->sph_density);
   if (half & 1)
-    hipLaunchKernelGGL(k_solver_psi<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity, kk,
-                       (const V4<T>*)f->pos, (const V4<T>*)f->vel_adv, psi,
+    hipLaunchKernelGGL(k_solver_psi<T>, dim3(coop_blocks<kCoop>(f->n)), dim3(kBlock), 0, st, k,
+                       f->n, f->capacity, kk, (const V4<T>*)f->pos, (const V4<T>*)f->vel_adv, psi,
                        (const T*)f->rest_density, (const T*)f->alpha, f->cell_start,
                        (const V4<T>*)b->pos, b->cell_start, f->nbr_f, f->nbr_b, f->nbr_nf,
                        f->nbr_nb, (T*)f->psi_adv, (T*)f->kappa, (V4<T>*)L.krec,
                        (const V4<T>*)L.a1b, (V4<T>*)tape_v, (T*)tape_k, (const T*)clamp_ref,
                        L.partial, ctrl);
   if (half & 2)
-    hipLaunchKernelGGL(k_solver_update<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
-                       kk, (const V4<T>*)f->pos, (const T*)f->mass, (const T*)f->kappa,
+    hipLaunchKernelGGL(k_solver_update<T>, dim3(coop_blocks<kCoopU>(f->n)), dim3(kBlock), 0, st,
+                       k, f->n, f->capacity, kk, (const V4<T>*)f->pos, (const T*)f->mass, (const T*)f->kappa,
                        (const V4<T>*)L.krec, (const V4<T>*)f->alpha_1, f->cell_start, (const V4<T>*)b->pos, b->cell_start, f->nbr_f, f->nbr_b,
                        f->nbr_nf, f->nbr_nb, (V4<T>*)f->vel_adv, L.partial, ctrl);
   TSPH_LAUNCH_CHECK("solver_iteration");
@@ -1248,8 +1250,8 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
   if (f->n == 0) return 0;
   int nb = blocks_for(f->n);
   const T* psi = (const T*)(prm.solver_type == TSPH_VFSPH ? f->sph_compression : f->sph_density);
-  hipLaunchKernelGGL(k_advect<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
-                     (const V4<T>*)f->pos, (const T*)f->volume_frac, (const T*)f->rest_density,
+  hipLaunchKernelGGL(k_advect<T>, dim3(coop_blocks<kCoop>(f->n)), dim3(kBlock), 0, st, k, f->n,
+                     f->capacity, (const V4<T>*)f->pos, (const T*)f->volume_frac, (const T*)f->rest_density,
                      f->cell_start, b->cell_start, (const V4<T>*)b->pos, f->nbr_f, f->nbr_nf,
                      (V4<T>*)f->vel_adv, (V4<T>*)f->vel, (V4<T>*)f->acce_adv,
                      (V4<T>*)f->normal, (const T*)f->mass, psi, (V4<T>*)L.krec);
@@ -1279,17 +1281,17 @@ int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws,
                      (const V4<T>*)f->vel_adv, (const V4<T>*)f->vel, (const T*)f->rest_density,
                      (const T*)f->volume_frac, (V4<T>*)f->acce_adv, (V4<T>*)f->acce,
                      (T*)f->fbm_zeta, (V4<T>*)f->drift_vel, (T*)f->volume_frac_tmp, f->flag, ctrl);
-  auto flux = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+  auto flux = [&](auto kern, int nbk) {
+    hipLaunchKernelGGL(kern, dim3(nbk), dim3(kBlock), 0, st, k, f->n, f->capacity,
                        (const V4<T>*)f->pos, (const T*)f->rest_volume, (const T*)f->volume_frac,
                        (const V4<T>*)f->drift_vel, f->flag, f->cell_start, f->nbr_f, f->nbr_nf,
                        (T*)f->volume_frac_tmp, ctrl);
   };
   switch (prm.phase_num) {  // the cooperative sweep keeps NP phases' records in registers
-    case 1: flux(k_fbm_flux_coop<T, 1>); break;
-    case 2: flux(k_fbm_flux_coop<T, 2>); break;
-    case 3: flux(k_fbm_flux_coop<T, 3>); break;
-    default: flux(k_fbm_flux<T>); break;
+    case 1: flux(k_fbm_flux_coop<T, 1>, coop_blocks<kCoop>(f->n)); break;
+    case 2: flux(k_fbm_flux_coop<T, 2>, coop_blocks<kCoop>(f->n)); break;
+    case 3: flux(k_fbm_flux_coop<T, 3>, coop_blocks<kCoop>(f->n)); break;
+    default: flux(k_fbm_flux<T>, nb); break;
   }
   hipLaunchKernelGGL(k_fbm_check<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                      (const T*)f->volume_frac, (const T*)f->volume_frac_tmp, f->flag, L.partial,
@@ -1547,11 +1549,12 @@ __global__ void __launch_bounds__(kBlock)
   });
 }
 
-template <class T>
-__global__ void __launch_bounds__(kBlock) kb_solver_psi(const char* __restrict__ tab, int ns, int kk) {
-  for_tiles<T, kTileFluid>(tab, ns, [&](const SceneEntry<T>& e, int, Blk blk) {
+template <class T, int R>
+__global__ void __launch_bounds__(kBlock)
+    kb_solver_psi(const char* __restrict__ tab, int ns, int kk) {
+  for_coop_tiles<T, kCoop, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_solver_psi_body<T>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
+    k_solver_psi_body<T, R>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
                          (const V4<T>*)f.vel_adv, psi_of(e), (const T*)f.rest_density,
                          (const T*)f.alpha, f.cell_start, (const V4<T>*)e.b.pos, e.b.cell_start,
                          f.nbr_f, f.nbr_b, f.nbr_nf, f.nbr_nb, (T*)f.psi_adv, (T*)f.kappa,
@@ -1560,11 +1563,12 @@ __global__ void __launch_bounds__(kBlock) kb_solver_psi(const char* __restrict__
   });
 }
 
-template <class T>
-__global__ void __launch_bounds__(kBlock) kb_solver_update(const char* __restrict__ tab, int ns, int kk) {
-  for_tiles<T, kTileFluid>(tab, ns, [&](const SceneEntry<T>& e, int, Blk blk) {
+template <class T, int R>
+__global__ void __launch_bounds__(kBlock)
+    kb_solver_update(const char* __restrict__ tab, int ns, int kk) {
+  for_coop_tiles<T, kCoopU, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_solver_update_body<T>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
+    k_solver_update_body<T, R>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
                             (const T*)f.mass, (const T*)f.kappa, (const V4<T>*)e.L.krec,
                             (const V4<T>*)f.alpha_1, f.cell_start,
                             (const V4<T>*)e.b.pos, e.b.cell_start, f.nbr_f, f.nbr_b, f.nbr_nf,
@@ -1572,11 +1576,11 @@ __global__ void __launch_bounds__(kBlock) kb_solver_update(const char* __restric
   });
 }
 
-template <class T>
+template <class T, int R>
 __global__ void __launch_bounds__(kBlock) kb_advect(const char* __restrict__ tab, int ns) {
-  for_tiles<T, kTileFluid>(tab, ns, [&](const SceneEntry<T>& e, int, Blk blk) {
+  for_coop_tiles<T, kCoop, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_advect_body<T>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, (const T*)f.volume_frac,
+    k_advect_body<T, R>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, (const T*)f.volume_frac,
                      (const T*)f.rest_density, f.cell_start, e.b.cell_start,
                      (const V4<T>*)e.b.pos, f.nbr_f, f.nbr_nf, (V4<T>*)f.vel_adv, (V4<T>*)f.vel,
                      (V4<T>*)f.acce_adv, (V4<T>*)f.normal, (const T*)f.mass, psi_of(e),
@@ -1647,11 +1651,20 @@ int batch_solver_begin(const TsphBatchInfo& bi, char* tab, int solve, uint64_t* 
 template <class T>
 int batch_solver_half(const TsphBatchInfo& bi, char* tab, int kk, int half, int grid,
                       hipStream_t st) {
-  const int g = grid_for(bi.tiles[kTileFluid], grid);
-  if (!g) return 0;
-  if (half & 1) hipLaunchKernelGGL(kb_solver_psi<T>, dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes, kk);
-  if (half & 2)
-    hipLaunchKernelGGL(kb_solver_update<T>, dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes, kk);
+  const int tiles = bi.tiles[kTileFluid];
+  if (tiles <= 0) return 0;
+  auto launch = [&](auto kern, int blocks) {
+    hipLaunchKernelGGL(kern, dim3(grid_for(blocks, grid)), dim3(kBlock), 0, st, tab, bi.nscenes, kk);
+  };
+  const bool split = coop_split(tiles);
+  if (half & 1) {
+    if (split) launch(kb_solver_psi<T, 1>, tiles * kCoop);
+    else launch(kb_solver_psi<T, kCoop>, tiles);
+  }
+  if (half & 2) {
+    if (split) launch(kb_solver_update<T, 1>, tiles * kCoopU);
+    else launch(kb_solver_update<T, kCoopU>, tiles);
+  }
   TSPH_LAUNCH_CHECK("batch_solver_iteration");
   return 0;
 }
@@ -1660,7 +1673,12 @@ template <class T>
 int batch_advect(const TsphBatchInfo& bi, char* tab, int grid, hipStream_t st) {
   const int g = grid_for(bi.tiles[kTileFluid], grid);
   if (!g) return 0;
-  hipLaunchKernelGGL(kb_advect<T>, dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
+  const int tiles = bi.tiles[kTileFluid];
+  if (coop_split(tiles))
+    hipLaunchKernelGGL((kb_advect<T, 1>), dim3(grid_for(tiles * kCoop, grid)), dim3(kBlock), 0, st,
+                       tab, bi.nscenes);
+  else
+    hipLaunchKernelGGL((kb_advect<T, kCoop>), dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
   hipLaunchKernelGGL(kb_surface_tension<T>, dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
   TSPH_LAUNCH_CHECK("batch_advect");
   return 0;

@@ -202,16 +202,50 @@ constexpr int kCoop = 4;    // lanes per particle of the gather-heavy sweeps
 constexpr int kCoopU = 2;   // lanes per particle of the update sweep (one gather per pair)
 constexpr int kCoopNb = 4;  // gathers in flight per lane
 
-// A block covers its kBlock particles in C rounds of kBlock / C particles.
+// A block covers kBlock / C particles, one per group: C rounds of as many
+// particles in a C-th of the blocks leave a small launch short of blocks and
+// a large one with long last blocks, and hold more registers.  In us, C rounds
+// and one: psi, update, advection at 1M 74.0, 49.6, 74.4 and 68.9, 46.6,
+// 66.1; at 4M 370, 250, 370 and 335, 243, 340.
+//
+// Blocks of a sweep over n particles: C per kBlock particles, so that they are
+// also the sub-tiles of a grouped launch's fluid tiles and a scene's block
+// partials are the same in both.
+template <int C>
+__host__ __device__ __forceinline__ int coop_blocks(int n) {
+  return (int)(((long)(n > 0 ? n : 1) + kBlock - 1) / kBlock) * C;
+}
+// Round r of the R rounds of block blk: the sub-tile of the particles it
+// takes, and the particle of this thread's group in a sub-tile (n or more:
+// none).  R = 1 except in grouped launches (for_coop_tiles).
+template <int R = 1>
+__device__ __forceinline__ int coop_sub(Blk blk, int r = 0) {
+  return xcd_block(blk.b, blk.nb) * R + r;
+}
+template <int C>
+__device__ __forceinline__ int coop_particle(int sub) {
+  return sub * (kBlock / C) + (int)(threadIdx.x / C);
+}
+// Every scene's sweep in a grouped launch; f(entry, blk).  A block takes R of
+// a fluid tile's C sub-tiles: finding a tile's scene and its constants is a
+// chain of dependent loads, which R = C pays once per tile where the tiles
+// alone fill the chip (24 scenes, 2,700 tiles: psi 45.4 us, split 52.3);
+// fewer tiles are split (coop_split), as a single scene's launch is.
+template <class T, int C, int R, class F>
+__device__ __forceinline__ void for_coop_tiles(const char* __restrict__ tab, int ns, F&& f) {
+  constexpr int split = C / R;
+  const int total = tile_prefix<T, kTileFluid>(tab, ns)[ns] * split;
+  for (int t = blockIdx.x; t < total; t += gridDim.x)
+    on_tile<T, kTileFluid>(tab, ns, t / split, [&](const SceneEntry<T>& e, int, Blk tile) {
+      f(e, Blk{tile.b * split + t % split, tile.nb * split});
+    });
+}
+constexpr int kCoopTilesFull = 2048;  // fluid tiles that fill the 256 CUs eight times
+inline bool coop_split(int tiles) { return tiles < kCoopTilesFull; }
 template <int C>
 __device__ __forceinline__ int coop_lane() {
   return threadIdx.x & (C - 1);
 }
-template <int C>
-__device__ __forceinline__ int coop_particle(int base, int round) {
-  return base + round * (kBlock / C) + (int)(threadIdx.x / C);
-}
-
 template <int C, class T>
 __device__ __forceinline__ T group_sum(T v) {
 #pragma unroll
