@@ -60,3 +60,51 @@ def test_batch_at_block_edges_is_bit_identical():
             assert st.compression == batch.sims[k].control().compression, (step, BLOCKS[k])
             for f in ("pos", "vel"):
                 assert np.array_equal(batch.sims[k].fluid.to_numpy(f), sim.fluid.to_numpy(f)), (step, BLOCKS[k], f)
+
+
+def _lists(sim):
+    """The fluid and boundary lists' counts and entries, slot by slot."""
+    f = sim.fluid
+    n, cap = f.part_num, f.t["pos"].shape[0]
+    out = []
+    for rows, count, limit in (("nbr_f", "nbr_nf", f.list_cap_f), ("nbr_b", "nbr_nb", f.list_cap_b)):
+        cnt = f.t[count][:n].cpu().numpy()
+        lst = f.t[rows].cpu().numpy().reshape(limit, cap)[:, :n]
+        out += [cnt, np.where(np.arange(limit)[:, None] < np.minimum(cnt, limit)[None, :], lst, -1)]
+    return out
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("caps", [(64, 48), (9, 3)], ids=["lists", "overflow"])
+def test_pass_a_by_quads_is_that_by_single_lanes(dim, precision, caps):
+    """A small scene's own step runs pass A with a quad of lanes per particle,
+    a grouped step with one: every field and list entry is the same, bit for
+    bit, also where lists overflow, and around particles outside the grid, at
+    one position, or crowded into one cell (more than a list in LDS holds)."""
+    from tichi_sph_amd import simulation_from_dicts
+    from tichi_sph_amd.batch import SceneBatch
+    scn, cfg = scene((33, 29, 0) if dim == 2 else (11, 13, 9))
+    rng = np.random.default_rng(7)
+    sims = []
+    for _ in range(2):
+        sim = simulation_from_dicts(cfg, scn, precision=precision, cfl=False, list_cap_f=caps[0], list_cap_b=caps[1])
+        sims.append(sim)
+    x = sims[0].fluid.to_numpy("pos")
+    x = x + rng.uniform(-0.2, 0.2, x.shape) * sims[0].config.part_size[1]
+    x[5] = x[4]
+    x[6] = -1.0
+    x[7] = 1e9
+    x[40:140] = x[30] + rng.uniform(-0.1, 0.1, (100, dim)) * sims[0].config.part_size[1]
+    for sim in sims:
+        sim.fluid.from_numpy("pos", x.astype(sim.fluid.np_dtype))
+    batch = SceneBatch([sims[1]])
+    sims[0].sph_step()
+    batch.step()
+    names = ("W", "sph_density", "sph_compression", "alpha", "alpha_1", "alpha_2", "vol", "pos", "vel")
+    for name in names:
+        assert np.array_equal(sims[0].fluid.to_numpy(name), sims[1].fluid.to_numpy(name), equal_nan=True), name
+    for name in names[:4] + ("alpha_2",):
+        assert np.array_equal(sims[0].bound.to_numpy(name), sims[1].bound.to_numpy(name), equal_nan=True), name
+    for a, b in zip(_lists(sims[0]), _lists(sims[1])):
+        assert np.array_equal(a, b)

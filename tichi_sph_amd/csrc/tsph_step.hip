@@ -59,6 +59,49 @@ struct PassAAcc {
     }
     return true;
   }
+  // add() for one list slot per lane of a quad: the sums take the quad's terms
+  // in lane order (a lane without one adds an exact zero).
+  template <bool FQ, bool XM>
+  __device__ __forceinline__ void add_quad(const KP<T>& k, const V4<T>& p, const V4<T>& q, T mj,
+                                           T vj, bool valid, bool apart, bool fluid) {
+    const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+    T r2, r, qh;
+    {
+      TSPH_STRICT
+      r2 = s_r2(dx, dy, dz);
+      r = pa_sqrt<FQ>(r2);
+      qh = pa_quot<FQ>(k, r);
+      const T Wr = valid ? s_W_q_sel(k, qh) : T(0);
+      w = quad_add(w, Wr);
+      cp = quad_add(cp, Wr * vj);
+      dn = quad_add(dn, Wr * mj);
+    }
+    const T u = T(1) - qh;
+    T g = qh <= T(0.5) ? k.wg_a * (T(3) * qh - T(2)) : -k.wg_b * (u * u) * f_rcp(r);
+    const T Xj = q.w;
+    const T xg = valid && apart ? Xj * g : T(0);
+    const T x2m = XM ? Xj : (Xj * Xj) * f_rcp(mj);
+    const T t2 = valid && apart ? (g * g) * r2 : T(0);
+    add_lane<0>(xg, dx, dy, dz, t2, x2m, fluid);
+    add_lane<1>(xg, dx, dy, dz, t2, x2m, fluid);
+    add_lane<2>(xg, dx, dy, dz, t2, x2m, fluid);
+    add_lane<3>(xg, dx, dy, dz, t2, x2m, fluid);
+  }
+  template <int K>
+  __device__ __forceinline__ void add_lane(T xg_, T dx_, T dy_, T dz_, T t2, T x2m, bool fluid) {
+    const T xg = quad_lane<K>(xg_), dx = quad_lane<K>(dx_), dy = quad_lane<K>(dy_),
+            dz = quad_lane<K>(dz_);
+    ax += xg * dx;
+    ay += xg * dy;
+    az += xg * dz;
+    if (fluid) {
+      a2 += quad_lane<K>(t2) * quad_lane<K>(x2m);
+    } else {
+      bx += xg * dx;
+      by += xg * dy;
+      bz += xg * dz;
+    }
+  }
 };
 
 // List slots per particle staged in LDS by pass A (kPassAK x kBlock ints per
@@ -172,6 +215,55 @@ __device__ __forceinline__ void k_pass_a_fluid_body(Blk blk, const KP<T>& k, int
                   vel_adv, nbr_nf, nbr_nb, ctrl);
 }
 
+// Pass A of the fluid, a quad of lanes per particle (walk_quad).  Every sum
+// takes the quad's terms in walk order, so all of them are those of
+// k_pass_a_fluid_body, bit for bit.
+template <class T>
+struct PassARec {
+  V4<T> q;
+  T o;  // mass or rest volume, whichever is not the alias in q.w
+};
+template <class T, bool FQ, bool XM>
+__device__ __forceinline__ void pass_a_quad_fluid(
+    int sub, const KP<T>& k, const TsphObject& f, const TsphObject& b, V4<T>* __restrict__ a1b,
+    TsphControl* ctrl, WalkLds& lds) {
+  const int i = coop_particle<kQuad>(sub), c = coop_lane<kQuad>();
+  if (i >= f.n) return;
+  const V4<T>* __restrict__ fpos = (const V4<T>*)f.pos;
+  const V4<T> p = fpos[i];
+  const T mi = ((const T*)f.mass)[i];
+  const unsigned below = (1u << c) - 1;
+  PassAAcc<T> acc;
+  int cnt[2] = {0, 0};
+#pragma unroll
+  for (int ob = 0; ob < 2; ++ob) {
+    const TsphObject& o = ob == 0 ? f : b;
+    const V4<T>* __restrict__ opos = (const V4<T>*)o.pos;
+    const T* __restrict__ oo = (const T*)(XM ? o.rest_volume : o.mass);
+    int* __restrict__ list = ob == 0 ? f.nbr_f : f.nbr_b;
+    const int lcap = ob == 0 ? k.list_cap_f : k.list_cap_b;
+    int nl = 0;
+    if (ob == 0 || b.n > 0)
+      walk_quad(k, o.cell_start, opos, p, lds,
+                [&](int j) { return PassARec<T>{opos[j], oo[j]}; },
+                [&](const PassARec<T>& r, int j, bool valid, bool apart) {
+                  acc.template add_quad<FQ, XM>(k, p, r.q, XM ? r.q.w : r.o, XM ? r.o : r.q.w,
+                                                valid, apart, ob == 0);
+                  const unsigned v = quad_vote(valid && apart);
+                  const int slot = nl + __popc(v & below);
+                  if (valid && apart && slot < lcap) list[(long)slot * f.capacity + i] = j;
+                  nl += __popc(v);
+                });
+    cnt[ob] = nl;
+  }
+  if (c != 0) return;
+  f.flag[i] = 0;  // SPH_clean_value, sph.py:30
+  a1b[i] = V4<T>{acc.bx, acc.by, acc.bz, T(0)};
+  pass_a_epilogue(k, i, p, mi, acc, cnt[0], cnt[1], (T*)f.W, (T*)f.sph_compression,
+                  (T*)f.sph_density, (V4<T>*)f.alpha_1, (T*)f.alpha_2, (T*)f.alpha, (T*)f.vol,
+                  (const V4<T>*)f.vel, (V4<T>*)f.vel_adv, f.nbr_nf, f.nbr_nb, ctrl);
+}
+
 // Runs f(fq, xm) with the fluid body's compile-time variant for these
 // constants: the verified fast quotient, and whether X is the mass.
 template <class T, class F>
@@ -206,6 +298,12 @@ __global__ void __launch_bounds__(kBlock)
     k_pass_a_fluid_body<T, decltype(fq)::value, decltype(xm)::value>(blk, k, n, cap, fpos, fmass, frvol, fstart, nb, bpos, bmass, brvol, bstart, W, comp, dens, alpha_1, alpha_2, alpha, vol, vel, vel_adv, nbr_f, nbr_b, nbr_nf, nbr_nb, flag, a1b, ctrl, stage);
   });
 }
+
+template <class T>
+struct BoundRec {
+  V4<T> q;
+  T v, m;  // rest volume, mass
+};
 
 // Pass A, boundary particles: SPH_prepare_attr (b,b)(b,f), SPH_prepare_alpha_2
 // (b,f), SPH_prepare_alpha (alpha_1 of the boundary is never accumulated).
@@ -284,6 +382,100 @@ __global__ void __launch_bounds__(kBlock)
                    V4<T>* __restrict__ alpha_1, T* __restrict__ alpha_2, T* __restrict__ alpha,
                    T* __restrict__ vol, V4<T>* __restrict__ ss, int kept) {
   k_pass_a_bound_body<T, false>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, nb, bpos, bmass, brvol, bstart, fpos, fmass, frvol, fstart, W, comp, dens, alpha_1, alpha_2, alpha, vol, ss, kept != 0);
+}
+
+// Pass A of the boundary, a quad of lanes per particle (walk_quad): the sums
+// of k_pass_a_bound_body, each in walk order.
+template <class T>
+__device__ __forceinline__ void pass_a_quad_bound(int sub, const KP<T>& k, const TsphObject& f,
+                                                  const TsphObject& b, bool kept, WalkLds& lds) {
+  TSPH_STRICT
+  const int i = coop_particle<kQuad>(sub), c = coop_lane<kQuad>();
+  if (i >= b.n) return;
+  const V4<T>* __restrict__ bpos = (const V4<T>*)b.pos;
+  const V4<T>* __restrict__ fpos = (const V4<T>*)f.pos;
+  V4<T>* ss = (V4<T>*)b.static_sums;
+  const V4<T> p = bpos[i];
+  const T mi = ((const T*)b.mass)[i];
+  T w = 0, cp = 0, dn = 0, a2 = 0;
+  if (ss != nullptr && kept) {
+    const V4<T> s0 = ss[i];
+    w = s0.x;
+    cp = s0.y;
+    dn = s0.z;
+  } else {
+    const T* __restrict__ bm = (const T*)b.mass;
+    const T* __restrict__ bv = (const T*)b.rest_volume;
+    walk_quad(k, b.cell_start, bpos, p, lds,
+              [&](int j) { return BoundRec<T>{bpos[j], bv[j], bm[j]}; },
+              [&](const BoundRec<T>& r, int, bool valid, bool) {
+                TSPH_STRICT
+                const T d = s_sqrt(s_r2(p.x - r.q.x, p.y - r.q.y, p.z - r.q.z));
+                const T Wr = valid ? s_W_q_sel(k, d / k.h) : T(0);
+                w = quad_add(w, Wr);
+                cp = quad_add(cp, Wr * r.v);
+                dn = quad_add(dn, Wr * r.m);
+              });
+    if (ss != nullptr && c == 0) ss[i] = V4<T>{w, cp, dn, T(0)};
+  }
+  if (f.n > 0) {
+    const T* __restrict__ fm = (const T*)f.mass;
+    const T* __restrict__ fv = (const T*)f.rest_volume;
+    walk_quad(k, f.cell_start, fpos, p, lds,
+              [&](int j) { return BoundRec<T>{fpos[j], fv[j], fm[j]}; },
+              [&](const BoundRec<T>& r, int, bool valid, bool apart) {
+                TSPH_STRICT
+                const T d = s_sqrt(s_r2(p.x - r.q.x, p.y - r.q.y, p.z - r.q.z));
+                const T qh = d / k.h;
+                const T Wr = valid ? s_W_q_sel(k, qh) : T(0);
+                w = quad_add(w, Wr);
+                cp = quad_add(cp, Wr * r.v);
+                dn = quad_add(dn, Wr * r.m);
+                const T wg = s_Wg_q(k, qh);
+                const T Xj = r.q.w;
+                const T wg2 = wg * wg;
+                a2 = quad_add(a2, valid && apart ? wg2 * (Xj * Xj) / r.m : T(0));
+              });
+  }
+  if (c != 0) return;
+  ((T*)b.W)[i] = w;
+  ((T*)b.sph_compression)[i] = cp;
+  ((T*)b.sph_density)[i] = dn;
+  ((V4<T>*)b.alpha_1)[i] = V4<T>{T(0), T(0), T(0), T(0)};
+  ((T*)b.alpha_2)[i] = a2;
+  T al = T(0) / mi + a2;
+  if (al < T(1e-4)) al = T(1e-4);
+  ((T*)b.alpha)[i] = al;
+  const T psi = k.solver == TSPH_VFSPH ? cp : dn;
+  ((T*)b.vol)[i] = p.w / psi;
+}
+
+// Pass A of both objects by quads, for small scenes.  One lane per particle
+// walks its 200 or so candidates one trip after the other: that chain takes
+// 65 us however few the particles (8,000: 125 waves on 1,024 SIMDs), and the
+// quads cut it to a quarter.  They spend more instructions per candidate (the
+// votes and the list in LDS), so once the chip is full the single lanes win.
+// us per launch, one lane / quads: 3D FP32 8k 71 / 30, 64k 72 / 39, 133k 78 /
+// 67, 149k 80 / 73, 195k 82 / 85, 1M 238 / 368; FP64 8k 87 / 32, 64k 91 / 66,
+// 97k 105 / 89, 195k 130 / 156; 2D FP32 8k 24 / 17, 78k 24.8 / 23.1, 102k
+// 25.5 / 26.
+template <class T>
+static constexpr int pass_a_quad_max(int dim) {
+  return dim == 2 ? 80 * 1024 : sizeof(T) == 4 ? 144 * 1024 : 96 * 1024;
+}
+template <class T>
+__global__ void __launch_bounds__(kBlock)
+    k_pass_a_quad(KP<T> k, TsphObject f, TsphObject b, int nbf, V4<T>* a1b, TsphControl* ctrl) {
+  __shared__ WalkLds lds;
+  if ((int)blockIdx.x < nbf) {
+    const int sub = coop_sub(Blk{(int)blockIdx.x, nbf});
+    pass_a_fluid_variant(k, [&](auto fq, auto xm) {
+      pass_a_quad_fluid<T, decltype(fq)::value, decltype(xm)::value>(sub, k, f, b, a1b, ctrl, lds);
+    });
+  } else {
+    pass_a_quad_bound<T>(coop_sub(Blk{(int)blockIdx.x - nbf, (int)gridDim.x - nbf}), k, f, b,
+                         (b.flags & TSPH_OBJ_STATIC_SUMS) != 0, lds);
+  }
 }
 
 // Per-step reset of the control block's step-scoped state: general_flag = 1
@@ -1103,6 +1295,15 @@ static int pass_a(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphContr
                   bool with_bound, const WsLayout& L, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   hipLaunchKernelGGL(k_step_reset, dim3(1), dim3(64), 0, st, ctrl);
+  if (with_bound && f->n > 0 && f->n <= pass_a_quad_max<T>(prm.dim) &&
+      b->n <= 2 * pass_a_quad_max<T>(prm.dim)) {
+    const int nbf = coop_blocks<kQuad>(f->n);
+    hipLaunchKernelGGL(k_pass_a_quad<T>, dim3(nbf + (b->n > 0 ? coop_blocks<kQuad>(b->n) : 0)),
+                       dim3(kBlock), 0, st, k, *f, *b, nbf, (V4<T>*)L.a1b, ctrl);
+    TSPH_LAUNCH_CHECK("density_alpha");
+    if (b->n > 0 && b->static_sums) b->flags |= TSPH_OBJ_STATIC_SUMS;
+    return 0;
+  }
   if (with_bound && f->n > 0 && b->n > 0) {
     const int nbf = blocks_for(f->n);
     hipLaunchKernelGGL(k_pass_a_both<T>, dim3(nbf + blocks_for(b->n)), dim3(kBlock), 0, st, k, *f,

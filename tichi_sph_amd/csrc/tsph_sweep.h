@@ -322,4 +322,164 @@ __device__ __forceinline__ void sweep_lists_coop(const KP<T>& k, int cap, int i,
   });
 }
 
+// ---------------------------------------------------------------------------
+// Cooperative cell walk.  A quad of lanes shares one particle.  The quad reads
+// four consecutive candidates of a row run at once, tests them, and appends
+// those in range to a list in LDS, in walk order (a candidate's slot is the
+// quad's count so far plus the hits among the lanes before it); whenever the
+// list fills, and at the end, the quad works the list off, each lane taking
+// every fourth slot, so that the pair math runs on full quads.  The runs of a
+// particle's rows are looked up once, side by side, and only the rows that
+// hold particles are walked.
+// ---------------------------------------------------------------------------
+constexpr int kQuad = 4;
+constexpr int kQuads = kBlock / kQuad;  // particles per block
+constexpr int kWalkRows = 9;            // row runs looked up at a time
+constexpr int kWalkS = 48;              // list slots per particle
+// Candidates and list slots in flight per lane.  Pass A at 64k / 195k: 2 and 2
+// 51 / 102 us, 2 and 1 40 / 88, 1 and 1 45 / 95, 3 and 1 39 / 85.
+constexpr int kWalkU = 3;
+constexpr int kWalkNb = 1;
+
+struct WalkLds {
+  int2 run[kWalkRows][kQuads];
+  int list[kWalkS][kQuads];
+};
+
+// The value of lane K of the quad, in all its lanes.
+template <int K>
+__device__ __forceinline__ int quad_lane(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, K * 0x55, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(quad_lane<K>(__float_as_int(v)));
+}
+template <int K>
+__device__ __forceinline__ double quad_lane(double v) {
+  return __hiloint2double(quad_lane<K>(__double2hiint(v)), quad_lane<K>(__double2loint(v)));
+}
+// acc + the quad's four values in lane order, one rounding each.
+template <class T>
+__device__ __forceinline__ T quad_add(T acc, T v) {
+  TSPH_STRICT
+  acc = acc + quad_lane<0>(v);
+  acc = acc + quad_lane<1>(v);
+  acc = acc + quad_lane<2>(v);
+  return acc + quad_lane<3>(v);
+}
+// The quad's four votes, lane 0 in bit 0.
+__device__ __forceinline__ unsigned quad_vote(bool v) {
+  const unsigned long long m = __ballot(v);
+  const unsigned lane = threadIdx.x & 63;
+  const unsigned half = lane < 32 ? (unsigned)m : (unsigned)(m >> 32);
+  return (half >> (lane & 28)) & 15u;
+}
+// LDS written by lanes of this wave is read by others of it: the wave's LDS
+// accesses complete in order, so only the compiler has to keep theirs.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// load(j) gathers what the pair terms need of candidate j; term(record, j,
+// valid, apart) adds one list slot per lane (valid: the lane holds one;
+// apart: r > 0) and runs with the whole quad.  Candidates in range are those
+// with r^2 <= r2max.
+template <class T, class Load, class Term>
+__device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict__ cstart,
+                                          const V4<T>* __restrict__ pos, const V4<T>& p,
+                                          WalkLds& lds, Load&& load, Term&& term) {
+  const int c = threadIdx.x & (kQuad - 1), g = threadIdx.x / kQuad;
+  const unsigned below = (1u << c) - 1;
+  const int R = k.R, side = 2 * R + 1, rows = k.dim == 3 ? side * side : side;
+  int cc[3];
+  node_encode(k, p.x, p.y, p.z, cc);
+  for (int row0 = 0; row0 < rows; row0 += kWalkRows) {
+    int nrun = 0;
+#pragma unroll
+    for (int q = 0; q < (kWalkRows + kQuad - 1) / kQuad; ++q) {
+      const int r = c + kQuad * q, row = row0 + r;
+      int2 run = make_int2(0, 0);
+      if (r < kWalkRows && row < rows) {
+        const int dy = row % side - R, dz = k.dim == 3 ? row / side - R : 0;
+        const int c0 = dim_encode(k, wadd(cc[0], -R), wadd(cc[1], dy), wadd(cc[2], dz));
+        const long lo = c0 < 1 ? 1 : (long)c0;
+        long hi = (long)c0 + 2 * R;
+        if (hi > k.node_num - 1) hi = k.node_num - 1;
+        if (lo <= hi) run = make_int2(cstart[lo], cstart[hi + 1]);
+      }
+      const unsigned v = quad_vote(run.x < run.y);
+      if (run.x < run.y) lds.run[nrun + __popc(v & below)][g] = run;
+      nrun += __popc(v);
+    }
+    if (nrun == 0) continue;
+    wave_lds_fence();
+    int at = 0, j = lds.run[0][g].x, end = lds.run[0][g].y, cnt = 0;
+    bool more = true;
+    int cj[kWalkU];
+    V4<T> cq[kWalkU];
+#pragma unroll
+    for (int u = 0; u < kWalkU; ++u) {
+      cj[u] = j + c + kQuad * u;
+      cq[u] = pos[min(cj[u], end - 1)];
+    }
+    while (more) {
+      while (more && cnt <= kWalkS - kQuad * kWalkU) {
+        // the next trip's candidates are requested before this one's tests
+        const int cend = end;
+        j += kQuad * kWalkU;
+        if (j >= end) {
+          ++at;
+          more = at < nrun;
+          if (more) {
+            const int2 run = lds.run[at][g];
+            j = run.x;
+            end = run.y;
+          }
+        }
+        int nj[kWalkU];
+        V4<T> nq[kWalkU];
+        if (more) {
+#pragma unroll
+          for (int u = 0; u < kWalkU; ++u) {
+            nj[u] = j + c + kQuad * u;
+            nq[u] = pos[min(nj[u], end - 1)];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kWalkU; ++u) {
+          const T r2 = s_r2(p.x - cq[u].x, p.y - cq[u].y, p.z - cq[u].z);
+          const bool take = r2 <= k.r2max && cj[u] < cend;
+          const unsigned v = quad_vote(take);
+          // the sign bit marks a candidate at r = 0
+          if (take) lds.list[cnt + __popc(v & below)][g] = r2 > T(0) ? cj[u] : ~cj[u];
+          cnt += __popc(v);
+        }
+        if (more) {
+#pragma unroll
+          for (int u = 0; u < kWalkU; ++u) {
+            cj[u] = nj[u];
+            cq[u] = nq[u];
+          }
+        }
+      }
+      wave_lds_fence();
+      for (int s0 = 0; s0 < cnt; s0 += kQuad * kWalkNb) {
+        int e[kWalkNb];
+        decltype(load(0)) rec[kWalkNb];
+#pragma unroll
+        for (int u = 0; u < kWalkNb; ++u) e[u] = lds.list[min(s0 + c + kQuad * u, cnt - 1)][g];
+#pragma unroll
+        for (int u = 0; u < kWalkNb; ++u) rec[u] = load(e[u] < 0 ? ~e[u] : e[u]);
+#pragma unroll
+        for (int u = 0; u < kWalkNb; ++u)
+          term(rec[u], e[u] < 0 ? ~e[u] : e[u], s0 + c + kQuad * u < cnt, e[u] >= 0);
+      }
+      wave_lds_fence();
+      cnt = 0;
+    }
+  }
+}
+
 }  // namespace tsph
