@@ -6,8 +6,8 @@
  * points.  Every pointer inside TsphObject / TsphControl / workspace is a
  * DEVICE pointer owned by the caller (in the Python host layer: torch
  * tensors); the library never allocates or frees device memory and never
- * synchronises the host.  All entry points enqueue work on `stream`
- * (a hipStream_t passed as void*) and return 0 on success or a negative
+ * synchronises the host (tsph_step alone waits, for words that the device
+ * writes).  All entry points enqueue work on `stream` (a hipStream_t passed as void*) and return 0 on success or a negative
  * TSPH_E* code; tsph_last_error() then holds a message (thread-local).
  *
  * Arithmetic type: TsphParams.precision selects float (4) or double (8) for
@@ -334,6 +334,32 @@ int tsph_tail(const TsphParams* p, TsphObject* fluid, TsphControl* ctrl, int32_t
  */
 int tsph_wcsph(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphControl* ctrl,
                void* stream);
+
+/*
+ * One whole step of main.py:175-256 (with cfl_condition before it when `cfl`
+ * is set, main.py:348): tsph_sort_object(fluid), tsph_density_alpha, the two
+ * solves to their stop rule around tsph_advect, [tsph_wcsph], [tsph_fbm_round
+ * while any particle was flagged, at most 1000 times], tsph_tail, on sorted
+ * boundaries, with the same results.  Between launches the calling thread
+ * waits where the next launch depends on the device: for each solve's
+ * decision and each FBM round's flag, through the early stop signal
+ * (tsph_solver_begin_signal) without draining the stream.  It returns with
+ * the tail enqueued.  As after tsph_sort_object, *fluid's front and back
+ * state pointers are swapped, also when a later part fails.
+ */
+typedef struct TsphStep {
+  int32_t cfl, wcsph, fbm;
+  int32_t token;         /* last token used; advanced by each wait */
+  uint64_t *signal_host; /* 8 bytes of tsph_signal_alloc: the host's address, */
+  uint64_t *signal;      /* and the device's */
+  int32_t pred[2];       /* iterations of each solve launched before its first wait; on
+                            return those that ran (at least 1), the next step's guess */
+  int32_t iters[2];      /* out: iterations that ran (divergence, density) */
+  int32_t fbm_rounds;    /* out: FBM rounds launched */
+  int32_t pad;
+} TsphStep;
+int tsph_step(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphControl* ctrl,
+              TsphStep* step, void* workspace, size_t ws_bytes, void* stream);
 
 /*
  * map_velocity (sph.py:382-397) onto a Grid (sph_obj.py:328-344): node I of

@@ -89,6 +89,12 @@ class TsphBatchInfo(ctypes.Structure):
     _fields_ = [("nscenes", _i32), ("precision", _i32), ("tiles", _i32 * 4)]
 
 
+class TsphStep(ctypes.Structure):
+    _fields_ = [("cfl", _i32), ("wcsph", _i32), ("fbm", _i32), ("token", _i32),
+                ("signal_host", _vp), ("signal", _vp), ("pred", _i32 * 2), ("iters", _i32 * 2),
+                ("fbm_rounds", _i32), ("pad", _i32)]
+
+
 KERNEL_IDS = {
     "SPH_clean_value": 0, "cfl_condition": 1, "SPH_prepare_attr": 2,
     "SPH_prepare_alpha_1": 3, "SPH_prepare_alpha_2": 4, "SPH_prepare_alpha": 5,
@@ -114,7 +120,7 @@ EXPORTED = [
     "tsph_batch_solver_begin", "tsph_batch_solver_begin_signal", "tsph_batch_solver_psi",
     "tsph_batch_solver_update",
     "tsph_batch_advect", "tsph_batch_tail", "tsph_batch_stop_state", "tsph_map_velocity",
-    "tsph_wcsph", "tsph_sort_object_static", "tsph_sort_static_scratch_bytes",
+    "tsph_wcsph", "tsph_step", "tsph_sort_object_static", "tsph_sort_static_scratch_bytes",
     "tsph_sort_static_max_particles", "tsph_sort_static_max_cells",
 ]
 
@@ -192,6 +198,7 @@ def load(path=None):
         "tsph_batch_stop_state": [BI, _vp, _vp, _vp],
         "tsph_map_velocity": [P, O, _vp, _f64, _vp, _vp],
         "tsph_wcsph": [P, O, O, C, _vp],
+        "tsph_step": [P, O, O, C, ctypes.POINTER(TsphStep), _vp, sz, _vp],
     }
     for name, args in sigs.items():
         fn = getattr(lib, name)

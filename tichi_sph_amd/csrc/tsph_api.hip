@@ -115,7 +115,8 @@ int adj_bound_sums(const TsphParams&, TsphObject*, TsphObject*, TsphAdjoint*, hi
 template <class T>
 int advect(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
 template <class T>
-int fbm_round(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
+int fbm_round(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int,
+              hipStream_t);
 template <class T>
 int tail(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
 template <class T>
@@ -202,6 +203,34 @@ static int check_obj(const TsphObject* o, const char* what) {
   TSPH_REQUIRE(o->n >= 0 && o->n <= o->capacity, TSPH_ECAPACITY,
                "%s: part_num %d exceeds capacity %d", what, o->n, o->capacity);
   return 0;
+}
+
+// Waits until the device has stored `token` in the high half of *word and
+// done(low half) holds, or the stream has drained (a launch that never
+// signalled, or a failed one): then *low comes from read_device.  The pause
+// keeps the spin off the core's other thread; the stream is asked every few
+// thousand pauses (about 100 us) only.
+template <class Done, class Read>
+static int wait_word(const uint64_t* word, int32_t token, hipStream_t st, uint32_t* low,
+                     Done&& done, Read&& read_device) {
+  for (uint32_t spins = 1;; ++spins) {
+    const uint64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if ((uint32_t)(v >> 32) == (uint32_t)token && done((uint32_t)v)) {
+      *low = (uint32_t)v;
+      return 0;
+    }
+    __asm__ volatile("pause");
+    if (spins % 4096) continue;
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipErrorNotReady) continue;
+    TSPH_REQUIRE(e == hipSuccess, TSPH_EHIP, "tsph_step: %s", hipGetErrorString(e));
+    const uint64_t w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if ((uint32_t)(w >> 32) == (uint32_t)token && done((uint32_t)w)) {
+      *low = (uint32_t)w;
+      return 0;
+    }
+    return read_device(low);
+  }
 }
 
 }  // namespace tsph
@@ -374,7 +403,7 @@ int tsph_fbm_round(const TsphParams* p, TsphObject* f, TsphControl* ctrl, void* 
                    void* stream) {
   if (int rc = check_params(p)) return rc;
   if (int rc = check_obj(f, "tsph_fbm_round")) return rc;
-  return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, (hipStream_t)stream);
+  return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, (uint64_t*)nullptr, 0, (hipStream_t)stream);
 }
 
 int tsph_tail(const TsphParams* p, TsphObject* f, TsphControl* ctrl, int32_t fbm, void* ws,
@@ -453,6 +482,73 @@ int tsph_wcsph(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* c
   if (int rc = check_obj(b, "tsph_wcsph")) return rc;
   TSPH_REQUIRE(p->wc_gamma != 0, TSPH_EINVAL, "tsph_wcsph: solver_wc_gamma must be non-zero");
   return DISPATCH(p, wcsph, *p, f, b, ctrl, (hipStream_t)stream);
+}
+
+// One solve to its stop rule: `pred` iterations enqueued, then single ones
+// while the device says to go on.
+static int step_solve(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
+                      TsphStep* s, int solve, void* ws, size_t wsb, void* stream) {
+  const hipStream_t st = (hipStream_t)stream;
+  s->token = s->token % 0x7fffffff + 1;
+  if (int rc = tsph_solver_begin_signal(p, ctrl, solve, s->signal, s->token, stream)) return rc;
+  const int kmax = p->iter_max + 1;
+  int k = 0, it = 0, chunk = s->pred[solve] > 1 ? s->pred[solve] : 1;
+  while (k < kmax) {
+    for (int c = 0; c < chunk && k < kmax; ++c, ++k)
+      if (int rc = solver_entry(p, f, b, ctrl, k, 3, ws, wsb, stream)) return rc;
+    uint32_t w = 0;
+    // it and stop are the first two words after dt and compression
+    const int rc = wait_word(
+        s->signal_host, s->token, st, &w,
+        [&](uint32_t v) { return (v & 1) || (int)(v >> 1) >= k; },
+        [&](uint32_t* low) -> int {
+          int32_t is[2];
+          const hipError_t e = hipMemcpy(is, (const char*)ctrl + 16, sizeof(is), hipMemcpyDeviceToHost);
+          TSPH_REQUIRE(e == hipSuccess, TSPH_EHIP, "tsph_step: %s", hipGetErrorString(e));
+          *low = (uint32_t)(2 * is[0] + (is[1] ? 1 : 0));
+          return 0;
+        });
+    if (rc) return rc;
+    it = (int)(w >> 1);
+    if (w & 1) break;
+    chunk = 1;
+  }
+  s->iters[solve] = it;
+  s->pred[solve] = it > 1 ? it : 1;
+  return 0;
+}
+
+int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl, TsphStep* s,
+              void* ws, size_t wsb, void* stream) {
+  TSPH_REQUIRE(s && s->signal_host && s->signal, TSPH_EINVAL, "tsph_step: null step or signal");
+  if (int rc = tsph_sort_object(p, f, ctrl, s->cfl, ws, wsb, stream)) return rc;
+  if (int rc = tsph_density_alpha(p, f, b, ctrl, ws, wsb, stream)) return rc;
+  if (int rc = step_solve(p, f, b, ctrl, s, 0, ws, wsb, stream)) return rc;
+  if (int rc = tsph_advect(p, f, b, ctrl, ws, wsb, stream)) return rc;
+  if (int rc = step_solve(p, f, b, ctrl, s, 1, ws, wsb, stream)) return rc;
+  if (s->wcsph)
+    if (int rc = tsph_wcsph(p, f, b, ctrl, stream)) return rc;
+  s->fbm_rounds = 0;
+  while (s->fbm && f->n > 0 && s->fbm_rounds < 1000) {
+    const hipStream_t st = (hipStream_t)stream;
+    s->token = s->token % 0x7fffffff + 1;
+    if (int rc = DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, s->signal, (int)s->token, st))
+      return rc;
+    ++s->fbm_rounds;
+    uint32_t flag = 0;
+    const int rc = wait_word(
+        s->signal_host, s->token, st, &flag, [](uint32_t) { return true; },
+        [&](uint32_t* low) -> int {
+          int32_t v;
+          const hipError_t e = hipMemcpy(&v, &ctrl->general_flag, sizeof(v), hipMemcpyDeviceToHost);
+          TSPH_REQUIRE(e == hipSuccess, TSPH_EHIP, "tsph_step: %s", hipGetErrorString(e));
+          *low = (uint32_t)v;
+          return 0;
+        });
+    if (rc) return rc;
+    if (!flag) break;
+  }
+  return tsph_tail(p, f, ctrl, s->fbm, ws, wsb, stream);
 }
 
 int tsph_map_velocity(const TsphParams* p, const TsphObject* obj, const int32_t* grid_shape,

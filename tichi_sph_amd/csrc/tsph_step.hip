@@ -1226,12 +1226,19 @@ __global__ void __launch_bounds__(kBlock)
 
 // general_flag = any particle flagged this round (sph.py:368-372); skipped,
 // like the round itself, once the flag is clear.
+// With a signal, the flag also goes to the host: (token << 32) | flag.
 __global__ void __launch_bounds__(kBlock)
-    k_fbm_check_finish(const double* __restrict__ partial, int nblk, TsphControl* ctrl) {
+    k_fbm_check_finish(const double* __restrict__ partial, int nblk, TsphControl* ctrl,
+                       uint64_t* signal, int token) {
   __shared__ double lds[kWaves];
-  if (!ctrl->general_flag) return;
-  double a = sum_partials(partial, nblk, lds);
-  if (threadIdx.x == 0) ctrl->general_flag = a > 0 ? 1 : 0;
+  int flag = 0;
+  if (ctrl->general_flag) {
+    double a = sum_partials(partial, nblk, lds);
+    if (threadIdx.x == 0) ctrl->general_flag = flag = a > 0 ? 1 : 0;
+  }
+  if (signal && threadIdx.x == 0)
+    __hip_atomic_store(signal, ((uint64_t)(uint32_t)token << 32) | (uint32_t)flag,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------------
@@ -1471,7 +1478,7 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
 
 template <class T>
 int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws, size_t wsb,
-              hipStream_t st) {
+              uint64_t* signal, int token, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
@@ -1497,7 +1504,8 @@ int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws,
   hipLaunchKernelGGL(k_fbm_check<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                      (const T*)f->volume_frac, (const T*)f->volume_frac_tmp, f->flag, L.partial,
                      ctrl);
-  hipLaunchKernelGGL(k_fbm_check_finish, dim3(1), dim3(kBlock), 0, st, L.partial, nb, ctrl);
+  hipLaunchKernelGGL(k_fbm_check_finish, dim3(1), dim3(kBlock), 0, st, L.partial, nb, ctrl,
+                     signal, token);
   TSPH_LAUNCH_CHECK("fbm_round");
   return 0;
 }
@@ -1923,8 +1931,8 @@ template int solver_half<float>(const TsphParams&, TsphObject*, TsphObject*, Tsp
 template int solver_half<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, hipStream_t);
 template int advect<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
 template int advect<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
-template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
-template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
+template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
+template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
 template int tail<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
 template int tail<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
 

@@ -187,6 +187,8 @@ class Simulation:
             _lib.check(self.lib.tsph_signal_alloc(8, ctypes.byref(h), ctypes.byref(d)), "tsph_signal_alloc")
             self._signal_host, self._signal_dev = h, d
             self._signal_np = np.ctypeslib.as_array(ctypes.cast(h, ctypes.POINTER(ctypes.c_uint64)), shape=(1,))
+        self._step = _lib.TsphStep()  # tsph_step's options and results
+        self._step.signal_host, self._step.signal = self._signal_host, self._signal_dev
         self.ngrid = Ngrid(self)
         self.bound_dirty = True
         self.pred = [max(config.iter_threshold_min, 1), max(config.iter_threshold_min, 1)]
@@ -481,11 +483,14 @@ class Simulation:
         With no fluid particles it still sorts and updates the boundary, and
         each solve runs its minimum iteration count (the reference's empty
         mean is NaN)."""
+        if self.bound_needs_sort():
+            self._sort_bound()
+        if self.timer is None:
+            its = self._step_native()
+            return StepStats(self.control(), self.precision) if stats else its
         P = ctypes.byref(self.params)
         ws, wsb = self._ws()
         st = self.stream_ptr()
-        if self.bound_needs_sort():
-            self._sort_bound()
         self._call("sort", self.lib.tsph_sort_object, P, ctypes.byref(self.fluid.struct()), self.ctrl_ptr(),
                    1 if self.cfl else 0, ws, wsb, st)
         self.fluid.adopt_swaps()
@@ -508,6 +513,26 @@ class Simulation:
         if stats:
             return StepStats(self.control(), self.precision)
         return div_it, inc_it
+
+    def _step_native(self):
+        """sph_step's launches and waits in one library call (tsph_step).  A
+        timed step issues the same calls one by one instead, each between its
+        events.  Issued from Python a step takes the host 150 us, which is
+        more than the GPU needs for scenes below some 30 thousand particles."""
+        self._require_gpu("sph_step")
+        t, ws = self._step, self.ws
+        t.cfl, t.wcsph, t.fbm = bool(self.cfl), bool(self.wcsph), bool(self.fbm)
+        t.token = self._token
+        t.pred[0], t.pred[1] = self.pred
+        self.calls += 1
+        rc = self.lib.tsph_step(ctypes.byref(self.params), ctypes.byref(self.fluid.struct()),
+                                ctypes.byref(self.bound.struct()), self.ctrl.data_ptr(), ctypes.byref(t),
+                                ws.data_ptr(), ws.numel(), self.stream_ptr())
+        self._token = t.token
+        self.fluid.adopt_swaps()
+        _lib.check(rc, "tsph_step")
+        self.pred = [t.pred[0], t.pred[1]]
+        return t.iters[0], t.iters[1]
 
     # -------------------------------------------------- reference-order step
     def sph_step_reference(self, wcsph=None, fbm=None):

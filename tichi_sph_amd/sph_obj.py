@@ -164,11 +164,10 @@ class Fluid:
         descriptor again."""
         self.cell_table_ok = True
         self.layout_epoch += 1  # a SceneBatch holding this object's descriptor rebuilds it
-        s = self._struct
-        for name in ("pos", "vel", "mass", "rest_density", "rest_volume", "volume_frac", "pid"):
-            if getattr(s, name) != self.t[name].data_ptr():
-                self.t[name], self.t[name + "_b"] = self.t[name + "_b"], self.t[name]
-        self._refresh_struct()
+        t, s = self.t, self._struct
+        if s.pos != t["pos"].data_ptr():
+            for name in self._SWAPPED:
+                t[name], t[name + "_b"] = t[name + "_b"], t[name]
 
     @property
     def compression(self):
