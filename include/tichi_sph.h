@@ -104,7 +104,8 @@ typedef struct TsphObject {
   int32_t *cell_structured;                   /* [cap][4] neighb_cell_structured_seq */
   int32_t *in_cell;                           /* [cap] neighb_in_cell_seq */
   int32_t *cell_count, *cell_start;           /* [node_num + 2] per-object cell table */
-  int32_t *nbr_f, *nbr_b;                     /* [list_cap][cap] slot-major neighbour lists */
+  int32_t *nbr_f, *nbr_b;                     /* [list_cap][cap] slot-major neighbour lists (a capacity
+                                                 that is a multiple of 64 keeps rows on whole lines) */
   int32_t *nbr_nf, *nbr_nb;                   /* [cap] list lengths (cap+1 = overflow) */
   /* back buffers of the persistent state, swapped by tsph_sort_object */
   void *pos_b, *vel_b, *mass_b, *rest_density_b, *rest_volume_b, *volume_frac_b;

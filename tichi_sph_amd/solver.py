@@ -168,9 +168,8 @@ class Simulation:
                                                            list_cap_b)
         self.bound = bound if bound is not None else Fluid(config, bm, 1, device, precision, list_cap_f,
                                                            list_cap_b)
-        fm, bm = self.fluid.max_part_num, self.bound.max_part_num
         self.fluid.sim = self.bound.sim = self
-        cap = max(fm, 1) + max(bm, 1)
+        cap = self.fluid.capacity + self.bound.capacity
         self.ws = torch.zeros(int(self.lib.tsph_workspace_bytes(ctypes.byref(self.params), cap)),
                               dtype=torch.uint8, device=self.device)
         self.ctrl = torch.zeros(int(self.lib.tsph_control_bytes()), dtype=torch.uint8, device=self.device)
