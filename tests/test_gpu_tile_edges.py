@@ -108,3 +108,24 @@ def test_pass_a_by_quads_is_that_by_single_lanes(dim, precision, caps):
         assert np.array_equal(sims[0].bound.to_numpy(name), sims[1].bound.to_numpy(name), equal_nan=True), name
     for a, b in zip(_lists(sims[0]), _lists(sims[1])):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("block", BLOCKS, ids=lambda b: "x".join(map(str, b)))
+def test_reference_kernels_at_block_edges_match_oracle(block, precision):
+    """The sph.py kernels one by one (a quad of lanes per particle in the pair
+    kernels) against the oracle, bit for bit, with surface tension."""
+    from tichi_sph_amd import simulation_from_dicts
+    scn, cfg = scene(block)
+    cfg["solver_surface_tension_gamma"] = 0.07
+    print(f"[case] block {block} precision {precision}", flush=True)
+    sim = simulation_from_dicts(cfg, scn, precision=precision)
+    o = O.Oracle(cfg, scn, precision)
+    o.init_scenario()
+    d_it, i_it, _, _, _ = sim.sph_step_reference()
+    st = o.step(O.STEP_CFL)
+    assert (d_it, i_it) == (st.div_iter, st.incom_iter)
+    for obj, fl, names in ((0, sim.fluid, ("pos", "vel", "sph_density", "alpha", "psi_adv", "acce_adv", "normal")),
+                           (1, sim.bound, ("W", "sph_density", "alpha"))):
+        for f in names:
+            assert np.array_equal(fl.to_numpy(f), o.get(obj, f).reshape(fl.to_numpy(f).shape)), (obj, f)

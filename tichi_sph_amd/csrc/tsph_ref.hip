@@ -1,12 +1,12 @@
 // The reference's kernel surface on the GPU: each sph.py kernel with its
 // (ngrid, obj, nobj) signature, walking the shared Ngrid
 // (node_part_count / node_part_shift / part_pid_in_node / part_uid_in_node,
-// sph_obj.py:280-323) with the uid filter exactly as the reference does
-// (sph.py:9-19).  Strict arithmetic in the reference's evaluation order, one
-// thread per particle of `obj`, accumulation into the existing field values.
+// sph_obj.py:280-323) with the uid filter, in the reference's order
+// (sph.py:9-19).  Strict arithmetic in the reference's evaluation order,
+// accumulation into the existing field values.
 // These kernels are the drop-in for callers that drive the solver kernel by
 // kernel; the fused step (tsph_step.hip) is the fast path.
-#include "tsph_host.h"
+#include "tsph_sweep.h"
 
 namespace tsph {
 
@@ -128,54 +128,6 @@ __global__ void __launch_bounds__(kBlock)
         }
       }
       break;
-    case TSPH_K_SPH_prepare_attr:  // sph.py:50-64
-      if (act) {
-        V4<T> p = o.pos[i];
-        T w = o.W[i], cp = o.comp[i], dn = o.dens[i];
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j];
-          T Wr = s_W(k, ref_norm(p.x - q.x, p.y - q.y, p.z - q.z));
-          w = w + Wr;
-          cp = cp + Wr * no.rest_volume[j];
-          dn = dn + Wr * no.mass[j];
-        });
-        o.W[i] = w; o.comp[i] = cp; o.dens[i] = dn;
-      }
-      return;
-    case TSPH_K_SPH_prepare_alpha_1:  // sph.py:67-81
-      if (act) {
-        V4<T> p = o.pos[i];
-        V4<T> a = o.alpha_1[i];
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j];
-          T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-          T r = ref_norm(dx, dy, dz);
-          if (r > T(0)) {
-            T Xj = Xof(k, no, j), wg = s_Wg(k, r);
-            a.x = a.x + Xj * dx / r * wg;
-            a.y = a.y + Xj * dy / r * wg;
-            a.z = a.z + Xj * dz / r * wg;
-          }
-        });
-        o.alpha_1[i] = a;
-      }
-      return;
-    case TSPH_K_SPH_prepare_alpha_2:  // sph.py:84-97
-      if (act) {
-        V4<T> p = o.pos[i];
-        T a2 = o.alpha_2[i];
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j];
-          T r = ref_norm(p.x - q.x, p.y - q.y, p.z - q.z);
-          if (r > T(0)) {
-            T wg = s_Wg(k, r), Xj = Xof(k, no, j);
-            T wg2 = wg * wg;
-            a2 = a2 + wg2 * (Xj * Xj) / no.mass[j];
-          }
-        });
-        o.alpha_2[i] = a2;
-      }
-      return;
     case TSPH_K_SPH_prepare_alpha:  // sph.py:100-105
       if (act) {
         V4<T> a = o.alpha_1[i];
@@ -190,34 +142,6 @@ __global__ void __launch_bounds__(kBlock)
         o.acce_adv[i] = V4<T>{a.x + k.g[0], a.y + k.g[1], a.z + k.g[2], a.w};
       }
       return;
-    case TSPH_K_SPH_advection_viscosity_acc:  // sph.py:114-129
-      if (act) {
-        V4<T> p = o.pos[i], vi = o.vel[i], a = o.acce_adv[i];
-        T rd = o.rest_density[i];
-        const T mu = mu_of(k, o.vf, i);  // the global mu, or the per-phase extension
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j], vj = no.vel[j];
-          T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-          T r = ref_norm(dx, dy, dz);
-          if (r > T(0)) {
-            T Vj = Xof(k, no, j) / psiof(k, no, j);
-            T s = k.two_d2 * Vj * s_Wg(k, r);
-            T inv = T(1) / ref_norm(dx, dy, dz);
-            T Ax = (vi.x - vj.x) * dx;
-            Ax = Ax + (vi.y - vj.y) * dy;
-            if (k.dim == 3) Ax = Ax + (vi.z - vj.z) * dz;
-            T den = k.eps + r * r;
-            a.x = a.x + s * (inv * dx) * Ax / den * mu / rd;
-            a.y = a.y + s * (inv * dy) * Ax / den * mu / rd;
-            if (k.dim == 3) a.z = a.z + s * (inv * dz) * Ax / den * mu / rd;
-          }
-        });
-        o.acce_adv[i] = a;
-      }
-      return;
-    case TSPH_K_SPH_advection_surface_tension_acc:
-    case TSPH_K_SPH_FBM_convect:
-      return;  // two-loop kernels: launched as two passes by the host (see below)
     case TSPH_K_WC_pressure_val:  // sph.py:169-175
       if (act) {
         T cs2 = (T)(k.cs * k.cs);
@@ -234,48 +158,8 @@ __global__ void __launch_bounds__(kBlock)
         o.pressure[i] = pr;
       }
       return;
-    case TSPH_K_WC_pressure_acce:  // sph.py:178-193
-      if (act) {
-        V4<T> p = o.pos[i], a = o.acce_adv[i];
-        T pi = o.pressure[i], di = o.dens[i];
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j];
-          T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-          T r = ref_norm(dx, dy, dz);
-          T dj = no.dens[j];
-          T pt = pi / (di * di) + no.pressure[j] / (dj * dj);
-          if (r > T(0)) {
-            T wg = s_Wg(k, r);
-            T mj = no.mass[j];
-            a.x = a.x + -pt * mj * dx / r * wg;
-            a.y = a.y + -pt * mj * dy / r * wg;
-            if (k.dim == 3) a.z = a.z + -pt * mj * dz / r * wg;
-          }
-        });
-        o.acce_adv[i] = a;
-      }
-      return;
     case TSPH_K_IPPE_adv_psi_init:  // sph.py:196-199
       if (act) o.psi_adv[i] = psiof(k, o, i) - rpsiof(k, o, i);
-      return;
-    case TSPH_K_IPPE_adv_psi:  // sph.py:202-216
-      if (act) {
-        V4<T> p = o.pos[i], va = o.vel_adv[i];
-        T psi = o.psi_adv[i];
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j], vj = no.vel_adv[j];
-          T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-          T r = ref_norm(dx, dy, dz);
-          if (r > T(0)) {
-            T wg = s_Wg(k, r);
-            T dot = (dx / r * wg) * (va.x - vj.x);
-            dot = dot + (dy / r * wg) * (va.y - vj.y);
-            if (k.dim == 3) dot = dot + (dz / r * wg) * (va.z - vj.z);
-            psi = psi + dot * Xof(k, no, j) * dt;
-          }
-        });
-        o.psi_adv[i] = psi;
-      }
       return;
     case TSPH_K_IPPE_psi_adv_non_negative:  // sph.py:219-226
       if (act) {
@@ -285,28 +169,6 @@ __global__ void __launch_bounds__(kBlock)
         red0 = (double)(psi / rpsiof(k, o, i));
       }
       break;
-    case TSPH_K_IPPE_update_vel_adv:  // sph.py:229-244
-      if (act) {
-        V4<T> p = o.pos[i], va = o.vel_adv[i];
-        T pi = o.psi_adv[i], ai = o.alpha[i], Xi = Xof(k, o, i), mi = o.mass[i];
-        T c = -(T(1) / dt);
-        ref_walk(k, g, cs, no.uid, [&](int j) {
-          V4<T> q = no.pos[j];
-          T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-          T r = ref_norm(dx, dy, dz);
-          if (r > T(0)) {
-            T a = pi * Xof(k, no, j) / ai;
-            T b = no.psi_adv[j] * Xi / no.alpha[j];
-            T s = c * (a + b);
-            T wg = s_Wg(k, r);
-            va.x = va.x + s * (dx / r * wg) / mi;
-            va.y = va.y + s * (dy / r * wg) / mi;
-            if (k.dim == 3) va.z = va.z + s * (dz / r * wg) / mi;
-          }
-        });
-        o.vel_adv[i] = va;
-      }
-      return;
     case TSPH_K_SPH_advection_update_vel_adv:  // sph.py:247-250
       if (act) {
         V4<T> v = o.vel[i], a = o.acce_adv[i];
@@ -357,8 +219,9 @@ __global__ void __launch_bounds__(kBlock)
         for (int q = 0; q < P; ++q) acc[q] = o.vf_tmp[(long)i * P + q];
         T pre = dt * k.fbmD;
         ref_walk(k, g, cs, no.uid, [&](int j) {
-          if (no.flag[j] != 0) return;
           V4<T> q = no.pos[j];
+          if (!(s_r2(p.x - q.x, p.y - q.y, p.z - q.z) <= k.r2max)) return;  // exact zeros
+          if (no.flag[j] != 0) return;
           T r = ref_norm(p.x - q.x, p.y - q.y, p.z - q.z);
           if (r > T(0)) {
             T wg = s_Wg(k, r);
@@ -401,48 +264,197 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// Surface tension: loop 1 (normals) and loop 2 (forces), sph.py:134-166.
+// ---------------------------------------------------------------------------
+// The pair kernels, one instance per kernel id, a quad of lanes per particle
+// (tsph_sweep.h: walk_quad_cells): the quad tests the candidates of the Ngrid
+// four at a time and works off those in range, and every sum takes its terms
+// in the reference's order.  Beyond h the reference's terms are exact zeros
+// (W, W' and C vanish), so leaving them out changes no value.  One kernel with
+// a switch over all ids, one lane per particle and the whole pair math on each
+// of the 200 or so candidates took 130-170 us per call at 100k particles; these
+// take 36-66 us there, bound by the dependent loads of the walk (entry, then
+// position).  A whole reference step at 4k / 100k / 1M: 3.5 / 4.0 / 15.5 ms,
+// now 0.94 / 1.42 / 8.7.
+// ---------------------------------------------------------------------------
+constexpr int kRefNormal = 100, kRefForce = 101;  // surface tension's two loops
+
+// The walk around cell cs[] of particle p over nuid's candidates in range, or
+// (ALL) all of them with r > 0.
+template <bool ALL, class T, class Load, class Term>
+__device__ __forceinline__ void ref_quad(const KP<T>& k, const RefGrid& g, const int* cs, int nuid,
+                                         const V4<T>* __restrict__ npos, const V4<T>& p,
+                                         WalkLds& lds, Load&& load, Term&& term) {
+  walk_quad_cells(
+      k, cs, lds, [&](int lo, int hi) { return make_int2(g.nps[lo], g.nps[hi] + g.npc[hi]); },
+      [&](int s) {
+        Cand<T> d;
+        d.j = g.uin[s] == nuid ? g.pin[s] : -1;
+        d.q = d.j >= 0 ? npos[d.j] : p;
+        return d;
+      },
+      [&](const Cand<T>& d, bool* apart) {
+        const T r2 = s_r2(p.x - d.q.x, p.y - d.q.y, p.z - d.q.z);
+        *apart = r2 > T(0);  // as r > 0: the square root of a positive value is positive
+        return ALL ? *apart : r2 <= k.r2max;
+      },
+      load, term);
+}
+
 template <class T>
+struct RefRec {
+  V4<T> q, v;
+  T a, b, c;
+};
+
+template <class T, int KID>
 __global__ void __launch_bounds__(kBlock)
-    k_ref_st(int pass, KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no) {
+    k_ref_pair(KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no, const TsphControl* ctrl) {
   TSPH_STRICT
-  int i = blockIdx.x * kBlock + threadIdx.x;
+  __shared__ WalkLds lds;
+  const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= o.n) return;
+  const bool lead = coop_lane<kQuad>() == 0;
+  const T dt = (T)ctrl->dt;
+  const bool d3 = k.dim == 3;
   const int* cs = o.cs + 4 * i;
-  V4<T> p = o.pos[i];
-  if (pass == 0) {
-    T nx = 0, ny = 0, nz = 0;
-    ref_walk(k, g, cs, no.uid, [&](int j) {
-      V4<T> q = no.pos[j];
-      T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-      T r = ref_norm(dx, dy, dz);
-      if (r > T(0)) {
-        T s = -Xof(k, no, j) / psiof(k, no, j) * s_Wg(k, r);
-        nx = nx + s * dx / r;
-        ny = ny + s * dy / r;
-        nz = nz + s * dz / r;
-      }
-    });
-    o.normal[i] = V4<T>{nx * k.h, ny * k.h, nz * k.h, T(0)};
-    return;
-  }
-  V4<T> a = o.acce_adv[i];
-  V4<T> ni = o.normal[i];
-  T fi = o.vf[(long)i * k.P];
-  ref_walk(k, g, cs, no.uid, [&](int j) {
-    V4<T> q = no.pos[j];
-    T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    T r = ref_norm(dx, dy, dz);
-    if (r > T(0) && fi > T(0.99) && no.vf[(long)j * k.P] > T(0.99)) {
-      T cs2 = -k.gamma * no.mass[j] * s_C(k, r);
-      V4<T> nj = no.normal[j];
-      T f = T(2) * rpsiof(k, o, i) / (psiof(k, o, i) + psiof(k, no, j));
-      a.x = a.x + f * (cs2 * dx / r + k.gamma * (ni.x - nj.x));
-      a.y = a.y + f * (cs2 * dy / r + k.gamma * (ni.y - nj.y));
-      if (k.dim == 3) a.z = a.z + f * (cs2 * dz / r + k.gamma * (ni.z - nj.z));
+  const V4<T> p = o.pos[i];
+  // add(load, pair): pair(record, dx, dy, dz, r, on) with on = the lane holds
+  // a candidate (r > 0, except for W(0) in prepare_attr)
+  auto add = [&](auto&& load, auto&& pair) {
+    ref_quad<KID == kRefForce>(k, g, cs, no.uid, no.pos, p, lds, load,
+                               [&](const RefRec<T>& d, int, bool valid, bool apart) {
+                                 TSPH_STRICT
+                                 const T dx = p.x - d.q.x, dy = p.y - d.q.y, dz = p.z - d.q.z;
+                                 pair(d, dx, dy, dz, ref_norm(dx, dy, dz),
+                                      valid && (apart || KID == TSPH_K_SPH_prepare_attr));
+                               });
+  };
+  // acc + the quad's terms, component by component
+  auto add3 = [&](V4<T>& acc, T x, T y, T z, bool on) {
+    acc.x = quad_add(acc.x, on ? x : T(0));
+    acc.y = quad_add(acc.y, on ? y : T(0));
+    acc.z = quad_add(acc.z, on ? z : T(0));
+  };
+  if constexpr (KID == TSPH_K_SPH_prepare_attr) {  // sph.py:50-64
+    T w = o.W[i], cp = o.comp[i], dn = o.dens[i];
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, no.rest_volume[j], no.mass[j], T(0)}; },
+        [&](const RefRec<T>& d, T, T, T, T r, bool on) {
+          TSPH_STRICT
+          const T Wr = s_W(k, r);
+          w = quad_add(w, on ? Wr : T(0));
+          cp = quad_add(cp, on ? Wr * d.a : T(0));
+          dn = quad_add(dn, on ? Wr * d.b : T(0));
+        });
+    if (lead) {
+      o.W[i] = w;
+      o.comp[i] = cp;
+      o.dens[i] = dn;
     }
-  });
-  o.acce_adv[i] = a;
+  } else if constexpr (KID == TSPH_K_SPH_prepare_alpha_1) {  // sph.py:67-81
+    V4<T> a = o.alpha_1[i];
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, Xof(k, no, j), T(0), T(0)}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T wg = s_Wg(k, r);
+          add3(a, d.a * dx / r * wg, d.a * dy / r * wg, d.a * dz / r * wg, on);
+        });
+    if (lead) o.alpha_1[i] = a;
+  } else if constexpr (KID == TSPH_K_SPH_prepare_alpha_2) {  // sph.py:84-97
+    T a2 = o.alpha_2[i];
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, Xof(k, no, j), no.mass[j], T(0)}; },
+        [&](const RefRec<T>& d, T, T, T, T r, bool on) {
+          TSPH_STRICT
+          const T wg = s_Wg(k, r);
+          const T wg2 = wg * wg;
+          a2 = quad_add(a2, on ? wg2 * (d.a * d.a) / d.b : T(0));
+        });
+    if (lead) o.alpha_2[i] = a2;
+  } else if constexpr (KID == TSPH_K_SPH_advection_viscosity_acc) {  // sph.py:114-129
+    const V4<T> vi = o.vel[i];
+    V4<T> a = o.acce_adv[i];
+    const T rd = o.rest_density[i];
+    const T mu = mu_of(k, o.vf, i);  // the global mu, or the per-phase extension
+    add([&](int j) { return RefRec<T>{no.pos[j], no.vel[j], Xof(k, no, j), psiof(k, no, j), T(0)}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T Vj = d.a / d.b;
+          const T s = k.two_d2 * Vj * s_Wg(k, r);
+          const T inv = T(1) / ref_norm(dx, dy, dz);
+          T Ax = (vi.x - d.v.x) * dx;
+          Ax = Ax + (vi.y - d.v.y) * dy;
+          if (d3) Ax = Ax + (vi.z - d.v.z) * dz;
+          const T den = k.eps + r * r;
+          add3(a, s * (inv * dx) * Ax / den * mu / rd, s * (inv * dy) * Ax / den * mu / rd,
+               d3 ? s * (inv * dz) * Ax / den * mu / rd : T(0), on);
+        });
+    if (lead) o.acce_adv[i] = a;
+  } else if constexpr (KID == TSPH_K_WC_pressure_acce) {  // sph.py:178-193
+    V4<T> a = o.acce_adv[i];
+    const T pi = o.pressure[i], di = o.dens[i];
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, no.dens[j], no.pressure[j], no.mass[j]}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T pt = pi / (di * di) + d.b / (d.a * d.a);
+          const T wg = s_Wg(k, r);
+          add3(a, -pt * d.c * dx / r * wg, -pt * d.c * dy / r * wg,
+               d3 ? -pt * d.c * dz / r * wg : T(0), on);
+        });
+    if (lead) o.acce_adv[i] = a;
+  } else if constexpr (KID == TSPH_K_IPPE_adv_psi) {  // sph.py:202-216
+    const V4<T> va = o.vel_adv[i];
+    T psi = o.psi_adv[i];
+    add([&](int j) { return RefRec<T>{no.pos[j], no.vel_adv[j], Xof(k, no, j), T(0), T(0)}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T wg = s_Wg(k, r);
+          T dot = (dx / r * wg) * (va.x - d.v.x);
+          dot = dot + (dy / r * wg) * (va.y - d.v.y);
+          if (d3) dot = dot + (dz / r * wg) * (va.z - d.v.z);
+          psi = quad_add(psi, on ? dot * d.a * dt : T(0));
+        });
+    if (lead) o.psi_adv[i] = psi;
+  } else if constexpr (KID == TSPH_K_IPPE_update_vel_adv) {  // sph.py:229-244
+    V4<T> va = o.vel_adv[i];
+    const T pi = o.psi_adv[i], ai = o.alpha[i], Xi = Xof(k, o, i), mi = o.mass[i];
+    const T c = -(T(1) / dt);
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, Xof(k, no, j), no.psi_adv[j], no.alpha[j]}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T a = pi * d.a / ai;
+          const T b = d.b * Xi / d.c;
+          const T s = c * (a + b);
+          const T wg = s_Wg(k, r);
+          add3(va, s * (dx / r * wg) / mi, s * (dy / r * wg) / mi,
+               d3 ? s * (dz / r * wg) / mi : T(0), on);
+        });
+    if (lead) o.vel_adv[i] = va;
+  } else if constexpr (KID == kRefNormal) {  // sph.py:141-149
+    V4<T> n{};
+    add([&](int j) { return RefRec<T>{no.pos[j], V4<T>{}, Xof(k, no, j), psiof(k, no, j), T(0)}; },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T s = -d.a / d.b * s_Wg(k, r);
+          add3(n, s * dx / r, s * dy / r, s * dz / r, on);
+        });
+    if (lead) o.normal[i] = V4<T>{n.x * k.h, n.y * k.h, n.z * k.h, T(0)};
+  } else {  // kRefForce, sph.py:151-166: over all candidates with r > 0
+    if (!(o.vf[(long)i * k.P] > T(0.99))) return;  // the whole quad: one particle
+    V4<T> a = o.acce_adv[i];
+    const V4<T> ni = o.normal[i];
+    const T ri = rpsiof(k, o, i), pi = psiof(k, o, i);
+    add([&](int j) {
+          return RefRec<T>{no.pos[j], no.normal[j], no.mass[j], psiof(k, no, j), no.vf[(long)j * k.P]};
+        },
+        [&](const RefRec<T>& d, T dx, T dy, T dz, T r, bool on) {
+          TSPH_STRICT
+          const T cs2 = -k.gamma * d.a * s_C(k, r);
+          const T f = T(2) * ri / (pi + d.b);
+          add3(a, f * (cs2 * dx / r + k.gamma * (ni.x - d.v.x)),
+               f * (cs2 * dy / r + k.gamma * (ni.y - d.v.y)),
+               d3 ? f * (cs2 * dz / r + k.gamma * (ni.z - d.v.z)) : T(0), on && d.c > T(0.99));
+        });
+    if (lead) o.acce_adv[i] = a;
+  }
 }
 
 // SPH_FBM_convect loop 1 (drift velocities) and loop 2 (flux), sph.py:329-363.
@@ -491,9 +503,10 @@ __global__ void __launch_bounds__(kBlock)
   for (int q = 0; q < P; ++q) acc[q] = o.vf_tmp[(long)i * P + q];
   T pre = k.fbmC * dt;
   ref_walk(k, g, cs, no.uid, [&](int j) {
-    if (no.flag[j] != 0) return;
     V4<T> q = no.pos[j];
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+    if (!(s_r2(dx, dy, dz) <= k.r2max)) return;  // exact zeros
+    if (no.flag[j] != 0) return;
     T r = ref_norm(dx, dy, dz);
     if (r > T(0)) {
       T wg = s_Wg(k, r);
@@ -524,9 +537,28 @@ int ref_kernel(const TsphParams& prm, int kid, TsphObject* obj, const TsphObject
   RefObj<T> o = ref_obj<T>(obj);
   RefObj<T> no = ref_obj<T>(nobj ? nobj : obj);
   int nb = blocks_for(obj->n > 0 ? obj->n : 1);
-  if (kid == TSPH_K_SPH_advection_surface_tension_acc) {
-    hipLaunchKernelGGL(k_ref_st<T>, dim3(nb), dim3(kBlock), 0, st, 0, k, g, o, no);
-    hipLaunchKernelGGL(k_ref_st<T>, dim3(nb), dim3(kBlock), 0, st, 1, k, g, o, no);
+  auto pair = [&](auto kern) {
+    if (o.n > 0)
+      hipLaunchKernelGGL(kern, dim3(coop_blocks<kQuad>(o.n)), dim3(kBlock), 0, st, k, g, o, no,
+                         ctrl);
+  };
+  if (kid == TSPH_K_SPH_prepare_attr) {
+    pair(k_ref_pair<T, TSPH_K_SPH_prepare_attr>);
+  } else if (kid == TSPH_K_SPH_prepare_alpha_1) {
+    pair(k_ref_pair<T, TSPH_K_SPH_prepare_alpha_1>);
+  } else if (kid == TSPH_K_SPH_prepare_alpha_2) {
+    pair(k_ref_pair<T, TSPH_K_SPH_prepare_alpha_2>);
+  } else if (kid == TSPH_K_SPH_advection_viscosity_acc) {
+    pair(k_ref_pair<T, TSPH_K_SPH_advection_viscosity_acc>);
+  } else if (kid == TSPH_K_WC_pressure_acce) {
+    pair(k_ref_pair<T, TSPH_K_WC_pressure_acce>);
+  } else if (kid == TSPH_K_IPPE_adv_psi) {
+    pair(k_ref_pair<T, TSPH_K_IPPE_adv_psi>);
+  } else if (kid == TSPH_K_IPPE_update_vel_adv) {
+    pair(k_ref_pair<T, TSPH_K_IPPE_update_vel_adv>);
+  } else if (kid == TSPH_K_SPH_advection_surface_tension_acc) {
+    pair(k_ref_pair<T, kRefNormal>);
+    if (k.gamma != T(0)) pair(k_ref_pair<T, kRefForce>);  // else every term is an exact zero
   } else if (kid == TSPH_K_SPH_FBM_convect) {
     hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 0, k, g, o, no, ctrl);
     hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 1, k, g, o, no, ctrl);

@@ -382,19 +382,24 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// load(j) gathers what the pair terms need of candidate j; term(record, j,
-// valid, apart) adds one list slot per lane (valid: the lane holds one;
-// apart: r > 0) and runs with the whole quad.  Candidates in range are those
-// with r^2 <= r2max.
-template <class T, class Load, class Term>
-__device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict__ cstart,
-                                          const V4<T>* __restrict__ pos, const V4<T>& p,
-                                          WalkLds& lds, Load&& load, Term&& term) {
+// The walk around cell cc[].  bounds(lo, hi) is the range of candidates of the
+// cells lo .. hi (one row run); fetch(s) is candidate s of it; take(fetched,
+// &apart) says whether it belongs to the list, and apart whether r > 0 (r = 0
+// goes to the list with a mark).  load(j) gathers what the pair terms need of
+// candidate j; term(record, j, valid, apart) adds one list slot per lane
+// (valid: the lane holds one) and runs with the whole quad.
+template <class T>
+struct Cand {
+  V4<T> q;
+  int j;  // negative: none
+};
+template <class T, class Bounds, class Fetch, class Take, class Load, class Term>
+__device__ __forceinline__ void walk_quad_cells(const KP<T>& k, const int* cc, WalkLds& lds,
+                                                Bounds&& bounds, Fetch&& fetch, Take&& take,
+                                                Load&& load, Term&& term) {
   const int c = threadIdx.x & (kQuad - 1), g = threadIdx.x / kQuad;
   const unsigned below = (1u << c) - 1;
   const int R = k.R, side = 2 * R + 1, rows = k.dim == 3 ? side * side : side;
-  int cc[3];
-  node_encode(k, p.x, p.y, p.z, cc);
   for (int row0 = 0; row0 < rows; row0 += kWalkRows) {
     int nrun = 0;
 #pragma unroll
@@ -407,7 +412,7 @@ __device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict_
         const long lo = c0 < 1 ? 1 : (long)c0;
         long hi = (long)c0 + 2 * R;
         if (hi > k.node_num - 1) hi = k.node_num - 1;
-        if (lo <= hi) run = make_int2(cstart[lo], cstart[hi + 1]);
+        if (lo <= hi) run = bounds((int)lo, (int)hi);
       }
       const unsigned v = quad_vote(run.x < run.y);
       if (run.x < run.y) lds.run[nrun + __popc(v & below)][g] = run;
@@ -417,17 +422,19 @@ __device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict_
     wave_lds_fence();
     int at = 0, j = lds.run[0][g].x, end = lds.run[0][g].y, cnt = 0;
     bool more = true;
-    int cj[kWalkU];
-    V4<T> cq[kWalkU];
+    Cand<T> cur[kWalkU];
+    auto trip = [&](Cand<T>* d) {
 #pragma unroll
-    for (int u = 0; u < kWalkU; ++u) {
-      cj[u] = j + c + kQuad * u;
-      cq[u] = pos[min(cj[u], end - 1)];
-    }
+      for (int u = 0; u < kWalkU; ++u) {
+        const int s = j + c + kQuad * u;
+        d[u] = fetch(s < end ? s : end - 1);
+        if (s >= end) d[u].j = -1;
+      }
+    };
+    trip(cur);
     while (more) {
       while (more && cnt <= kWalkS - kQuad * kWalkU) {
         // the next trip's candidates are requested before this one's tests
-        const int cend = end;
         j += kQuad * kWalkU;
         if (j >= end) {
           ++at;
@@ -438,30 +445,20 @@ __device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict_
             end = run.y;
           }
         }
-        int nj[kWalkU];
-        V4<T> nq[kWalkU];
-        if (more) {
-#pragma unroll
-          for (int u = 0; u < kWalkU; ++u) {
-            nj[u] = j + c + kQuad * u;
-            nq[u] = pos[min(nj[u], end - 1)];
-          }
-        }
+        Cand<T> nxt[kWalkU];
+        if (more) trip(nxt);
 #pragma unroll
         for (int u = 0; u < kWalkU; ++u) {
-          const T r2 = s_r2(p.x - cq[u].x, p.y - cq[u].y, p.z - cq[u].z);
-          const bool take = r2 <= k.r2max && cj[u] < cend;
-          const unsigned v = quad_vote(take);
+          bool apart;
+          const bool hit = take(cur[u], &apart) && cur[u].j >= 0;
+          const unsigned v = quad_vote(hit);
           // the sign bit marks a candidate at r = 0
-          if (take) lds.list[cnt + __popc(v & below)][g] = r2 > T(0) ? cj[u] : ~cj[u];
+          if (hit) lds.list[cnt + __popc(v & below)][g] = apart ? cur[u].j : ~cur[u].j;
           cnt += __popc(v);
         }
         if (more) {
 #pragma unroll
-          for (int u = 0; u < kWalkU; ++u) {
-            cj[u] = nj[u];
-            cq[u] = nq[u];
-          }
+          for (int u = 0; u < kWalkU; ++u) cur[u] = nxt[u];
         }
       }
       wave_lds_fence();
@@ -480,6 +477,25 @@ __device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict_
       cnt = 0;
     }
   }
+}
+
+// The walk of an object in cell order around p, taking the candidates in range
+// (r^2 <= r2max).
+template <class T, class Load, class Term>
+__device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict__ cstart,
+                                          const V4<T>* __restrict__ pos, const V4<T>& p,
+                                          WalkLds& lds, Load&& load, Term&& term) {
+  int cc[3];
+  node_encode(k, p.x, p.y, p.z, cc);
+  walk_quad_cells(
+      k, cc, lds, [&](int lo, int hi) { return make_int2(cstart[lo], cstart[hi + 1]); },
+      [&](int s) { return Cand<T>{pos[s], s}; },
+      [&](const Cand<T>& d, bool* apart) {
+        const T r2 = s_r2(p.x - d.q.x, p.y - d.q.y, p.z - d.q.z);
+        *apart = r2 > T(0);
+        return r2 <= k.r2max;
+      },
+      load, term);
 }
 
 }  // namespace tsph
