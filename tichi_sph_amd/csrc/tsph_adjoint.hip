@@ -375,6 +375,11 @@ __global__ void __launch_bounds__(kBlock)
   brec[i] = V4<T>{s * u.x, s * u.y, s * u.z, T(0)};
 }
 
+// A quad of lanes per particle, as in the forward walk, with kStRevU candidate
+// records of two gathers each in flight per lane.  At 200k particles, one lane
+// with 4 in flight 90 us; quads with 1 / 2 / 3 / 4 / 6 in flight 75 / 72 / 74 /
+// 92 (with a branch per candidate) / 79 us.
+constexpr int kStRevU = 2;
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_adj_surface_tension(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
@@ -387,7 +392,8 @@ __global__ void __launch_bounds__(kBlock)
                           V4<T>* __restrict__ xbar, double* __restrict__ partial,
                           const TsphControl* ctrl) {
   __shared__ double lds[kWaves];
-  const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int cl = coop_lane<kQuad>();
   double gsum = 0;
   if (i < n) {
     const T dt = (T)ctrl->dt;
@@ -410,15 +416,15 @@ __global__ void __launch_bounds__(kBlock)
       // spare lane (negative where j's 0.99 gate fails; the forward advection
       // writes it) and b_j
       auto loadn = [&](int j) { return Rec2<T>{tnormal[j], brec[j]}; };
-      walk_cells_prefetch<kStU>(k, fstart, c, loadn, [&](int j, const Rec2<T>& d) {
-        if (j == i || !(d.a.w > T(0))) return;
-        if (j >= own0 && j < own1) {
+      walk_quad_all<kStRevU>(k, fstart, c, loadn, [&](int j, const Rec2<T>& d, bool valid) {
+        bool on = valid && j != i && d.a.w > T(0);
+        if (on && j >= own0 && j < own1) {
           const V4<T> q = fpos[j];
-          if (!(s_r2(p.x - q.x, p.y - q.y, p.z - q.z) > T(0))) return;
+          on = s_r2(p.x - q.x, p.y - q.y, p.z - q.z) > T(0);
         }
         const V4<T>& nj = d.a;
         const V4<T>& bj = d.b;
-        const T rden = f_rcp(rhoi + nj.w);
+        const T rden = on ? f_rcp(rhoi + nj.w) : T(0);  // a factor of every term
         const T fij = T(2) * r0i * rden, r2d = T(2) * rden;
         const T dnx = ni.x - nj.x, dny = ni.y - nj.y, dnz = ni.z - nj.z;
         // e_lj = f_lj a_l - f_jl a_j
@@ -460,22 +466,25 @@ __global__ void __launch_bounds__(kBlock)
         az += -gam * (cr * wz + s * dz);
         rb += -gam * rden * (r2d * mi * cr * bd - fij * mj * cr * ad);
       };
-      const int nf = nbr_nf[i];
-      if (nf <= k.list_cap_f) {
-        sweep_one_list_coop<1, Rec3<T>, 2>(cap, i, 0, nbr_f, nf, loadc, coh);
-      } else {
-        walk_cells(k, fstart, c, [&](int j) {
-          const V4<T> q = fpos[j];
-          const T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
-          if (r2 > T(0) && r2 <= k.r2max) coh(loadc(j), true);
-        });
-      }
+      sweep_lists_coop<kQuad, T, Rec3<T>, 2>(
+          k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, loadc,
+          loadc, coh, [&](const Rec3<T>&, bool) {});
+      nbx = group_sum<kQuad>(nbx);
+      nby = group_sum<kQuad>(nby);
+      nbz = group_sum<kQuad>(nbz);
+      ax = group_sum<kQuad>(ax);
+      ay = group_sum<kQuad>(ay);
+      az = group_sum<kQuad>(az);
+      rb = group_sum<kQuad>(rb);
+      gs = group_sum<kQuad>(gs);
     }
-    nbar[i] = v4(nbx, nby, nbz);
-    rhobar[i] += rb;
-    V4<T> xb = xbar[i];
-    xbar[i] = v4(xb.x + ax, xb.y + ay, xb.z + az);
-    gsum = (double)gs;
+    if (cl == 0) {
+      nbar[i] = v4(nbx, nby, nbz);
+      rhobar[i] += rb;
+      V4<T> xb = xbar[i];
+      xbar[i] = v4(xb.x + ax, xb.y + ay, xb.z + az);
+      gsum = (double)gs;
+    }
   }
   double s = block_sum(gsum, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
@@ -769,14 +778,15 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
     // forward Jacobi iterations)
     hipLaunchKernelGGL(k_adj_st_rec<T>, dim3(nb), dim3(kBlock), 0, st, f->n,
                        (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.krec, ctrl);
-    hipLaunchKernelGGL(k_adj_surface_tension<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
+    hipLaunchKernelGGL(k_adj_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
                        f->capacity, (const V4<T>*)f->pos, (const T*)f->mass,
                        (const T*)f->sph_density, (const T*)f->rest_density,
                        (const T*)f->volume_frac, f->cell_start, f->nbr_f, f->nbr_nf,
                        (const V4<T>*)a->tape_normal, (const V4<T>*)a->vbar,
                        (const V4<T>*)L.krec, (V4<T>*)a->nbar,
                        (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
-    hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial, nb, a->grad, 1);
+    hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
+                       coop_blocks<kQuad>(f->n), a->grad, 1);
   }
   // (dt vbar, fv) per particle into the workspace's boundary alpha_1 buffer
   // (pass A's output for the forward psi sweeps, free during a reverse)

@@ -907,9 +907,12 @@ __global__ void __launch_bounds__(kBlock)
 // beyond h, so it is summed over the in-range list.  Both terms share the
 // factor 2 psi_0 / (psi_i + psi_j) and gamma.  With gamma == 0 every term is
 // an exact zero and only the update runs.
-// Candidate records in flight per lane of the forward curvature walk.
-constexpr int kStFwdU = 8;
-template <class T>
+// A quad of lanes per particle, kStFwdU gathers in flight per lane: a row run
+// holds about 24 candidates, one trip of six.  us, one lane with 8 in flight /
+// quads with 2, 3, 4, 6, 7, 8: 4k 29 / 14.3, 12.4, 13.4, 11.8, 12.5, 12.3; 200k
+// 50 / 52, 50, 57, 46, 49, 54; 2M 246 / 259, 244, 276, 229, 245, 266.
+constexpr int kStFwdU = 6;
+template <class T, int R = 1>
 __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, int n, int cap,
                       const V4<T>* __restrict__ fpos, const T* __restrict__ psi_rho,
                       const T* __restrict__ rdens, const T* __restrict__ vf,
@@ -918,68 +921,65 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
                       const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
                       V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
                       const TsphControl* ctrl) {
-  int i = xcd_block(blk.b, blk.nb) * kBlock + threadIdx.x;
-  if (i >= n) return;
+  const int cl = coop_lane<kQuad>();
   const T dt = (T)ctrl->dt;
-  V4<T> a = acce_adv[i];
-  if (k.gamma != T(0) && vf[(long)i * k.P] > T(0.99)) {
-    V4<T> p = fpos[i];
-    V4<T> ni = normal[i];
-    T rp = rest_psi_of(k, rdens, i);
-    T psi_i = psi_rho[i];
-    int c[3];
-    node_encode(k, p.x, p.y, p.z, c);
-    // the normal record's spare lane holds +-psi_j, negative where j's 0.99
-    // gate fails (the advection sweep writes it).  Reciprocal square root
-    // and reciprocals instead of the IEEE forms: the pair terms of these
-    // sums are not part of the bit-exact sums.
-    T ux = 0, uy = 0, uz = 0;  // sum of (n_i - n_j) / (psi_i + psi_j)
-    walk_cells_prefetch<kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
-                                 [&](int j, const V4<T>& nj) {
-      if (j != i && nj.w > T(0)) {
-        const T w = f_rcp(psi_i + nj.w);
+#pragma unroll 1
+  for (int r = 0; r < R; ++r) {
+    const int i = coop_particle<kQuad>(coop_sub<R>(blk, r));
+    if (i >= n) break;
+    V4<T> a = acce_adv[i];
+    if (k.gamma != T(0) && vf[(long)i * k.P] > T(0.99)) {
+      V4<T> p = fpos[i];
+      V4<T> ni = normal[i];
+      T rp = rest_psi_of(k, rdens, i);
+      T psi_i = psi_rho[i];
+      int c[3];
+      node_encode(k, p.x, p.y, p.z, c);
+      // the normal record's spare lane holds +-psi_j, negative where j's 0.99
+      // gate fails (the advection sweep writes it).  Reciprocal square root
+      // and reciprocals instead of the IEEE forms: the pair terms of these
+      // sums are not part of the bit-exact sums.
+      T ux = 0, uy = 0, uz = 0;  // sum of (n_i - n_j) / (psi_i + psi_j)
+      walk_quad_all<kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
+                             [&](int j, const V4<T>& nj, bool valid) {
+        const T w = valid && j != i && nj.w > T(0) ? f_rcp(psi_i + nj.w) : T(0);
         ux += w * (ni.x - nj.x);
         uy += w * (ni.y - nj.y);
         uz += w * (ni.z - nj.z);
-      }
-    });
-    // per in-range neighbour: (x_j, m_j) and the normal record
-    auto load = [&](int j) { return Rec2<T>{strec[j], normal[j]}; };
-    T hx = 0, hy = 0, hz = 0;  // sum of m_j C(r) x_ij / r / (psi_i + psi_j)
-    auto coh = [&](const Rec2<T>& d) {
-      if (d.b.w > T(0)) {
+      });
+      // per in-range neighbour: (x_j, m_j) and the normal record
+      auto load = [&](int j) { return Rec2<T>{strec[j], normal[j]}; };
+      auto coh = [&](const Rec2<T>& d, bool ok) {  // - m_j C(r) x_ij / r / (psi_i + psi_j)
         const V4<T>& q = d.a;
         const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         const T r2 = dx * dx + dy * dy + dz * dz;
         const T rinv = f_rsqrt(r2);
-        const T s = q.w * f_coh(k, r2 * rinv * k.inv_h) * rinv * f_rcp(psi_i + d.b.w);
-        hx += s * dx;
-        hy += s * dy;
-        hz += s * dz;
-      }
-    };
-    const int nf = nbr_nf[i];
-    if (nf <= k.list_cap_f) {
-      sweep_one_list<Rec2<T>>(cap, i, nbr_f, nf, load, coh);
-    } else {
-      walk_cells(k, fstart, c, [&](int j) {
-        const V4<T> q = fpos[j];
-        const T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
-        if (r2 > T(0) && r2 <= k.r2max) coh(load(j));
-      });
+        T s = q.w * f_coh(k, r2 * rinv * k.inv_h) * rinv * f_rcp(psi_i + d.b.w);
+        s = ok && d.b.w > T(0) ? s : T(0);
+        ux -= s * dx;
+        uy -= s * dy;
+        uz -= s * dz;
+      };
+      sweep_lists_coop<kQuad, T, Rec2<T>>(
+          k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, load,
+          load, coh, [&](const Rec2<T>&, bool) {});
+      ux = group_sum<kQuad>(ux);
+      uy = group_sum<kQuad>(uy);
+      uz = group_sum<kQuad>(uz);
+      // 2 psi_0 / (psi_i + psi_j) (cohesion + curvature), cohesion =
+      // -gamma m_j C(r) x_ij / r, curvature = gamma (n_i - n_j)
+      const T f = T(2) * rp * k.gamma;
+      a.x += f * ux;
+      a.y += f * uy;
+      a.z += f * uz;
+      if (cl == 0) acce_adv[i] = a;
     }
-    // 2 psi_0 / (psi_i + psi_j) (cohesion + curvature), cohesion =
-    // -gamma m_j C(r) x_ij / r, curvature = gamma (n_i - n_j)
-    const T f = T(2) * rp * k.gamma;
-    a.x += f * (ux - hx);
-    a.y += f * (uy - hy);
-    a.z += f * (uz - hz);
-    acce_adv[i] = a;
-  }
-  {
-    TSPH_STRICT  // SPH_advection_update_vel_adv, sph.py:247-250
-    const V4<T> v = vel[i];
-    vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
+    if (cl != 0) continue;
+    {
+      TSPH_STRICT  // SPH_advection_update_vel_adv, sph.py:247-250
+      const V4<T> v = vel[i];
+      vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
+    }
   }
 }
 
@@ -1467,7 +1467,7 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
     hipLaunchKernelGGL(k_vel_adv_update<T>, dim3(nb), dim3(kBlock), 0, st, f->n,
                        (const V4<T>*)f->vel, (const V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl);
   else
-    hipLaunchKernelGGL(k_surface_tension<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
+    hipLaunchKernelGGL(k_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
                        f->capacity, (const V4<T>*)f->pos, psi, (const T*)f->rest_density,
                        (const T*)f->volume_frac, f->cell_start, (const V4<T>*)f->normal,
                        (const V4<T>*)L.krec, f->nbr_f, f->nbr_nf, (const V4<T>*)f->vel,
@@ -1797,11 +1797,11 @@ __global__ void __launch_bounds__(kBlock) kb_advect(const char* __restrict__ tab
   });
 }
 
-template <class T>
+template <class T, int R>
 __global__ void __launch_bounds__(kBlock) kb_surface_tension(const char* __restrict__ tab, int ns) {
-  for_tiles<T, kTileFluid>(tab, ns, [&](const SceneEntry<T>& e, int, Blk blk) {
+  for_coop_tiles<T, kQuad, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_surface_tension_body<T>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e),
+    k_surface_tension_body<T, R>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e),
                               (const T*)f.rest_density, (const T*)f.volume_frac, f.cell_start,
                               (const V4<T>*)f.normal, (const V4<T>*)e.L.krec, f.nbr_f, f.nbr_nf,
                               (const V4<T>*)f.vel, (V4<T>*)f.acce_adv, (V4<T>*)f.vel_adv, e.ctrl);
@@ -1888,7 +1888,12 @@ int batch_advect(const TsphBatchInfo& bi, char* tab, int grid, hipStream_t st) {
                        tab, bi.nscenes);
   else
     hipLaunchKernelGGL((kb_advect<T, kCoop>), dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
-  hipLaunchKernelGGL(kb_surface_tension<T>, dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
+  if (coop_split(tiles))
+    hipLaunchKernelGGL((kb_surface_tension<T, 1>), dim3(grid_for(tiles * kQuad, grid)),
+                       dim3(kBlock), 0, st, tab, bi.nscenes);
+  else
+    hipLaunchKernelGGL((kb_surface_tension<T, kQuad>), dim3(g), dim3(kBlock), 0, st, tab,
+                       bi.nscenes);
   TSPH_LAUNCH_CHECK("batch_advect");
   return 0;
 }

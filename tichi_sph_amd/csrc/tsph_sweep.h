@@ -69,7 +69,6 @@ __device__ __forceinline__ void walk_cells_batched(const KP<T>& k, const int* __
   walk_cells_prefetch<U>(k, cstart, c, [&](int j) { return pos[j]; }, f);
 }
 constexpr int kPassAU = 4;
-constexpr int kStU = 4;  // prefetch depth of the surface-tension cell walks
 
 template <class T>
 __device__ __forceinline__ T rest_psi_of(const KP<T>& k, const T* rdens, int i) {
@@ -111,71 +110,6 @@ __device__ __forceinline__ void for_bound_nbrs(const KP<T>& k, int i, int cap, i
       if (r2 > T(0) && r2 <= k.r2max) f(j);
     });
   }
-}
-
-// Neighbour iteration of the list sweeps for one lane, in the recorded
-// (reference) order: fluid list, then boundary list.  The sweeps are bound
-// by the latency of dependent loads (list entry -> neighbour data), so the
-// lists are consumed in batches of kNb: all kNb indices are loaded, then all
-// their neighbour records, then the pair terms are applied in order.  A lane
-// whose list overflowed walks the cells with the same in-range test.
-constexpr int kNb = 8;
-
-// One list, software-pipelined: the next batch's list entries are loaded
-// right after this batch's records are requested, so a batch costs one
-// round trip to memory instead of two (index, then record).
-template <class Rec, class Load, class Pair>
-__device__ __forceinline__ void sweep_one_list(int cap, int i, const int* __restrict__ list, int n,
-                                               Load&& load, Pair&& pair) {
-  int j[kNb];
-#pragma unroll
-  for (int u = 0; u < kNb; ++u) j[u] = u < n ? list[(long)u * cap + i] : -1;
-  for (int s0 = 0; s0 < n; s0 += kNb) {
-    Rec d[kNb];
-#pragma unroll
-    for (int u = 0; u < kNb; ++u)
-      if (j[u] >= 0) d[u] = load(j[u]);
-    int jn[kNb];
-#pragma unroll
-    for (int u = 0; u < kNb; ++u) {
-      const int s = s0 + kNb + u;
-      jn[u] = s < n ? list[(long)s * cap + i] : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < kNb; ++u)
-      if (j[u] >= 0) pair(d[u]);
-#pragma unroll
-    for (int u = 0; u < kNb; ++u) j[u] = jn[u];
-  }
-}
-
-template <class T, class Rec, class LoadF, class LoadB, class PairF, class PairB>
-__device__ __forceinline__ void sweep_lists(const KP<T>& k, int cap, int i, V4<T> p,
-                                            const int* __restrict__ fstart,
-                                            const int* __restrict__ bstart,
-                                            const V4<T>* __restrict__ fpos,
-                                            const V4<T>* __restrict__ bpos,
-                                            const int* __restrict__ nbr_f,
-                                            const int* __restrict__ nbr_b, int nf, int nbb,
-                                            LoadF&& load_f, LoadB&& load_b, PairF&& pair_f,
-                                            PairB&& pair_b) {
-  if (nf <= k.list_cap_f && nbb <= k.list_cap_b) {
-    sweep_one_list<Rec>(cap, i, nbr_f, nf, load_f, pair_f);
-    if (nbb > 0) sweep_one_list<Rec>(cap, i, nbr_b, nbb, load_b, pair_b);
-    return;
-  }
-  int c[3];
-  node_encode(k, p.x, p.y, p.z, c);
-  walk_cells(k, fstart, c, [&](int j) {
-    V4<T> q = fpos[j];
-    T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
-    if (r2 > T(0) && r2 <= k.r2max) pair_f(load_f(j));
-  });
-  walk_cells(k, bstart, c, [&](int j) {
-    V4<T> q = bpos[j];
-    T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
-    if (r2 > T(0) && r2 <= k.r2max) pair_b(load_b(j));
-  });
 }
 
 template <class T>
@@ -475,6 +409,53 @@ __device__ __forceinline__ void walk_quad_cells(const KP<T>& k, const int* cc, W
       }
       wave_lds_fence();
       cnt = 0;
+    }
+  }
+}
+
+// Every candidate of the cells around cc[], a quad per particle, without a
+// list: the quad's lanes look the row runs up side by side and take every
+// fourth candidate of a run, U gathers in flight per lane; f(j, record, valid).
+// Sums are per lane.
+template <int U, class T, class Load, class F>
+__device__ __forceinline__ void walk_quad_all(const KP<T>& k, const int* __restrict__ cstart,
+                                              const int* cc, Load&& load, F&& f) {
+  const int c = threadIdx.x & (kQuad - 1);
+  const int R = k.R, side = 2 * R + 1, rows = k.dim == 3 ? side * side : side;
+  constexpr int kQ = (kWalkRows + kQuad - 1) / kQuad;
+  for (int row0 = 0; row0 < rows; row0 += kWalkRows) {
+    int lo_[kQ], hi_[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int r = c + kQuad * q, row = row0 + r;
+      lo_[q] = hi_[q] = 0;
+      if (r < kWalkRows && row < rows) {
+        const int dy = row % side - R, dz = k.dim == 3 ? row / side - R : 0;
+        const int c0 = dim_encode(k, wadd(cc[0], -R), wadd(cc[1], dy), wadd(cc[2], dz));
+        const long lo = c0 < 1 ? 1 : (long)c0;
+        long hi = (long)c0 + 2 * R;
+        if (hi > k.node_num - 1) hi = k.node_num - 1;
+        if (lo <= hi) {
+          lo_[q] = cstart[lo];
+          hi_[q] = cstart[hi + 1];
+        }
+      }
+    }
+    auto run = [&](int j0, int j1) {
+      for (int j = j0; j < j1; j += kQuad * U) {
+        decltype(load(0)) rec[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) rec[u] = load(min(j + c + kQuad * u, j1 - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u) f(j + c + kQuad * u, rec[u], j + c + kQuad * u < j1);
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      run(quad_lane<0>(lo_[q]), quad_lane<0>(hi_[q]));
+      if (4 * q + 1 < kWalkRows) run(quad_lane<1>(lo_[q]), quad_lane<1>(hi_[q]));
+      if (4 * q + 2 < kWalkRows) run(quad_lane<2>(lo_[q]), quad_lane<2>(hi_[q]));
+      if (4 * q + 3 < kWalkRows) run(quad_lane<3>(lo_[q]), quad_lane<3>(hi_[q]));
     }
   }
 }
