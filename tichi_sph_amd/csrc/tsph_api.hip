@@ -19,7 +19,8 @@ void set_error(const char* fmt, ...) {
 }
 
 template <class T>
-int sort_object(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
+int sort_object(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, SolveOpen,
+                hipStream_t);
 template <class T>
 int sort_object_static(const TsphParams&, TsphObject*, TsphControl*, int, hipStream_t);
 size_t static_sort_scratch_bytes();
@@ -29,7 +30,7 @@ template <class T>
 int ngrid_build(const TsphParams&, TsphObject* const*, int, int*, int*, int*, int*, int*, void*,
                 size_t, hipStream_t);
 template <class T>
-int density_alpha(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t,
+int density_alpha(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, bool,
                   hipStream_t);
 template <class T>
 int solver_begin(const TsphParams&, TsphControl*, int, int*, int, hipStream_t);
@@ -113,7 +114,8 @@ int adj_density_alpha(const TsphParams&, TsphObject*, TsphObject*, TsphAdjoint*,
 template <class T>
 int adj_bound_sums(const TsphParams&, TsphObject*, TsphObject*, TsphAdjoint*, hipStream_t);
 template <class T>
-int advect(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
+int advect(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen,
+           hipStream_t);
 template <class T>
 int fbm_round(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int,
               hipStream_t);
@@ -284,11 +286,16 @@ size_t tsph_workspace_bytes(const TsphParams* p, int32_t capacity) {
   return ws_bytes_needed(capacity, p->node_num);
 }
 
-int tsph_sort_object(const TsphParams* p, TsphObject* obj, TsphControl* ctrl, int32_t cfl,
-                     void* ws, size_t wsb, void* stream) {
+static int sort_object_open(const TsphParams* p, TsphObject* obj, TsphControl* ctrl, int32_t cfl,
+                            void* ws, size_t wsb, void* stream, SolveOpen open) {
   if (int rc = check_params(p)) return rc;
   if (int rc = check_obj(obj, "tsph_sort_object")) return rc;
-  return DISPATCH(p, sort_object, *p, obj, ctrl, cfl, ws, wsb, (hipStream_t)stream);
+  return DISPATCH(p, sort_object, *p, obj, ctrl, cfl, ws, wsb, open, (hipStream_t)stream);
+}
+
+int tsph_sort_object(const TsphParams* p, TsphObject* obj, TsphControl* ctrl, int32_t cfl,
+                     void* ws, size_t wsb, void* stream) {
+  return sort_object_open(p, obj, ctrl, cfl, ws, wsb, stream, SolveOpen{});
 }
 
 int tsph_sort_object_static(const TsphParams* p, TsphObject* obj, TsphControl* ctrl, int32_t cfl,
@@ -322,14 +329,19 @@ int tsph_neighbor_lists(const TsphParams* p, const TsphObject* obj, int32_t n_ui
                   shift, count, (hipStream_t)stream);
 }
 
-int tsph_density_alpha(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
-                       void* ws, size_t wsb, void* stream) {
+static int density_alpha_open(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
+                              void* ws, size_t wsb, void* stream, bool opened) {
   if (int rc = check_params(p)) return rc;
   if (int rc = check_obj(f, "tsph_density_alpha")) return rc;
   if (int rc = check_obj(b, "tsph_density_alpha")) return rc;
   TSPH_REQUIRE(p->list_cap_f >= 1 && p->list_cap_b >= 1, TSPH_EINVAL,
                "tsph_density_alpha: list capacities must be positive");
-  return DISPATCH(p, density_alpha, *p, f, b, ctrl, ws, wsb, (hipStream_t)stream);
+  return DISPATCH(p, density_alpha, *p, f, b, ctrl, ws, wsb, opened, (hipStream_t)stream);
+}
+
+int tsph_density_alpha(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
+                       void* ws, size_t wsb, void* stream) {
+  return density_alpha_open(p, f, b, ctrl, ws, wsb, stream, false);
 }
 
 int tsph_solver_begin(const TsphParams* p, TsphControl* ctrl, int32_t solve, void* stream) {
@@ -392,11 +404,16 @@ int tsph_relist(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* 
   return DISPATCH(p, relist, *p, f, b, ctrl, ws, wsb, (hipStream_t)stream);
 }
 
-int tsph_advect(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl, void* ws,
-                size_t wsb, void* stream) {
+static int advect_open(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
+                       void* ws, size_t wsb, void* stream, SolveOpen open) {
   if (int rc = check_params(p)) return rc;
   if (int rc = check_obj(f, "tsph_advect")) return rc;
-  return DISPATCH(p, advect, *p, f, b, ctrl, ws, wsb, (hipStream_t)stream);
+  return DISPATCH(p, advect, *p, f, b, ctrl, ws, wsb, open, (hipStream_t)stream);
+}
+
+int tsph_advect(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl, void* ws,
+                size_t wsb, void* stream) {
+  return advect_open(p, f, b, ctrl, ws, wsb, stream, SolveOpen{});
 }
 
 int tsph_fbm_round(const TsphParams* p, TsphObject* f, TsphControl* ctrl, void* ws, size_t wsb,
@@ -484,13 +501,13 @@ int tsph_wcsph(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* c
   return DISPATCH(p, wcsph, *p, f, b, ctrl, (hipStream_t)stream);
 }
 
-// One solve to its stop rule: `pred` iterations enqueued, then single ones
-// while the device says to go on.
+static int32_t next_token(TsphStep* s) { return s->token = s->token % 0x7fffffff + 1; }
+
+// One solve, opened with s->token, to its stop rule: `pred` iterations
+// enqueued, then single ones while the device says to go on.
 static int step_solve(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl,
                       TsphStep* s, int solve, void* ws, size_t wsb, void* stream) {
   const hipStream_t st = (hipStream_t)stream;
-  s->token = s->token % 0x7fffffff + 1;
-  if (int rc = tsph_solver_begin_signal(p, ctrl, solve, s->signal, s->token, stream)) return rc;
   const int kmax = p->iter_max + 1;
   int k = 0, it = 0, chunk = s->pred[solve] > 1 ? s->pred[solve] : 1;
   while (k < kmax) {
@@ -521,17 +538,23 @@ static int step_solve(const TsphParams* p, TsphObject* f, TsphObject* b, TsphCon
 int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl, TsphStep* s,
               void* ws, size_t wsb, void* stream) {
   TSPH_REQUIRE(s && s->signal_host && s->signal, TSPH_EINVAL, "tsph_step: null step or signal");
-  if (int rc = tsph_sort_object(p, f, ctrl, s->cfl, ws, wsb, stream)) return rc;
-  if (int rc = tsph_density_alpha(p, f, b, ctrl, ws, wsb, stream)) return rc;
+  // the step's reset and the solves' openings ride in the sort's first kernel
+  // and the advection's last: three launches less than the calls one by one
+  const SolveOpen open0{s->signal, next_token(s), 1};
+  if (int rc = sort_object_open(p, f, ctrl, s->cfl, ws, wsb, stream, open0)) return rc;
+  if (int rc = density_alpha_open(p, f, b, ctrl, ws, wsb, stream, true)) return rc;
   if (int rc = step_solve(p, f, b, ctrl, s, 0, ws, wsb, stream)) return rc;
-  if (int rc = tsph_advect(p, f, b, ctrl, ws, wsb, stream)) return rc;
+  const SolveOpen open1{s->signal, next_token(s), 1};
+  if (int rc = advect_open(p, f, b, ctrl, ws, wsb, stream, open1)) return rc;
+  if (f->n == 0)  // no advection was launched
+    if (int rc = tsph_solver_begin_signal(p, ctrl, 1, s->signal, s->token, stream)) return rc;
   if (int rc = step_solve(p, f, b, ctrl, s, 1, ws, wsb, stream)) return rc;
   if (s->wcsph)
     if (int rc = tsph_wcsph(p, f, b, ctrl, stream)) return rc;
   s->fbm_rounds = 0;
   while (s->fbm && f->n > 0 && s->fbm_rounds < 1000) {
     const hipStream_t st = (hipStream_t)stream;
-    s->token = s->token % 0x7fffffff + 1;
+    next_token(s);
     if (int rc = DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, s->signal, (int)s->token, st))
       return rc;
     ++s->fbm_rounds;

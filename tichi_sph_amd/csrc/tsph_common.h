@@ -387,18 +387,22 @@ __device__ __forceinline__ double min_partials(const double* part, int n, double
 // another inside a launch.
 enum FinalizeMode { kFinCfl = 0, kFinEnergy = 1, kFinFlag = 2, kFinCompression = 3 };
 
+// dt from the smallest CFL candidate (sph.py:41-47)
+template <class T>
+__device__ __forceinline__ void cfl_finish(const KP<T>& k, double all, TsphControl* ctrl) {
+  TSPH_STRICT
+  T d = k.gps / (T)k.cs;  // sph.py:43
+  if (all < (double)d) d = (T)all;
+  ctrl->dt = (double)d;
+}
+
 template <class T>
 __device__ __forceinline__ void k_finalize_body(Blk blk, KP<T> k, int mode, const double* __restrict__ partial, int nblk, int n,
                TsphControl* ctrl) {
   __shared__ double lds[kWaves];
   if (mode == kFinCfl) {
     double all = min_partials(partial, nblk, lds, 1e300);
-    if (threadIdx.x == 0) {
-      TSPH_STRICT
-      T d = k.gps / (T)k.cs;  // sph.py:43
-      if (all < (double)d) d = (T)all;
-      ctrl->dt = (double)d;
-    }
+    if (threadIdx.x == 0) cfl_finish(k, all, ctrl);
   } else if (mode == kFinEnergy) {
     double a = sum_partials(partial, nblk, lds);
     double b = sum_partials(partial + nblk, nblk, lds);
@@ -424,5 +428,49 @@ __global__ void __launch_bounds__(kBlock)
                TsphControl* ctrl) {
   k_finalize_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, mode, partial, nblk, n, ctrl);
 }
+
+// Per-step reset of the control block's step-scoped state: general_flag = 1
+// (SPH_clean_value, sph.py:24), FBM round count, list-overflow counters.
+__device__ __forceinline__ void step_reset_body(TsphControl* ctrl) {
+  if (threadIdx.x == 0) {
+    ctrl->general_flag = 1;
+    ctrl->fbm_rounds = 0;
+    ctrl->overflow_f = 0;
+    ctrl->overflow_b = 0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Solver stop state (main.py:201-213 / 222-234).
+// ---------------------------------------------------------------------------
+template <class T>
+__device__ __forceinline__ void solver_begin_body(const KP<T>& k, TsphControl* ctrl, int solve,
+                                                  int* signal = nullptr, int token = 0) {
+  int t = threadIdx.x;
+  T thr = solve == 0 ? k.div_thr : k.comp_thr;
+  T comp = (T)ctrl->compression;
+  bool enter = (0 < k.iter_min) || (comp > thr);
+  // run_u[q] = 1 iff iteration q of this solve runs; decided one iteration ahead
+  for (int q = t; q < TSPH_MAX_ITER_LOG; q += blockDim.x) ctrl->run_u[q] = (q == 0 && enter) ? 1 : 0;
+  if (t == 0) {
+    ctrl->it = 0;
+    ctrl->solve = solve;
+    ctrl->stop = enter ? 0 : 1;
+    if (solve == 0) ctrl->div_iter = 0;
+    else ctrl->incom_iter = 0;
+    ctrl->signal = (uint64_t)(uintptr_t)signal;
+    ctrl->token = token;
+    if (signal && !enter) {  // a solve that runs no iteration stops here: (it 0, stop)
+      const uint64_t w = ((uint64_t)(uint32_t)token << 32) | 1u;
+      __hip_atomic_store((uint64_t*)signal, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+// Opening a solve inside another kernel's block 0 (tsph_step: one launch less
+// than k_solver_begin); on = 0 leaves the solve alone.
+struct SolveOpen {
+  uint64_t* signal;
+  int token, on;
+};
 
 }  // namespace tsph

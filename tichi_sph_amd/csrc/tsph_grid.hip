@@ -106,9 +106,79 @@ __global__ void __launch_bounds__(kBlock)
   if (blk.b == 0) k_finalize_body<T>(blk, k, (int)kFinCfl, partial, nblk, n, ctrl);
 }
 
+// The scan of a small table in one launch: every block adds up the counts
+// before its tile itself, all of its loads in flight, instead of waiting for a
+// launch that reduces the tiles.  For up to kScanOneTiles tiles (65,536 cells)
+// that is 60 loads per thread at most.  With cfl (nblk > 0), block 0 finishes
+// cfl_condition as k_scan_reduce_cfl does.
+constexpr int kScanOneTiles = 32;
+constexpr int kScanOneThreads = 1024;
+template <class T>
+__global__ void __launch_bounds__(kScanOneThreads)
+    k_scan_one(const int* __restrict__ cnt, int len, int* __restrict__ start, KP<T> k,
+               const double* __restrict__ partial, int nblk, TsphControl* ctrl) {
+  __shared__ double low[kScanOneThreads / 64];
+  __shared__ int before[kScanOneThreads / 64], inside[kScanOneThreads / 64];
+  constexpr int per = kScanTile / kScanOneThreads;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, base = blockIdx.x * kScanTile;
+  int sum = 0;
+  for (int e = t; e < base; e += 16 * kScanOneThreads) {
+    int v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      v[u] = e + u * kScanOneThreads < base ? cnt[e + u * kScanOneThreads] : 0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) sum += v[u];
+  }
+  int v[per], loc = 0;
+#pragma unroll
+  for (int e = 0; e < per; ++e) {
+    const int i = base + t * per + e;
+    v[e] = i < len ? cnt[i] : 0;
+    loc += v[e];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  int x = loc;  // inclusive scan of the threads' totals
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) inside[w] = x;
+  if (lane == 0) before[w] = sum;
+  __syncthreads();
+  int run = x - loc;
+  for (int q = 0; q < kScanOneThreads / 64; ++q) run += before[q] + (q < w ? inside[q] : 0);
+#pragma unroll
+  for (int e = 0; e < per; ++e) {
+    const int i = base + t * per + e;
+    if (i < len) start[i] = run;
+    run += v[e];
+    if (i == len - 1) start[len] = run;
+  }
+  if (nblk > 0 && blockIdx.x == 0) {  // uniform per block
+    double m = 1e300;
+    for (int e = t; e < nblk; e += kScanOneThreads) m = fmin(m, partial[e]);
+    m = wave_min(m);
+    if (lane == 0) low[w] = m;
+    __syncthreads();
+    if (t == 0) {
+      for (int q = 1; q < kScanOneThreads / 64; ++q) m = fmin(m, low[q]);
+      cfl_finish(k, m, ctrl);
+    }
+  }
+}
+
 static int launch_scan(const int* cnt, long len, int* sums, int* start, hipStream_t st) {
   long nb = scan_blocks(len);
   if (nb < 1) nb = 1;
+  if (nb <= kScanOneTiles) {
+    hipLaunchKernelGGL(k_scan_one<float>, dim3(nb), dim3(kScanOneThreads), 0, st, cnt, (int)len,
+                       start, KP<float>{}, (const double*)nullptr, 0, (TsphControl*)nullptr);
+    TSPH_LAUNCH_CHECK("scan");
+    return 0;
+  }
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kBlock), 0, st, cnt, len, sums);
   hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kBlock), 0, st, cnt, len, sums, start);
   TSPH_LAUNCH_CHECK("scan");
@@ -117,6 +187,19 @@ static int launch_scan(const int* cnt, long len, int* sums, int* start, hipStrea
 
 __global__ void __launch_bounds__(kBlock) k_fill_i32(int* __restrict__ p, long n, int v) {
   long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) p[i] = v;
+}
+
+// k_fill_i32 with, in its block 0, the step's reset and the opening of its
+// divergence solve (tsph_step): two launches less.
+template <class T>
+__global__ void __launch_bounds__(kBlock)
+    k_fill_open(int* __restrict__ p, long n, int v, KP<T> k, TsphControl* ctrl, SolveOpen open) {
+  if (blockIdx.x == 0) {
+    step_reset_body(ctrl);
+    solver_begin_body(k, ctrl, 0, (int*)open.signal, open.token);
+  }
+  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) p[i] = v;
 }
 
@@ -264,13 +347,17 @@ struct SortScratch {
 
 template <class T>
 static int sort_object_core(const TsphParams& prm, TsphObject* o, TsphControl* ctrl, int cfl,
-                            const SortScratch& L, hipStream_t st) {
+                            const SortScratch& L, SolveOpen open, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   int n = o->n;
   o->flags &= ~TSPH_OBJ_STATIC_SUMS;  // new storage order: the kept sums no longer apply
   long len = (long)prm.node_num + 1;  // cells + trailing invalid bucket
-  hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(len + 1)), dim3(kBlock), 0, st, o->cell_count,
-                     len + 1, 0);
+  if (open.on)
+    hipLaunchKernelGGL(k_fill_open<T>, dim3(blocks_for(len + 1)), dim3(kBlock), 0, st,
+                       o->cell_count, len + 1, 0, k, ctrl, open);
+  else
+    hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(len + 1)), dim3(kBlock), 0, st, o->cell_count,
+                       len + 1, 0);
   int nb = blocks_for(n);
   const int nbl = nb > 0 ? nb : 1;  // k_keys' blocks (one also for n = 0 with CFL)
   if (n > 0 || cfl)
@@ -281,10 +368,15 @@ static int sort_object_core(const TsphParams& prm, TsphObject* o, TsphControl* c
   if (cfl) {  // the scan, with the CFL partials reduced in its first kernel
     long nbs = scan_blocks(len);
     if (nbs < 1) nbs = 1;
-    hipLaunchKernelGGL(k_scan_reduce_cfl<T>, dim3(nbs), dim3(kBlock), 0, st, o->cell_count, len,
-                       L.scan_sums, k, L.partial, nbl, n, ctrl);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nbs), dim3(kBlock), 0, st, o->cell_count, len,
-                       L.scan_sums, o->cell_start);
+    if (nbs <= kScanOneTiles) {
+      hipLaunchKernelGGL(k_scan_one<T>, dim3(nbs), dim3(kScanOneThreads), 0, st, o->cell_count,
+                         (int)len, o->cell_start, k, L.partial, nbl, ctrl);
+    } else {
+      hipLaunchKernelGGL(k_scan_reduce_cfl<T>, dim3(nbs), dim3(kBlock), 0, st, o->cell_count, len,
+                         L.scan_sums, k, L.partial, nbl, n, ctrl);
+      hipLaunchKernelGGL(k_scan_apply, dim3(nbs), dim3(kBlock), 0, st, o->cell_count, len,
+                         L.scan_sums, o->cell_start);
+    }
     TSPH_LAUNCH_CHECK("scan");
   } else if (int rc = launch_scan(o->cell_count, len, L.scan_sums, o->cell_start, st)) {
     return rc;
@@ -305,12 +397,12 @@ static int sort_object_core(const TsphParams& prm, TsphObject* o, TsphControl* c
 
 template <class T>
 int sort_object(const TsphParams& prm, TsphObject* o, TsphControl* ctrl, int cfl, void* ws,
-                size_t wsb, hipStream_t st) {
+                size_t wsb, SolveOpen open, hipStream_t st) {
   WsLayout W;
   TSPH_REQUIRE(carve_ws(ws, wsb, o->capacity, prm.node_num, &W), TSPH_ECAPACITY,
                "tsph_sort_object: workspace too small (%zu bytes)", wsb);
   const SortScratch L{W.partial, W.scan_sums, W.key, W.rank, W.tmp_idx, W.tmp_pid, W.tmp_key};
-  return sort_object_core<T>(prm, o, ctrl, cfl, L, st);
+  return sort_object_core<T>(prm, o, ctrl, cfl, L, open, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -380,7 +472,7 @@ int sort_object_static(const TsphParams& prm, TsphObject* o, TsphControl* ctrl, 
   p += kStaticScanBytes;
   int** idx[5] = {&L.key, &L.rank, &L.tmp_idx, &L.tmp_pid, &L.tmp_key};
   for (int q = 0; q < 5; ++q, p += kStaticIdxBytes) *idx[q] = (int*)p;
-  return sort_object_core<T>(prm, o, ctrl, cfl, L, st);
+  return sort_object_core<T>(prm, o, ctrl, cfl, L, SolveOpen{}, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -620,8 +712,8 @@ int batch_sort(const TsphBatchInfo& bi, char* tab, TsphObject* hostf, int cfl, i
 template int batch_sort<float>(const TsphBatchInfo&, char*, TsphObject*, int, int, hipStream_t);
 template int batch_sort<double>(const TsphBatchInfo&, char*, TsphObject*, int, int, hipStream_t);
 
-template int sort_object<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
-template int sort_object<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
+template int sort_object<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, SolveOpen, hipStream_t);
+template int sort_object<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, SolveOpen, hipStream_t);
 template int sort_object_static<float>(const TsphParams&, TsphObject*, TsphControl*, int, hipStream_t);
 template int sort_object_static<double>(const TsphParams&, TsphObject*, TsphControl*, int, hipStream_t);
 template int ngrid_build<float>(const TsphParams&, TsphObject* const*, int, int*, int*, int*, int*, int*, void*, size_t, hipStream_t);

@@ -478,16 +478,6 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// Per-step reset of the control block's step-scoped state: general_flag = 1
-// (SPH_clean_value, sph.py:24), FBM round count, list-overflow counters.
-__device__ __forceinline__ void step_reset_body(TsphControl* ctrl) {
-  if (threadIdx.x == 0) {
-    ctrl->general_flag = 1;
-    ctrl->fbm_rounds = 0;
-    ctrl->overflow_f = 0;
-    ctrl->overflow_b = 0;
-  }
-}
 __global__ void k_step_reset(TsphControl* ctrl) { step_reset_body(ctrl); }
 
 // Pass A of both objects in one launch: blocks [0, nbf) run the fluid body,
@@ -587,32 +577,6 @@ int verify_fast_quotient(const TsphParams& prm, int* out, hipStream_t st) {
   return 0;
 }
 
-// ---------------------------------------------------------------------------
-// Solver stop state (main.py:201-213 / 222-234).
-// ---------------------------------------------------------------------------
-template <class T>
-__device__ __forceinline__ void solver_begin_body(const KP<T>& k, TsphControl* ctrl, int solve,
-                                                  int* signal = nullptr, int token = 0) {
-  int t = threadIdx.x;
-  T thr = solve == 0 ? k.div_thr : k.comp_thr;
-  T comp = (T)ctrl->compression;
-  bool enter = (0 < k.iter_min) || (comp > thr);
-  // run_u[q] = 1 iff iteration q of this solve runs; decided one iteration ahead
-  for (int q = t; q < TSPH_MAX_ITER_LOG; q += blockDim.x) ctrl->run_u[q] = (q == 0 && enter) ? 1 : 0;
-  if (t == 0) {
-    ctrl->it = 0;
-    ctrl->solve = solve;
-    ctrl->stop = enter ? 0 : 1;
-    if (solve == 0) ctrl->div_iter = 0;
-    else ctrl->incom_iter = 0;
-    ctrl->signal = (uint64_t)(uintptr_t)signal;
-    ctrl->token = token;
-    if (signal && !enter) {  // a solve that runs no iteration stops here: (it 0, stop)
-      const uint64_t w = ((uint64_t)(uint32_t)token << 32) | 1u;
-      __hip_atomic_store((uint64_t*)signal, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
-}
 template <class T>
 __global__ void k_solver_begin(KP<T> k, TsphControl* ctrl, int solve, int* signal, int token) {
   solver_begin_body(k, ctrl, solve, signal, token);
@@ -923,12 +887,20 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
                       const TsphControl* ctrl) {
   const int cl = coop_lane<kQuad>();
   const T dt = (T)ctrl->dt;
+  if (k.gamma == T(0)) {  // a scene without it in a grouped launch: the update alone
+    TSPH_STRICT
+    const int i = coop_sub<R>(blk) * (kBlock / kQuad) + (int)threadIdx.x;
+    if ((int)threadIdx.x >= R * (kBlock / kQuad) || i >= n) return;
+    const V4<T> v = vel[i], a = acce_adv[i];
+    vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
+    return;
+  }
 #pragma unroll 1
   for (int r = 0; r < R; ++r) {
     const int i = coop_particle<kQuad>(coop_sub<R>(blk, r));
     if (i >= n) break;
     V4<T> a = acce_adv[i];
-    if (k.gamma != T(0) && vf[(long)i * k.P] > T(0.99)) {
+    if (vf[(long)i * k.P] > T(0.99)) {
       V4<T> p = fpos[i];
       V4<T> ni = normal[i];
       T rp = rest_psi_of(k, rdens, i);
@@ -988,9 +960,11 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
 // rather than at that of the surface-tension walk.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_vel_adv_update(int n, const V4<T>* __restrict__ vel, const V4<T>* __restrict__ acce_adv,
-                     V4<T>* __restrict__ vadv, const TsphControl* ctrl) {
+    k_vel_adv_update(KP<T> k, int n, const V4<T>* __restrict__ vel,
+                     const V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
+                     TsphControl* ctrl, SolveOpen open) {
   TSPH_STRICT
+  if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
   const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (i >= n) return;
   const T dt = (T)ctrl->dt;
@@ -1007,7 +981,8 @@ __global__ void __launch_bounds__(kBlock)
                       const V4<T>* __restrict__ strec, const int* __restrict__ nbr_f,
                       const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
                       V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
-                      const TsphControl* ctrl) {
+                      TsphControl* ctrl, SolveOpen open) {
+  if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
   k_surface_tension_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
 }
 
@@ -1299,9 +1274,9 @@ __global__ void __launch_bounds__(kBlock)
 // ---------------------------------------------------------------------------
 template <class T>
 static int pass_a(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctrl,
-                  bool with_bound, const WsLayout& L, hipStream_t st) {
+                  bool with_bound, const WsLayout& L, bool opened, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
-  hipLaunchKernelGGL(k_step_reset, dim3(1), dim3(64), 0, st, ctrl);
+  if (!opened) hipLaunchKernelGGL(k_step_reset, dim3(1), dim3(64), 0, st, ctrl);
   if (with_bound && f->n > 0 && f->n <= pass_a_quad_max<T>(prm.dim) &&
       b->n <= 2 * pass_a_quad_max<T>(prm.dim)) {
     const int nbf = coop_blocks<kQuad>(f->n);
@@ -1342,11 +1317,11 @@ static int pass_a(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphContr
 
 template <class T>
 int density_alpha(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctrl,
-                  void* ws, size_t wsb, hipStream_t st) {
+                  void* ws, size_t wsb, bool opened, hipStream_t st) {
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
                "tsph_density_alpha: workspace too small");
-  return pass_a<T>(prm, f, b, ctrl, true, L, st);
+  return pass_a<T>(prm, f, b, ctrl, true, L, opened, st);
 }
 
 // The fluid's neighbour lists alone, as pass A builds them (8 candidates in
@@ -1450,7 +1425,7 @@ int solver_half(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl
 
 template <class T>
 int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctrl, void* ws,
-           size_t wsb, hipStream_t st) {
+           size_t wsb, SolveOpen open, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
@@ -1464,14 +1439,15 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
                      (V4<T>*)f->vel_adv, (V4<T>*)f->vel, (V4<T>*)f->acce_adv,
                      (V4<T>*)f->normal, (const T*)f->mass, psi, (V4<T>*)L.krec);
   if (k.gamma == T(0))
-    hipLaunchKernelGGL(k_vel_adv_update<T>, dim3(nb), dim3(kBlock), 0, st, f->n,
-                       (const V4<T>*)f->vel, (const V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl);
+    hipLaunchKernelGGL(k_vel_adv_update<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
+                       (const V4<T>*)f->vel, (const V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl,
+                       open);
   else
     hipLaunchKernelGGL(k_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
                        f->capacity, (const V4<T>*)f->pos, psi, (const T*)f->rest_density,
                        (const T*)f->volume_frac, f->cell_start, (const V4<T>*)f->normal,
                        (const V4<T>*)L.krec, f->nbr_f, f->nbr_nf, (const V4<T>*)f->vel,
-                       (V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl);
+                       (V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl, open);
   TSPH_LAUNCH_CHECK("advect");
   return 0;
 }
@@ -1928,14 +1904,14 @@ TSPH_BATCH_INST(double)
 
 template int relist<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
 template int relist<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
-template int density_alpha<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
-template int density_alpha<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
+template int density_alpha<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, bool, hipStream_t);
+template int density_alpha<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, bool, hipStream_t);
 template int solver_begin<float>(const TsphParams&, TsphControl*, int, int*, int, hipStream_t);
 template int solver_begin<double>(const TsphParams&, TsphControl*, int, int*, int, hipStream_t);
 template int solver_half<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, hipStream_t);
 template int solver_half<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, hipStream_t);
-template int advect<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
-template int advect<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, hipStream_t);
+template int advect<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
+template int advect<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
 template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
 template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
 template int tail<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
