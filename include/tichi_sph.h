@@ -484,6 +484,16 @@ int tsph_adj_density_alpha(const TsphParams* p, TsphObject* fluid, TsphObject* b
 int tsph_adj_end(const TsphParams* p, TsphObject* fluid, TsphAdjoint* adj, const int32_t* pid,
                  void* xbar_ref, void* vbar_ref, void* stream);
 
+/* Up to TSPH_COPY_MAX device-to-device copies in one launch (what a taped step
+ * records, a checkpoint and its restore).  Regions must not overlap. */
+#define TSPH_COPY_MAX 16
+typedef struct TsphCopy {
+  void* dst;
+  const void* src;
+  uint64_t bytes;
+} TsphCopy;
+int tsph_copy_many(const TsphCopy* copies, int32_t count, void* stream);
+
 /* ----------------------------------------------------------------------
  * Batched scenes (no reference counterpart: the reference runs one scene
  * per process).  Many independent scenes of uneven particle counts are

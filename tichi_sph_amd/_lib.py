@@ -95,6 +95,13 @@ class TsphStep(ctypes.Structure):
                 ("fbm_rounds", _i32), ("pad", _i32)]
 
 
+COPY_MAX = 16
+
+
+class TsphCopy(ctypes.Structure):
+    _fields_ = [("dst", _vp), ("src", _vp), ("bytes", ctypes.c_uint64)]
+
+
 KERNEL_IDS = {
     "SPH_clean_value": 0, "cfl_condition": 1, "SPH_prepare_attr": 2,
     "SPH_prepare_alpha_1": 3, "SPH_prepare_alpha_2": 4, "SPH_prepare_alpha": 5,
@@ -115,7 +122,7 @@ EXPORTED = [
     "tsph_solver_iteration", "tsph_solver_psi", "tsph_solver_update", "tsph_advect",
     "tsph_fbm_round", "tsph_tail",
     "tsph_ref_kernel", "tsph_solver_psi_taped", "tsph_solver_psi_frozen", "tsph_relist", "tsph_adj_bound_sums", "tsph_adj_begin",
-    "tsph_adj_solver_iteration", "tsph_adj_advect", "tsph_adj_density_alpha", "tsph_adj_end",
+    "tsph_adj_solver_iteration", "tsph_adj_advect", "tsph_adj_density_alpha", "tsph_adj_end", "tsph_copy_many",
     "tsph_batch_table_bytes", "tsph_batch_prepare", "tsph_batch_sort", "tsph_batch_density_alpha",
     "tsph_batch_solver_begin", "tsph_batch_solver_begin_signal", "tsph_batch_solver_psi",
     "tsph_batch_solver_update",
@@ -198,6 +205,7 @@ def load(path=None):
         "tsph_batch_stop_state": [BI, _vp, _vp, _vp],
         "tsph_map_velocity": [P, O, _vp, _f64, _vp, _vp],
         "tsph_wcsph": [P, O, O, C, _vp],
+        "tsph_copy_many": [ctypes.POINTER(TsphCopy), _i32, _vp],
         "tsph_step": [P, O, O, C, ctypes.POINTER(TsphStep), _vp, sz, _vp],
     }
     for name, args in sigs.items():

@@ -129,21 +129,46 @@ class DiffRunner:
             self.sim.params.surface_tension_gamma = float(gamma)
 
     # --------------------------------------------------------------- state
+    def _copy(self, pairs):
+        """dst.copy_(src) for every pair (at most _lib.COPY_MAX): in one
+        launch those that only move bytes."""
+        moves = (_lib.TsphCopy * len(pairs))()
+        m = 0
+        for dst, src in pairs:
+            if (dst.dtype == src.dtype and dst.is_cuda and dst.device == src.device and dst.shape == src.shape
+                    and dst.is_contiguous() and src.is_contiguous()):
+                moves[m] = (dst.data_ptr(), src.data_ptr(), dst.numel() * dst.element_size())
+                m += 1
+            else:
+                dst.copy_(src)
+        self._move(moves, m)
+
+    def _clones(self, tensors):
+        """Tensors like these contiguous ones, and the moves that fill them."""
+        out = [torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in tensors]
+        moves = (_lib.TsphCopy * len(out))(*[(d.data_ptr(), t.data_ptr(), d.numel() * d.element_size())
+                                             for d, t in zip(out, tensors)])
+        return out, moves
+
+    def _move(self, moves, count=None):
+        rc = self.lib.tsph_copy_many(moves, len(moves) if count is None else count, self.sim.stream_ptr())
+        _lib.check(rc, "tsph_copy_many")
+
+    _STATE = ("pos", "vel", "mass", "rest_density", "rest_volume", "volume_frac", "pid")
+
     def checkpoint(self):
         f = self.sim.fluid
         n = f.part_num
-        st = {name: f.t[name][:n].clone() for name in
-              ("pos", "vel", "mass", "rest_density", "rest_volume", "volume_frac", "pid")}
-        st["ctrl"] = self.sim.ctrl.clone()
+        out, moves = self._clones([f.t[name][:n] for name in self._STATE] + [self.sim.ctrl])
+        self._move(moves)
+        st = dict(zip(self._STATE + ("ctrl",), out))
         st["step_index"] = self.step_index
         return st
 
     def restore(self, st):
         f = self.sim.fluid
         n = f.part_num
-        for name in ("pos", "vel", "mass", "rest_density", "rest_volume", "volume_frac", "pid"):
-            f.t[name][:n].copy_(st[name])
-        self.sim.ctrl.copy_(st["ctrl"])
+        self._copy([(f.t[name][:n], st[name]) for name in self._STATE] + [(self.sim.ctrl, st["ctrl"])])
         self.step_index = st["step_index"]
 
     def set_velocity_ref(self, v):
@@ -198,26 +223,23 @@ class DiffRunner:
             tp = StepTape()
             if self.tape_lists:
                 tp.nbr_f, tp.nbr_nf, tp.nbr_nb = lists
-            tp.pos = f.t["pos"][:n].clone()
-            tp.mass = f.t["mass"][:n].clone()
-            tp.rest_density = f.t["rest_density"][:n].clone()
-            tp.pid = f.t["pid"][:n].clone()
-            tp.cell_start = f.t["cell_start"].clone()
         fs, bs = ctypes.byref(f.struct()), ctypes.byref(b.struct())
         sim._call("density_alpha", sim.lib.tsph_density_alpha, P, fs, bs, sim.ctrl_ptr(), ws, wsb, stp)
         if tape:
-            tp.density = f.t["sph_density"][:n].clone()
-            tp.alpha = f.t["alpha"][:n].clone()
-            tp.vol = f.t["vol"][:n].clone()
-            tp.alpha_1 = f.t["alpha_1"][:n].clone()
+            # prepared here, where pass A keeps the device busy; moved after the
+            # advection (nothing writes these between the sort or pass A and
+            # there, and only the tail after it)
+            names = ("pos", "mass", "rest_density", "pid", "sph_density", "alpha", "vol", "alpha_1", "vel", "normal")
+            out, moves = self._clones([f.t[name][:n] for name in names] + [f.t["cell_start"]])
+            (tp.pos, tp.mass, tp.rest_density, tp.pid, tp.density, tp.alpha, tp.vol, tp.alpha_1, tp.vel, tp.normal,
+             tp.cell_start) = out
         fz = [None, None] if frozen is None else [[kap for _, kap in frozen.iters[q]] for q in (0, 1)]
         if frozen is not None and force[0] is None:
             force = (len(fz[0]), len(fz[1]))
         d_it = sim._solve(0, tape=tp.iters[0] if tape else None, force=force[0], frozen=fz[0])
         sim._call("advect", sim.lib.tsph_advect, P, fs, bs, sim.ctrl_ptr(), ws, wsb, stp)
         if tape:
-            tp.vel = f.t["vel"][:n].clone()
-            tp.normal = f.t["normal"][:n].clone()
+            self._move(moves)
         i_it = sim._solve(1, tape=tp.iters[1] if tape else None, force=force[1], frozen=fz[1])
         sim._call("tail", sim.lib.tsph_tail, P, fs, sim.ctrl_ptr(), 0, ws, wsb, stp)
         if tape:
@@ -307,8 +329,11 @@ class DiffRunner:
 class _Rollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, v0, mu, gamma, runner, steps, every, budget):
-        runner.set_params(mu.item(), gamma.item())
-        runner.surface_tension_grad = bool(gamma.requires_grad) or gamma.item() != 0.0
+        # read once, before the steps: reading a device tensor waits for all
+        # work enqueued before it
+        ctx.mu, ctx.gamma = float(mu.item()), float(gamma.item())
+        runner.set_params(ctx.mu, ctx.gamma)
+        runner.surface_tension_grad = bool(gamma.requires_grad) or ctx.gamma != 0.0
         runner.set_velocity_ref(v0.detach())
         runner.step_index = 0
         runner.iter_log = []
@@ -347,7 +372,6 @@ class _Rollout(torch.autograd.Function):
                 del kept[s_old]
         ctx.runner, ctx.ckpts, ctx.steps, ctx.every = runner, ckpts, steps, every
         ctx.kept = kept
-        ctx.mu, ctx.gamma = float(mu.item()), float(gamma.item())
         ctx.v0_dtype = v0.dtype
         return runner.positions_ref(), runner.velocities_ref()
 

@@ -92,7 +92,7 @@ __device__ __forceinline__ void add_J(T& ax, T& ay, T& az, const D2<T>& d, T dx,
 //   G_l = sum_b X_b g,     H_l = sum_b X_b hq x x^T,
 // so the reverse sweeps read three records instead of walking the boundary.
 // ---------------------------------------------------------------------------
-constexpr int kBsumU = 8;  // boundary candidates in flight per lane
+constexpr int kBsumU = 4;  // boundary candidates in flight per lane
 // Lanes per particle of the reverse Jacobi and viscosity sweeps.  Their pair
 // terms (kernel second derivatives, Hessian products) make them VALU-bound
 // about as much as gather-bound, so two lanes per particle, which leave fewer
@@ -104,16 +104,21 @@ constexpr int kCoopR = 2;
 // reach 5 waves but lose more to latency than they gain.
 constexpr int kNbVis = 2;
 
+// A quad of lanes per particle, kBsumU candidates in flight per lane: bound by
+// the latency of the walks of the few particles near a wall.  One lane with 8
+// in flight 21.0 us at 200k particles and 38.0 at 1M, quads with 2 / 4 in
+// flight 15.4 / 15.8 and 40.8 / 39.2.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_adj_bound_sums(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                      const int* __restrict__ nbr_nb, const V4<T>* __restrict__ bpos,
                      const int* __restrict__ bstart, V4<T>* __restrict__ bmom,
                      int* __restrict__ bflag) {
-  const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
+  const bool first = coop_lane<kQuad>() == 0;
   if (nbr_nb[i] == 0) {  // the step found no boundary neighbour: nothing to walk
-    bflag[i] = 0;
+    if (first) bflag[i] = 0;
     return;
   }
   const V4<T> p = fpos[i];
@@ -121,10 +126,11 @@ __global__ void __launch_bounds__(kBlock)
   node_encode(k, p.x, p.y, p.z, c);
   T ax = 0, ay = 0, az = 0, G = 0, hxx = 0, hyy = 0, hzz = 0, hxy = 0, hxz = 0, hyz = 0;
   int any = 0;
-  walk_cells_batched<kBsumU>(k, bstart, c, bpos, [&](int j, const V4<T>& q) {
+  walk_quad_all<kBsumU>(k, bstart, c, [&](int j) { return bpos[j]; },
+                        [&](int, const V4<T>& q, bool valid) {
     const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const T r2 = s_r2(dx, dy, dz);
-    if (!(r2 <= k.r2max && r2 > T(0))) return;  // the boundary lists' test
+    if (!(valid && r2 <= k.r2max && r2 > T(0))) return;  // the boundary lists' test
     const D2<T> e = kern_d2(k, r2);
     const T xg = q.w * e.g, xh = q.w * e.hq;
     ax += xg * dx;
@@ -139,11 +145,16 @@ __global__ void __launch_bounds__(kBlock)
     hyz += xh * dy * dz;
     any = 1;
   });
-  bflag[i] = any;
+  any = group_sum<kQuad>(any);
+  const V4<T> A = v4(group_sum<kQuad>(ax), group_sum<kQuad>(ay), group_sum<kQuad>(az), group_sum<kQuad>(G));
+  const V4<T> H = v4(group_sum<kQuad>(hxx), group_sum<kQuad>(hyy), group_sum<kQuad>(hzz), group_sum<kQuad>(hxy));
+  const V4<T> O = v4(group_sum<kQuad>(hxz), group_sum<kQuad>(hyz), T(0), T(0));
+  if (!first) return;
+  bflag[i] = any != 0;
   if (any) {
-    bmom[i] = v4(ax, ay, az, G);
-    bmom[(long)cap + i] = v4(hxx, hyy, hzz, hxy);
-    bmom[2L * cap + i] = v4(hxz, hyz, T(0), T(0));
+    bmom[i] = A;
+    bmom[(long)cap + i] = H;
+    bmom[2L * cap + i] = O;
   }
 }
 
@@ -361,20 +372,9 @@ __global__ void __launch_bounds__(kBlock)
 // which lies in l's own cell, so only that cell's candidates are tested.
 // The cohesion terms (C = C' = 0 beyond h) are summed over the in-range list.
 // A neighbour's rest density and velocity adjoint enter only as
-// b_j = rho0_j a_j (f_jl a_j = 2 b_j / (rho_l + rho_j)), which k_adj_st_rec
+// b_j = rho0_j a_j (f_jl a_j = 2 b_j / (rho_l + rho_j)), which k_adj_vel_rec
 // writes per particle, so that a candidate costs two 16-byte gathers.
 // ---------------------------------------------------------------------------
-template <class T>
-__global__ void __launch_bounds__(kBlock)
-    k_adj_st_rec(int n, const T* __restrict__ rdens, const V4<T>* __restrict__ vbar,
-                 V4<T>* __restrict__ brec, const TsphControl* ctrl) {
-  const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const T s = rdens[i] * (T)ctrl->dt;
-  const V4<T> u = vbar[i];
-  brec[i] = V4<T>{s * u.x, s * u.y, s * u.z, T(0)};
-}
-
 // A quad of lanes per particle, as in the forward walk, with kStRevU candidate
 // records of two gathers each in flight per lane.  At 200k particles, one lane
 // with 4 in flight 90 us; quads with 1 / 2 / 3 / 4 / 6 in flight 75 / 72 / 74 /
@@ -507,16 +507,21 @@ struct Rec4 {
 
 // Per fluid particle: a_bar = dt u and fv = 2 (2 + d) mu / rho0, the record
 // the viscosity reverse gathers per neighbour (one gather instead of u and
-// rho0 apart).
+// rho0 apart); with brec also rho0 dt u, the surface-tension reverse's.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_adj_vis_rec(KP<T> k, int n, const T* __restrict__ rdens, const V4<T>* __restrict__ vbar,
-                  V4<T>* __restrict__ arec, const TsphControl* ctrl) {
+    k_adj_vel_rec(KP<T> k, int n, const T* __restrict__ rdens, const V4<T>* __restrict__ vbar,
+                  V4<T>* __restrict__ arec, V4<T>* __restrict__ brec, const TsphControl* ctrl) {
   const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (i >= n) return;
   const T dt = (T)ctrl->dt;
   const V4<T> u = vbar[i];
-  arec[i] = v4(dt * u.x, dt * u.y, dt * u.z, k.two_d2 * k.mu * f_rcp(rdens[i]));
+  const T rho = rdens[i];
+  arec[i] = v4(dt * u.x, dt * u.y, dt * u.z, k.two_d2 * k.mu * f_rcp(rho));
+  if (brec) {
+    const T s = rho * dt;
+    brec[i] = v4(s * u.x, s * u.y, s * u.z);
+  }
 }
 
 template <class T>
@@ -616,6 +621,70 @@ __global__ void __launch_bounds__(kBlock)
   }
   double s = block_sum(msum, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// Several copies in one launch.  A taped step records eleven fields, a
+// checkpoint eight: as single copies of 1-16 MB each costs its launch and its
+// drain, here one launch moves them all at memory rate (a checkpoint of 200k
+// particles, 10 MB: 14.7 us as single copies back to back, now 4.5).  A block
+// moves one chunk of one copy; both ends are 16-byte aligned for whole
+// tensors, the 4-byte and byte paths are for what is not.
+constexpr int kCopyChunk = kBlock * 16 * 4;
+struct CopyList {
+  TsphCopy c[TSPH_COPY_MAX];
+  int first[TSPH_COPY_MAX];  // first block of each copy, INT_MAX past the last
+};
+typedef uint32_t Word4 __attribute__((ext_vector_type(4)));
+// Every trip's loads go out together: a slot past the end reads the last one
+// again (a branch around each load would wait for it before the next).
+template <class V>
+__device__ __forceinline__ void copy_chunk(char* d, const char* s, int bytes) {
+  constexpr int U = 4;
+  const int m = bytes / (int)sizeof(V);
+  for (int e = threadIdx.x; e < m; e += U * kBlock) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = ((const V*)s)[min(e + u * kBlock, m - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e + u * kBlock < m) ((V*)d)[e + u * kBlock] = v[u];
+  }
+  for (int e = m * (int)sizeof(V) + threadIdx.x; e < bytes; e += kBlock) d[e] = s[e];
+}
+__global__ void __launch_bounds__(kBlock) k_copy_many(CopyList l) {
+  int q = 0;
+#pragma unroll
+  for (int t = 1; t < TSPH_COPY_MAX; ++t) q += l.first[t] <= (int)blockIdx.x;
+  const long o = (long)((int)blockIdx.x - l.first[q]) * kCopyChunk;
+  const long left = (long)l.c[q].bytes - o;
+  char* d = (char*)l.c[q].dst + o;
+  const char* s = (const char*)l.c[q].src + o;
+  const int bytes = left < kCopyChunk ? (int)left : kCopyChunk;
+  const uintptr_t low = (uintptr_t)d | (uintptr_t)s;
+  if ((low & 15) == 0)
+    copy_chunk<Word4>(d, s, bytes);
+  else if ((low & 3) == 0)
+    copy_chunk<uint32_t>(d, s, bytes);
+  else
+    copy_chunk<uint8_t>(d, s, bytes);
+}
+
+int copy_many(const TsphCopy* c, int count, hipStream_t st) {
+  CopyList l{};
+  int m = 0;
+  long blocks = 0;
+  for (int q = 0; q < count; ++q) {
+    if (c[q].bytes == 0) continue;
+    l.c[m] = c[q];
+    l.first[m++] = (int)blocks;
+    blocks += (long)((c[q].bytes + kCopyChunk - 1) / kCopyChunk);
+    TSPH_REQUIRE(blocks < (1L << 30), TSPH_EINVAL, "tsph_copy_many: too many bytes");
+  }
+  if (m == 0) return 0;
+  for (int q = m; q < TSPH_COPY_MAX; ++q) l.first[q] = 0x7fffffff;
+  hipLaunchKernelGGL(k_copy_many, dim3((int)blocks), dim3(kBlock), 0, st, l);
+  TSPH_LAUNCH_CHECK("copy_many");
+  return 0;
 }
 
 // Adds the block partials of a parameter gradient into grad[slot], in a
@@ -773,11 +842,15 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
   int nb = blocks_for(f->n);
   // nbar == NULL: gamma == 0 and its gradient is not wanted, so every term
   // of the surface-tension reverse vanishes and it is skipped
+  //
+  // (dt vbar, fv) per particle into the workspace's boundary alpha_1 buffer
+  // (pass A's output for the forward psi sweeps, free during a reverse) and
+  // b_j = rho0_j dt vbar_j into its record buffer (free between forward Jacobi
+  // iterations)
+  hipLaunchKernelGGL(k_adj_vel_rec<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
+                     (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.a1b,
+                     a->nbar ? (V4<T>*)L.krec : (V4<T>*)nullptr, ctrl);
   if (a->nbar) {
-    // b_j = rho0_j dt vbar_j into the workspace's record buffer (free between
-    // forward Jacobi iterations)
-    hipLaunchKernelGGL(k_adj_st_rec<T>, dim3(nb), dim3(kBlock), 0, st, f->n,
-                       (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.krec, ctrl);
     hipLaunchKernelGGL(k_adj_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
                        f->capacity, (const V4<T>*)f->pos, (const T*)f->mass,
                        (const T*)f->sph_density, (const T*)f->rest_density,
@@ -788,10 +861,6 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
     hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
                        coop_blocks<kQuad>(f->n), a->grad, 1);
   }
-  // (dt vbar, fv) per particle into the workspace's boundary alpha_1 buffer
-  // (pass A's output for the forward psi sweeps, free during a reverse)
-  hipLaunchKernelGGL(k_adj_vis_rec<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
-                     (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.a1b, ctrl);
   hipLaunchKernelGGL(k_adj_viscosity<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
                      f->n, f->capacity,
                      (const V4<T>*)f->pos, (const T*)f->sph_density,
@@ -829,7 +898,7 @@ int adj_bound_sums(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphAdjo
                    hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   if (f->n == 0) return 0;
-  hipLaunchKernelGGL(k_adj_bound_sums<T>, dim3(blocks_for(f->n)), dim3(kBlock), 0, st, k, f->n,
+  hipLaunchKernelGGL(k_adj_bound_sums<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
                      f->capacity, (const V4<T>*)f->pos, f->nbr_nb, (const V4<T>*)b->pos,
                      b->cell_start, (V4<T>*)a->bmom, a->bflag);
   TSPH_LAUNCH_CHECK("adj_bound_sums");

@@ -113,6 +113,7 @@ template <class T>
 int adj_density_alpha(const TsphParams&, TsphObject*, TsphObject*, TsphAdjoint*, hipStream_t);
 template <class T>
 int adj_bound_sums(const TsphParams&, TsphObject*, TsphObject*, TsphAdjoint*, hipStream_t);
+int copy_many(const TsphCopy*, int, hipStream_t);
 template <class T>
 int advect(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen,
            hipStream_t);
@@ -446,6 +447,15 @@ int tsph_adj_end(const TsphParams* p, TsphObject* f, TsphAdjoint* adj, const int
   if (int rc = check_adj(p, adj, "tsph_adj_end")) return rc;
   TSPH_REQUIRE(pid && xbar_ref && vbar_ref, TSPH_EINVAL, "tsph_adj_end: null array");
   return DISPATCH(p, adj_end, *p, f, adj, pid, xbar_ref, vbar_ref, (hipStream_t)stream);
+}
+
+int tsph_copy_many(const TsphCopy* copies, int32_t count, void* stream) {
+  TSPH_REQUIRE(count >= 0 && count <= TSPH_COPY_MAX && (copies || count == 0), TSPH_EINVAL,
+               "tsph_copy_many: 0 to %d copies", TSPH_COPY_MAX);
+  for (int q = 0; q < count; ++q)
+    TSPH_REQUIRE(copies[q].bytes == 0 || (copies[q].dst && copies[q].src), TSPH_EINVAL,
+                 "tsph_copy_many: null array");
+  return copy_many(copies, count, (hipStream_t)stream);
 }
 
 int tsph_adj_solver_iteration(const TsphParams* p, TsphObject* f, TsphObject* b,
