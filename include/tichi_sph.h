@@ -138,7 +138,8 @@ typedef struct TsphControl {
   int32_t run_u[TSPH_MAX_ITER_LOG];
   double err_div[TSPH_MAX_ITER_LOG];
   double err_incom[TSPH_MAX_ITER_LOG];
-  int32_t overflow_f, overflow_b, counter2, pad;
+  int32_t overflow_f, overflow_b, counter2;
+  int32_t go;            /* tsph_step: the calls launched ahead of a solve's end may run */
   uint64_t signal;       /* host address for the early stop signal, or 0 (tsph_solver_begin_signal) */
   int32_t token, pad2;   /* the value the signal's first word receives */
 } TsphControl;
@@ -351,13 +352,13 @@ int tsph_wcsph(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphCo
 typedef struct TsphStep {
   int32_t cfl, wcsph, fbm;
   int32_t token;         /* last token used; advanced by each wait */
-  uint64_t *signal_host; /* 8 bytes of tsph_signal_alloc: the host's address, */
+  uint64_t *signal_host; /* 16 bytes of tsph_signal_alloc: the host's address, */
   uint64_t *signal;      /* and the device's */
   int32_t pred[2];       /* iterations of each solve launched before its first wait; on
                             return those that ran (at least 1), the next step's guess */
   int32_t iters[2];      /* out: iterations that ran (divergence, density) */
   int32_t fbm_rounds;    /* out: FBM rounds launched */
-  int32_t pad;
+  int32_t hold;          /* steps left that launch nothing ahead (after a wrong guess) */
 } TsphStep;
 int tsph_step(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphControl* ctrl,
               TsphStep* step, void* workspace, size_t ws_bytes, void* stream);

@@ -71,7 +71,7 @@ class TsphControl(ctypes.Structure):
         ("run_u", _i32 * TSPH_MAX_ITER_LOG),
         ("err_div", _f64 * TSPH_MAX_ITER_LOG),
         ("err_incom", _f64 * TSPH_MAX_ITER_LOG),
-        ("overflow_f", _i32), ("overflow_b", _i32), ("counter2", _i32), ("pad", _i32),
+        ("overflow_f", _i32), ("overflow_b", _i32), ("counter2", _i32), ("go", _i32),
         ("signal", ctypes.c_uint64), ("token", _i32), ("pad2", _i32),
     ]
 
@@ -92,7 +92,7 @@ class TsphBatchInfo(ctypes.Structure):
 class TsphStep(ctypes.Structure):
     _fields_ = [("cfl", _i32), ("wcsph", _i32), ("fbm", _i32), ("token", _i32),
                 ("signal_host", _vp), ("signal", _vp), ("pred", _i32 * 2), ("iters", _i32 * 2),
-                ("fbm_rounds", _i32), ("pad", _i32)]
+                ("fbm_rounds", _i32), ("hold", _i32)]
 
 
 COPY_MAX = 16

@@ -422,10 +422,20 @@ __device__ __forceinline__ void k_finalize_body(Blk blk, KP<T> k, int mode, cons
   }
 }
 
+// Kernels launched ahead (tsph_step): the advection goes when the divergence
+// solve stopped within the `after` iterations launched before it (0: not
+// launched ahead), which it records in ctrl->go for the kernels up to the
+// tail; the tail needs the density solve's stop as well.  A kernel that
+// may not go returns at once and is launched again after the wait.
+__device__ __forceinline__ bool may_go(const TsphControl* ctrl, int after) {
+  return after == 0 || ctrl->run_u[after] == 0;
+}
+
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_finalize(KP<T> k, int mode, const double* __restrict__ partial, int nblk, int n,
-               TsphControl* ctrl) {
+               TsphControl* ctrl, int after) {
+  if (after && !(ctrl->go && may_go(ctrl, after))) return;
   k_finalize_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, mode, partial, nblk, n, ctrl);
 }
 
@@ -471,6 +481,7 @@ __device__ __forceinline__ void solver_begin_body(const KP<T>& k, TsphControl* c
 struct SolveOpen {
   uint64_t* signal;
   int token, on;
+  int ahead;  // launched before the divergence solve was known to have ended
 };
 
 }  // namespace tsph

@@ -674,7 +674,9 @@ __global__ void __launch_bounds__(kBlock)
                  V4<T>* __restrict__ krec, const V4<T>* __restrict__ a1b,
                  V4<T>* __restrict__ tape_v, T* __restrict__ tape_k,
                  const T* __restrict__ clamp_ref,
-                 double* __restrict__ partial, TsphControl* ctrl) {
+                 double* __restrict__ partial, TsphControl* ctrl, int ahead) {
+  const int run = ctrl->run_u[kk], go = ctrl->go;  // in flight together
+  if (!run || (ahead && !go)) return;
   k_solver_psi_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, kk, fpos, vadv, psi_rho, rdens, alpha, fstart, bpos, bstart, nbr_f, nbr_b, nbr_nf, nbr_nb, psi_adv, kappa, krec, a1b, tape_v, tape_k, clamp_ref, partial, ctrl);
 }
 
@@ -773,7 +775,9 @@ __global__ void __launch_bounds__(kBlock)
                     const int* __restrict__ bstart, const int* __restrict__ nbr_f,
                     const int* __restrict__ nbr_b, const int* __restrict__ nbr_nf,
                     const int* __restrict__ nbr_nb, V4<T>* __restrict__ vadv,
-                    const double* __restrict__ partial, TsphControl* ctrl) {
+                    const double* __restrict__ partial, TsphControl* ctrl, int ahead) {
+  const int run = ctrl->run_u[kk], go = ctrl->go;  // in flight together
+  if (!run || (ahead && !go)) return;
   k_solver_update_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, kk, fpos, fmass, kappa, krec, alpha_1, fstart, bpos, bstart, nbr_f, nbr_b, nbr_nf, nbr_nb, vadv, partial, ctrl);
 }
 
@@ -857,7 +861,10 @@ __global__ void __launch_bounds__(kBlock)
              const int* __restrict__ nbr_f, const int* __restrict__ nbr_nf,
              V4<T>* __restrict__ vadv, V4<T>* __restrict__ vel, V4<T>* __restrict__ acce_adv,
              V4<T>* __restrict__ normal, const T* __restrict__ fmass,
-             const T* __restrict__ psi_rho, V4<T>* __restrict__ strec) {
+             const T* __restrict__ psi_rho, V4<T>* __restrict__ strec, TsphControl* ctrl, int after) {
+  const bool go = may_go(ctrl, after);
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->go = go;
+  if (!go) return;
   k_advect_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, vf, rdens, fstart, bstart, bpos, nbr_f, nbr_nf, vadv, vel, acce_adv, normal, fmass, psi_rho, strec);
 }
 
@@ -964,6 +971,7 @@ __global__ void __launch_bounds__(kBlock)
                      const V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
                      TsphControl* ctrl, SolveOpen open) {
   TSPH_STRICT
+  if (open.ahead && !ctrl->go) return;
   if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
   const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (i >= n) return;
@@ -982,6 +990,7 @@ __global__ void __launch_bounds__(kBlock)
                       const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
                       V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
                       TsphControl* ctrl, SolveOpen open) {
+  if (open.ahead && !ctrl->go) return;
   if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
   k_surface_tension_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
 }
@@ -1265,7 +1274,8 @@ __global__ void __launch_bounds__(kBlock)
     k_tail(KP<T> k, int n, int fbm, V4<T>* __restrict__ pos, V4<T>* __restrict__ vel,
            const V4<T>* __restrict__ vadv, T* __restrict__ mass, T* __restrict__ rdens,
            const T* __restrict__ rvol, T* __restrict__ vf, const T* __restrict__ tmp,
-           const int* __restrict__ flag, double* __restrict__ partial, TsphControl* ctrl) {
+           const int* __restrict__ flag, double* __restrict__ partial, TsphControl* ctrl, int after) {
+  if (after && !(ctrl->go && may_go(ctrl, after))) return;
   k_tail_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, fbm, pos, vel, vadv, mass, rdens, rvol, vf, tmp, flag, partial, ctrl);
 }
 
@@ -1397,7 +1407,7 @@ int solver_begin(const TsphParams& prm, TsphControl* ctrl, int solve, int* signa
 template <class T>
 int solver_half(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctrl, int kk,
                 int half, void* tape_v, void* tape_k, const void* clamp_ref, void* ws, size_t wsb,
-                hipStream_t st) {
+                int ahead, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
@@ -1413,12 +1423,12 @@ int solver_half(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl
                        (const V4<T>*)b->pos, b->cell_start, f->nbr_f, f->nbr_b, f->nbr_nf,
                        f->nbr_nb, (T*)f->psi_adv, (T*)f->kappa, (V4<T>*)L.krec,
                        (const V4<T>*)L.a1b, (V4<T>*)tape_v, (T*)tape_k, (const T*)clamp_ref,
-                       L.partial, ctrl);
+                       L.partial, ctrl, ahead);
   if (half & 2)
     hipLaunchKernelGGL(k_solver_update<T>, dim3(coop_blocks<kCoopU>(f->n)), dim3(kBlock), 0, st,
                        k, f->n, f->capacity, kk, (const V4<T>*)f->pos, (const T*)f->mass, (const T*)f->kappa,
                        (const V4<T>*)L.krec, (const V4<T>*)f->alpha_1, f->cell_start, (const V4<T>*)b->pos, b->cell_start, f->nbr_f, f->nbr_b,
-                       f->nbr_nf, f->nbr_nb, (V4<T>*)f->vel_adv, L.partial, ctrl);
+                       f->nbr_nf, f->nbr_nb, (V4<T>*)f->vel_adv, L.partial, ctrl, ahead);
   TSPH_LAUNCH_CHECK("solver_iteration");
   return 0;
 }
@@ -1437,7 +1447,7 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
                      f->capacity, (const V4<T>*)f->pos, (const T*)f->volume_frac, (const T*)f->rest_density,
                      f->cell_start, b->cell_start, (const V4<T>*)b->pos, f->nbr_f, f->nbr_nf,
                      (V4<T>*)f->vel_adv, (V4<T>*)f->vel, (V4<T>*)f->acce_adv,
-                     (V4<T>*)f->normal, (const T*)f->mass, psi, (V4<T>*)L.krec);
+                     (V4<T>*)f->normal, (const T*)f->mass, psi, (V4<T>*)L.krec, ctrl, open.ahead);
   if (k.gamma == T(0))
     hipLaunchKernelGGL(k_vel_adv_update<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                        (const V4<T>*)f->vel, (const V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl,
@@ -1488,7 +1498,7 @@ int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws,
 
 template <class T>
 int tail(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, int fbm, void* ws, size_t wsb,
-         hipStream_t st) {
+         int after, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
@@ -1497,9 +1507,9 @@ int tail(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, int fbm, void*
   hipLaunchKernelGGL(k_tail<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n, fbm, (V4<T>*)f->pos,
                      (V4<T>*)f->vel, (const V4<T>*)f->vel_adv, (T*)f->mass,
                      (T*)f->rest_density, (const T*)f->rest_volume, (T*)f->volume_frac,
-                     (const T*)f->volume_frac_tmp, f->flag, L.partial, ctrl);
+                     (const T*)f->volume_frac_tmp, f->flag, L.partial, ctrl, after);
   hipLaunchKernelGGL(k_finalize<T>, dim3(1), dim3(kBlock), 0, st, k, (int)kFinEnergy, L.partial, nb,
-                     f->n, ctrl);
+                     f->n, ctrl, after);
   TSPH_LAUNCH_CHECK("tail");
   return 0;
 }
@@ -1908,13 +1918,13 @@ template int density_alpha<float>(const TsphParams&, TsphObject*, TsphObject*, T
 template int density_alpha<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, bool, hipStream_t);
 template int solver_begin<float>(const TsphParams&, TsphControl*, int, int*, int, hipStream_t);
 template int solver_begin<double>(const TsphParams&, TsphControl*, int, int*, int, hipStream_t);
-template int solver_half<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, hipStream_t);
-template int solver_half<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, hipStream_t);
+template int solver_half<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, int, hipStream_t);
+template int solver_half<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, int, hipStream_t);
 template int advect<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
 template int advect<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
 template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
 template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
-template int tail<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
-template int tail<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, hipStream_t);
+template int tail<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, int, hipStream_t);
+template int tail<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, int, hipStream_t);
 
 }  // namespace tsph
