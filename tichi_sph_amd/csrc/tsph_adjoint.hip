@@ -95,9 +95,19 @@ __device__ __forceinline__ void add_J(T& ax, T& ay, T& az, const D2<T>& d, T dx,
 constexpr int kBsumU = 4;  // boundary candidates in flight per lane
 // Lanes per particle of the reverse Jacobi and viscosity sweeps.  Their pair
 // terms (kernel second derivatives, Hessian products) make them VALU-bound
-// about as much as gather-bound, so two lanes per particle, which leave fewer
-// lanes idle at the end of uneven lists, beat the forward sweeps' four.
+// about as much as gather-bound, so in large scenes two lanes per particle,
+// which leave fewer lanes idle at the end of uneven lists, beat the forward
+// sweeps' four; in small ones the lists' chains count and four win.  us with
+// two / four lanes, the kappa half: FP32 14k 6.6 / 5.0, 98k 12.4 / 11.5, 200k
+// (compressed) 19.6 / 18.6, 405k 36.0 / 36.0, 593k 49.0 / 50.5, 1M 83.7 / 87.4;
+// FP64 14k 9.7 / 6.8, 98k 20.8 / 21.8.  The FP32 viscosity gathers four records
+// a pair and takes four lanes at every size: 14k 10.9 / 7.5, 216k 30.1 / 30.2,
+// 405k 53.0 / 49.0, 1M 139.9 / 124.2; FP64 14k 12.6 / 10.1, 98k 27.0 / 29.6.
 constexpr int kCoopR = 2;
+template <class T>
+static constexpr int adj_quad_max() {
+  return sizeof(T) == 4 ? 256 * 1024 : 48 * 1024;
+}
 // Gathers in flight per lane in the reverse viscosity sweep.  Its four-vector
 // records take 152 VGPRs at four in flight (3 waves per SIMD); two keep it at
 // 110 (4 waves) and run faster.  The Jacobi sweeps keep four: at two they
@@ -221,7 +231,7 @@ __global__ void __launch_bounds__(kBlock)
 // the kernel that wrote vbar), so a neighbour costs two 16-byte gathers;
 // psi_bar is written into the w lane of the iteration's vel_adv record,
 // where the second half gathers it.
-template <class T>
+template <class T, int C>
 __global__ void __launch_bounds__(kBlock)
     k_adj_kappa(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                 const T* __restrict__ alpha, const V4<T>* __restrict__ vbar,
@@ -229,9 +239,9 @@ __global__ void __launch_bounds__(kBlock)
                 const int* __restrict__ nbr_nf, const V4<T>* __restrict__ bmom,
                 const int* __restrict__ bflag, V4<T>* __restrict__ tvel, T* __restrict__ rhobar,
                 T* __restrict__ alphabar, V4<T>* __restrict__ xbar, const TsphControl* ctrl) {
-  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int i = coop_particle<C>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
-  const int cl = coop_lane<kCoopR>();
+  const int cl = coop_lane<C>();
   const T dt = (T)ctrl->dt;
   const V4<T> p = fpos[i];
   const T Xi = p.w;
@@ -263,14 +273,14 @@ __global__ void __launch_bounds__(kBlock)
   };
   // (f,f) pairs; the (f,b) pairs (u_b = kappa_b = 0) are w_l . A_l and
   // kappa_l M_l w_l from the boundary sums
-  sweep_lists_coop<kCoopR, T, Rec2<T>>(
+  sweep_lists_coop<C, T, Rec2<T>>(
       k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0,
       [&](int j) { return Rec2<T>{fpos[j], vbar[j]}; }, [&](int) { return Rec2<T>{}; },
       term, [&](const Rec2<T>&, bool) {});
-  kb = group_sum<kCoopR>(kb);
-  ax = group_sum<kCoopR>(ax);
-  ay = group_sum<kCoopR>(ay);
-  az = group_sum<kCoopR>(az);
+  kb = group_sum<C>(kb);
+  ax = group_sum<C>(ax);
+  ay = group_sum<C>(ay);
+  az = group_sum<C>(az);
   if (cl != 0) return;
   if (hb) {
     kb += bs.dot_A(wx, wy, wz);
@@ -292,7 +302,7 @@ __global__ void __launch_bounds__(kBlock)
 //   x_bar_l += dt sum_j J (psib_l X_j + psib_j X_l) (v_l - v_j)
 // with v the recorded vel_adv entering the iteration (boundary: v_j = 0,
 // psib_j = 0).
-template <class T>
+template <class T, int C>
 __global__ void __launch_bounds__(kBlock)
     k_adj_vel(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
               const V4<T>* __restrict__ tvel, const V4<T>* __restrict__ vbar,
@@ -300,9 +310,9 @@ __global__ void __launch_bounds__(kBlock)
               const int* __restrict__ nbr_f, const int* __restrict__ nbr_nf,
               const V4<T>* __restrict__ bmom, const int* __restrict__ bflag,
               V4<T>* __restrict__ vbar_out, V4<T>* __restrict__ xbar, const TsphControl* ctrl) {
-  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int i = coop_particle<C>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
-  const int cl = coop_lane<kCoopR>();
+  const int cl = coop_lane<C>();
   const T dt = (T)ctrl->dt;
   const V4<T> p = fpos[i];
   const T Xi = p.w;
@@ -333,16 +343,16 @@ __global__ void __launch_bounds__(kBlock)
   };
   // (f,f) pairs; the (f,b) pairs (v_b = psib_b = 0) are psib_l A_l and
   // psib_l M_l v_l from the boundary sums
-  sweep_lists_coop<kCoopR, T, Rec2<T>>(
+  sweep_lists_coop<C, T, Rec2<T>>(
       k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0,
       [&](int j) { return Rec2<T>{fpos[j], tvel[j]}; }, [&](int) { return Rec2<T>{}; }, term,
       [&](const Rec2<T>&, bool) {});
-  vx = group_sum<kCoopR>(vx);
-  vy = group_sum<kCoopR>(vy);
-  vz = group_sum<kCoopR>(vz);
-  ax = group_sum<kCoopR>(ax);
-  ay = group_sum<kCoopR>(ay);
-  az = group_sum<kCoopR>(az);
+  vx = group_sum<C>(vx);
+  vy = group_sum<C>(vy);
+  vz = group_sum<C>(vz);
+  ax = group_sum<C>(ax);
+  ay = group_sum<C>(ay);
+  az = group_sum<C>(az);
   if (cl != 0) return;
   if (hb) {
     vx += pbi * bs.m0.x;
@@ -524,7 +534,7 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-template <class T>
+template <class T, int C>
 __global__ void __launch_bounds__(kBlock)
     k_adj_viscosity(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                     const T* __restrict__ dens,
@@ -538,8 +548,8 @@ __global__ void __launch_bounds__(kBlock)
                     V4<T>* __restrict__ xbar, double* __restrict__ partial,
                     const TsphControl* ctrl) {
   __shared__ double lds[kWaves];
-  const int i = coop_particle<kCoopR>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
-  const int cl = coop_lane<kCoopR>();
+  const int i = coop_particle<C>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int cl = coop_lane<C>();
   double msum = 0;
   if (i < n) {
     const T dt = (T)ctrl->dt;
@@ -595,21 +605,21 @@ __global__ void __launch_bounds__(kBlock)
       xby += -k.h * (e.g * cy + s * dy);
       xbz += -k.h * (e.g * cz + s * dz);
     };
-    sweep_lists_coop<kCoopR, T, Rec4<T>, kNbVis>(
+    sweep_lists_coop<C, T, Rec4<T>, kNbVis>(
         k, cap, i, cl, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
         [&](int j) {
           // tvel.w = V_j; arec = (dt u_j, fv_j)
           return Rec4<T>{fpos[j], tvel[j], arec[j], nbar ? nbar[j] : V4<T>{}};
         },
         [&](int j) { return Rec4<T>{}; }, term, [&](const Rec4<T>&, bool) {});
-    vbx = group_sum<kCoopR>(vbx);
-    vby = group_sum<kCoopR>(vby);
-    vbz = group_sum<kCoopR>(vbz);
-    xbx = group_sum<kCoopR>(xbx);
-    xby = group_sum<kCoopR>(xby);
-    xbz = group_sum<kCoopR>(xbz);
-    Vb = group_sum<kCoopR>(Vb);
-    ms = group_sum<kCoopR>(ms);
+    vbx = group_sum<C>(vbx);
+    vby = group_sum<C>(vby);
+    vbz = group_sum<C>(vbz);
+    xbx = group_sum<C>(xbx);
+    xby = group_sum<C>(xby);
+    xbz = group_sum<C>(xbz);
+    Vb = group_sum<C>(Vb);
+    ms = group_sum<C>(ms);
     if (cl == 0) {
       vbar_out[i] = v4(ui.x + vbx, ui.y + vby, ui.z + vbz, kn);
       // V_i = X_i / psi_i enters only pair terms; a particle outside the grid
@@ -815,18 +825,22 @@ int adj_solver_iteration(const TsphParams& prm, TsphObject* f, TsphObject* b, Ts
   KP<T> k = make_kp<T>(prm);
   if (f->n == 0) return 0;
   (void)b;  // the boundary enters through the boundary sums
-  hipLaunchKernelGGL(k_adj_kappa<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
-                     f->n, f->capacity,
-                     (const V4<T>*)f->pos, (const T*)f->alpha, (const V4<T>*)a->vbar,
-                     f->cell_start, f->nbr_f, f->nbr_nf, (const V4<T>*)a->bmom, a->bflag,
-                     (V4<T>*)a->tape_vel_adv, (T*)a->rhobar, (T*)a->alphabar, (V4<T>*)a->xbar,
-                     ctrl);
-  hipLaunchKernelGGL(k_adj_vel<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
-                     f->n, f->capacity,
-                     (const V4<T>*)f->pos, (const V4<T>*)a->tape_vel_adv, (const V4<T>*)a->vbar,
-                     (const T*)a->kappa_next, f->cell_start, f->nbr_f, f->nbr_nf,
-                     (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->vbar_out, (V4<T>*)a->xbar,
-                     ctrl);
+  auto iteration = [&](auto kappa, auto vel, int nb) {
+    hipLaunchKernelGGL(kappa, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                       (const V4<T>*)f->pos, (const T*)f->alpha, (const V4<T>*)a->vbar,
+                       f->cell_start, f->nbr_f, f->nbr_nf, (const V4<T>*)a->bmom, a->bflag,
+                       (V4<T>*)a->tape_vel_adv, (T*)a->rhobar, (T*)a->alphabar, (V4<T>*)a->xbar,
+                       ctrl);
+    hipLaunchKernelGGL(vel, dim3(nb), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                       (const V4<T>*)f->pos, (const V4<T>*)a->tape_vel_adv,
+                       (const V4<T>*)a->vbar, (const T*)a->kappa_next, f->cell_start, f->nbr_f,
+                       f->nbr_nf, (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->vbar_out,
+                       (V4<T>*)a->xbar, ctrl);
+  };
+  if (f->n <= adj_quad_max<T>())
+    iteration(k_adj_kappa<T, kQuad>, k_adj_vel<T, kQuad>, coop_blocks<kQuad>(f->n));
+  else
+    iteration(k_adj_kappa<T, kCoopR>, k_adj_vel<T, kCoopR>, coop_blocks<kCoopR>(f->n));
   TSPH_LAUNCH_CHECK("adj_solver_iteration");
   return 0;
 }
@@ -861,16 +875,19 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
     hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
                        coop_blocks<kQuad>(f->n), a->grad, 1);
   }
-  hipLaunchKernelGGL(k_adj_viscosity<T>, dim3(coop_blocks<kCoopR>(f->n)), dim3(kBlock), 0, st, k,
-                     f->n, f->capacity,
-                     (const V4<T>*)f->pos, (const T*)f->sph_density,
-                     (const T*)f->rest_density, f->cell_start, (const int*)nullptr,
-                     (const V4<T>*)nullptr, f->nbr_f, f->nbr_nf, (const V4<T>*)a->tape_vel,
-                     (const V4<T>*)a->nbar, (const V4<T>*)a->vbar, (const V4<T>*)L.a1b,
-                     (const T*)a->kappa_next,
-                     (V4<T>*)a->vbar_out, (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
-  hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
-                     coop_blocks<kCoopR>(f->n), a->grad, 0);
+  auto viscosity = [&](auto kern, int nbk) {
+    hipLaunchKernelGGL(kern, dim3(nbk), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                       (const V4<T>*)f->pos, (const T*)f->sph_density, (const T*)f->rest_density,
+                       f->cell_start, (const int*)nullptr, (const V4<T>*)nullptr, f->nbr_f,
+                       f->nbr_nf, (const V4<T>*)a->tape_vel, (const V4<T>*)a->nbar,
+                       (const V4<T>*)a->vbar, (const V4<T>*)L.a1b, (const T*)a->kappa_next,
+                       (V4<T>*)a->vbar_out, (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
+    hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial, nbk, a->grad, 0);
+  };
+  if (sizeof(T) == 4 || f->n <= adj_quad_max<T>())
+    viscosity(k_adj_viscosity<T, kQuad>, coop_blocks<kQuad>(f->n));
+  else
+    viscosity(k_adj_viscosity<T, kCoopR>, coop_blocks<kCoopR>(f->n));
   TSPH_LAUNCH_CHECK("adj_advect");
   return 0;
 }
