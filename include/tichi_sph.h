@@ -352,7 +352,7 @@ int tsph_wcsph(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphCo
 typedef struct TsphStep {
   int32_t cfl, wcsph, fbm;
   int32_t token;         /* last token used; advanced by each wait */
-  uint64_t *signal_host; /* 16 bytes of tsph_signal_alloc: the host's address, */
+  uint64_t *signal_host; /* 24 bytes of tsph_signal_alloc: the host's address, */
   uint64_t *signal;      /* and the device's */
   int32_t pred[2];       /* iterations of each solve launched before its first wait; on
                             return those that ran (at least 1), the next step's guess */

@@ -49,9 +49,11 @@ def test_step_without_a_signal_is_refused():
                             "solver_iter_threshold_max": 7}),
     # only the density solve runs past its prediction: the tail is launched again
     ("dambreak_3d_8k", {}, {"solver_compression_threshold": 0.0, "solver_iter_threshold_max": 7}),
+    # the same under an FBM round and a tail launched ahead
+    ("two_phase_3d_4k", {"fbm": True}, {"solver_compression_threshold": 0.0, "solver_iter_threshold_max": 7}),
     # no iteration at all: the solves signal from their begin
     ("dambreak_3d_8k", {}, {"solver_iter_threshold_min": 0}),
-], ids=["2d", "3d_f64", "wcsph", "fbm", "cap", "late", "none"])
+], ids=["2d", "3d_f64", "wcsph", "fbm", "cap", "late", "late_fbm", "none"])
 def test_native_step_is_the_call_by_call_step(name, kw, edit):
     from tichi_sph_amd import EventTimer, simulation_from_dicts
     cb, sb = load_scene(name)

@@ -118,7 +118,7 @@ template <class T>
 int advect(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen,
            hipStream_t);
 template <class T>
-int fbm_round(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int,
+int fbm_round(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, int,
               hipStream_t);
 template <class T>
 int tail(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, int, hipStream_t);
@@ -421,7 +421,8 @@ int tsph_fbm_round(const TsphParams* p, TsphObject* f, TsphControl* ctrl, void* 
                    void* stream) {
   if (int rc = check_params(p)) return rc;
   if (int rc = check_obj(f, "tsph_fbm_round")) return rc;
-  return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, (uint64_t*)nullptr, 0, (hipStream_t)stream);
+  return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, (uint64_t*)nullptr, 0, 0,
+                  (hipStream_t)stream);
 }
 
 static int tail_after(const TsphParams* p, TsphObject* f, TsphControl* ctrl, int32_t fbm,
@@ -594,16 +595,18 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
     if (k[q] > kmax) k[q] = kmax;
   }
   if (int rc = step_iterations(a, 0, k[0])) return rc;
-  // The advection, the density solve and the tail are launched without waiting
-  // for the divergence solve's stop: they check on the device that it stopped
-  // within the launched iterations, and return at once otherwise (then they
-  // are launched again).  The device so never waits for the host's answer:
-  // 2D 8k 118 -> 109 us a step, 3D 8k 133 -> 127, 3D 65k FP64 214 -> 209.  A
+  // The advection, the density solve, an FBM round and the tail are launched
+  // without waiting for the divergence solve's stop: they check on the device
+  // that the solves stopped within the launched iterations (the tail also that
+  // no further round is due), and return at once otherwise (then they are
+  // launched again).  The device so never waits for the host's answer:
+  // 2D 8k 118 -> 109 us a step, 3D 8k 133 -> 127, 3D 65k FP64 214 -> 209, the
+  // 4k mixture 171 -> 164 by its round and tail.  A
   // wrong guess costs the launches that returned (about 25 us): the next
   // kStepHold steps wait at each solve again.
   const bool ahead = s->hold <= 0 && f->n > 0 && f->n <= kStepAheadMax && k[0] > 0 &&
                      k[0] < TSPH_MAX_ITER_LOG && k[1] < TSPH_MAX_ITER_LOG;
-  const bool tail_ahead = ahead && !s->wcsph && !s->fbm;
+  const bool tail_ahead = ahead && !s->wcsph;
   if (s->hold > 0) --s->hold;
   s->fbm_rounds = 0;
   SolveOpen open1{s->signal + 1, 0, 1, 0};
@@ -616,28 +619,40 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
         return rc;
     return step_iterations(a, 0, k[1], after);
   };
+  int32_t round_token = 0;
+  auto fbm_launch = [&](int after) -> int {
+    round_token = next_token(s);
+    ++s->fbm_rounds;
+    return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, s->signal + 2, (int)round_token, after,
+                    (hipStream_t)stream);
+  };
   if (ahead)
     if (int rc = density_solve(k[0])) return rc;
-  if (tail_ahead)
-    if (int rc = tail_after(p, f, ctrl, 0, ws, wsb, stream, k[1])) return rc;
+  if (tail_ahead) {
+    if (s->fbm)
+      if (int rc = fbm_launch(k[1])) return rc;
+    if (int rc = tail_after(p, f, ctrl, s->fbm, ws, wsb, stream, k[1])) return rc;
+  }
   bool late0 = false, late1 = false;
   if (int rc = step_finish(a, 0, open0.token, k[0], &late0)) return rc;
   if (!ahead || late0)
     if (int rc = density_solve(0)) return rc;
   if (int rc = step_finish(a, 1, open1.token, k[1], &late1)) return rc;
-  if ((ahead && late0) || (tail_ahead && late1)) s->hold = kStepHold;
-  if (tail_ahead && !late0 && !late1) return 0;
+  // whether what was launched ahead of both solves' stops has run
+  const bool went = tail_ahead && !late0 && !late1;
+  if (ahead && (late0 || (tail_ahead && late1))) s->hold = kStepHold;
+  if (went && !s->fbm) return 0;
   if (s->wcsph)
     if (int rc = tsph_wcsph(p, f, b, ctrl, stream)) return rc;
-  while (s->fbm && f->n > 0 && s->fbm_rounds < 1000) {
-    const hipStream_t st = (hipStream_t)stream;
-    next_token(s);
-    if (int rc = DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, s->signal, (int)s->token, st))
-      return rc;
-    ++s->fbm_rounds;
+  if (!went) s->fbm_rounds = 0;
+  bool launched = went;  // the first round
+  while (s->fbm && f->n > 0 && (launched || s->fbm_rounds < 1000)) {
+    if (!launched)
+      if (int rc = fbm_launch(0)) return rc;
     uint32_t flag = 0;
     const int rc = wait_word(
-        s->signal_host, s->token, st, &flag, [](uint32_t) { return true; },
+        s->signal_host + 2, round_token, (hipStream_t)stream, &flag,
+        [](uint32_t) { return true; },
         [&](uint32_t* low) -> int {
           int32_t v;
           const hipError_t e = hipMemcpy(&v, &ctrl->general_flag, sizeof(v), hipMemcpyDeviceToHost);
@@ -646,7 +661,12 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
           return 0;
         });
     if (rc) return rc;
-    if (!flag) break;
+    if (!flag) {
+      if (launched) return 0;  // the tail went too
+      break;
+    }
+    if (launched) s->hold = kStepHold;
+    launched = false;
   }
   return tsph_tail(p, f, ctrl, s->fbm, ws, wsb, stream);
 }

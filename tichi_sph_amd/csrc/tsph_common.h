@@ -430,12 +430,21 @@ __device__ __forceinline__ void k_finalize_body(Blk blk, KP<T> k, int mode, cons
 __device__ __forceinline__ bool may_go(const TsphControl* ctrl, int after) {
   return after == 0 || ctrl->run_u[after] == 0;
 }
+// An FBM round while any particle is flagged; launched ahead, once the density
+// solve has stopped as well.  The tail launched ahead goes when no round is
+// left to run.
+__device__ __forceinline__ bool fbm_may_go(const TsphControl* ctrl, int after) {
+  return ctrl->general_flag && (after == 0 || (ctrl->go && may_go(ctrl, after)));
+}
+__device__ __forceinline__ bool tail_may_go(const TsphControl* ctrl, int after, int fbm) {
+  return after == 0 || (ctrl->go && may_go(ctrl, after) && !(fbm && ctrl->general_flag));
+}
 
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_finalize(KP<T> k, int mode, const double* __restrict__ partial, int nblk, int n,
-               TsphControl* ctrl, int after) {
-  if (after && !(ctrl->go && may_go(ctrl, after))) return;
+               TsphControl* ctrl, int after, int fbm) {
+  if (!tail_may_go(ctrl, after, fbm)) return;
   k_finalize_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, mode, partial, nblk, n, ctrl);
 }
 

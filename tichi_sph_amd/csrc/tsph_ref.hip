@@ -571,7 +571,7 @@ int ref_kernel(const TsphParams& prm, int kid, TsphObject* obj, const TsphObject
                : kid == TSPH_K_IPPE_psi_adv_non_negative ? kFinCompression : -1;
     if (mode >= 0)
       hipLaunchKernelGGL(k_finalize<T>, dim3(1), dim3(kBlock), 0, st, k, mode, L.partial, nb,
-                         obj->n, ctrl, 0);
+                         obj->n, ctrl, 0, 0);
   }
   TSPH_LAUNCH_CHECK("ref_kernel");
   return 0;

@@ -1003,9 +1003,9 @@ __global__ void __launch_bounds__(kBlock)
     k_fbm_drift(KP<T> k, int n, const V4<T>* __restrict__ vadv, const V4<T>* __restrict__ vel,
                 const T* __restrict__ rdens, const T* __restrict__ vf, V4<T>* __restrict__ acce_adv,
                 V4<T>* __restrict__ acce, T* __restrict__ zeta, V4<T>* __restrict__ drift,
-                T* __restrict__ tmp, const int* __restrict__ flag, TsphControl* ctrl) {
+                T* __restrict__ tmp, const int* __restrict__ flag, TsphControl* ctrl, int after) {
   TSPH_STRICT
-  if (!ctrl->general_flag) return;
+  if (!fbm_may_go(ctrl, after)) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->fbm_rounds += 1;
   int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (i >= n) return;
@@ -1048,9 +1048,9 @@ __global__ void __launch_bounds__(kBlock)
                const T* __restrict__ rvol, const T* __restrict__ vf,
                const V4<T>* __restrict__ drift, const int* __restrict__ flag,
                const int* __restrict__ fstart, const int* __restrict__ nbr_f_in,
-               const int* __restrict__ nbr_nf, T* __restrict__ tmp, const TsphControl* ctrl) {
+               const int* __restrict__ nbr_nf, T* __restrict__ tmp, const TsphControl* ctrl, int after) {
   TSPH_STRICT
-  if (!ctrl->general_flag) return;
+  if (!fbm_may_go(ctrl, after)) return;
   int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (i >= n || flag[i] != 0) return;
   const int* nbr_f = nbr_f_in;
@@ -1121,8 +1121,8 @@ __global__ void __launch_bounds__(kBlock)
                     const V4<T>* __restrict__ drift, const int* __restrict__ flag,
                     const int* __restrict__ fstart, const int* __restrict__ nbr_f,
                     const int* __restrict__ nbr_nf, T* __restrict__ tmp,
-                    const TsphControl* ctrl) {
-  if (!ctrl->general_flag) return;
+                    const TsphControl* ctrl, int after) {
+  if (!fbm_may_go(ctrl, after)) return;
   const int i = coop_particle<kCoop>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
   const int c = coop_lane<kCoop>();
@@ -1188,10 +1188,10 @@ __global__ void __launch_bounds__(kBlock)
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_fbm_check(KP<T> k, int n, const T* __restrict__ vf, const T* __restrict__ tmp,
-                int* __restrict__ flag, double* __restrict__ partial, TsphControl* ctrl) {
+                int* __restrict__ flag, double* __restrict__ partial, TsphControl* ctrl, int after) {
   TSPH_STRICT
   __shared__ double lds[kWaves];
-  if (!ctrl->general_flag) return;
+  if (!fbm_may_go(ctrl, after)) return;
   int nblk = gridDim.x;
   int i = xcd_block(blockIdx.x, nblk) * kBlock + threadIdx.x;
   double any = 0;
@@ -1213,9 +1213,10 @@ __global__ void __launch_bounds__(kBlock)
 // With a signal, the flag also goes to the host: (token << 32) | flag.
 __global__ void __launch_bounds__(kBlock)
     k_fbm_check_finish(const double* __restrict__ partial, int nblk, TsphControl* ctrl,
-                       uint64_t* signal, int token) {
+                       uint64_t* signal, int token, int after) {
   __shared__ double lds[kWaves];
   int flag = 0;
+  if (after && !(ctrl->go && may_go(ctrl, after))) return;
   if (ctrl->general_flag) {
     double a = sum_partials(partial, nblk, lds);
     if (threadIdx.x == 0) ctrl->general_flag = flag = a > 0 ? 1 : 0;
@@ -1275,7 +1276,7 @@ __global__ void __launch_bounds__(kBlock)
            const V4<T>* __restrict__ vadv, T* __restrict__ mass, T* __restrict__ rdens,
            const T* __restrict__ rvol, T* __restrict__ vf, const T* __restrict__ tmp,
            const int* __restrict__ flag, double* __restrict__ partial, TsphControl* ctrl, int after) {
-  if (after && !(ctrl->go && may_go(ctrl, after))) return;
+  if (!tail_may_go(ctrl, after, fbm)) return;
   k_tail_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, fbm, pos, vel, vadv, mass, rdens, rvol, vf, tmp, flag, partial, ctrl);
 }
 
@@ -1464,7 +1465,7 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
 
 template <class T>
 int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws, size_t wsb,
-              uint64_t* signal, int token, hipStream_t st) {
+              uint64_t* signal, int token, int after, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   WsLayout L;
   TSPH_REQUIRE(carve_ws(ws, wsb, f->capacity, prm.node_num, &L), TSPH_ECAPACITY,
@@ -1474,12 +1475,13 @@ int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws,
   hipLaunchKernelGGL(k_fbm_drift<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                      (const V4<T>*)f->vel_adv, (const V4<T>*)f->vel, (const T*)f->rest_density,
                      (const T*)f->volume_frac, (V4<T>*)f->acce_adv, (V4<T>*)f->acce,
-                     (T*)f->fbm_zeta, (V4<T>*)f->drift_vel, (T*)f->volume_frac_tmp, f->flag, ctrl);
+                     (T*)f->fbm_zeta, (V4<T>*)f->drift_vel, (T*)f->volume_frac_tmp, f->flag, ctrl,
+                     after);
   auto flux = [&](auto kern, int nbk) {
     hipLaunchKernelGGL(kern, dim3(nbk), dim3(kBlock), 0, st, k, f->n, f->capacity,
                        (const V4<T>*)f->pos, (const T*)f->rest_volume, (const T*)f->volume_frac,
                        (const V4<T>*)f->drift_vel, f->flag, f->cell_start, f->nbr_f, f->nbr_nf,
-                       (T*)f->volume_frac_tmp, ctrl);
+                       (T*)f->volume_frac_tmp, ctrl, after);
   };
   switch (prm.phase_num) {  // the cooperative sweep keeps NP phases' records in registers
     case 1: flux(k_fbm_flux_coop<T, 1>, coop_blocks<kCoop>(f->n)); break;
@@ -1489,9 +1491,9 @@ int fbm_round(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, void* ws,
   }
   hipLaunchKernelGGL(k_fbm_check<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                      (const T*)f->volume_frac, (const T*)f->volume_frac_tmp, f->flag, L.partial,
-                     ctrl);
+                     ctrl, after);
   hipLaunchKernelGGL(k_fbm_check_finish, dim3(1), dim3(kBlock), 0, st, L.partial, nb, ctrl,
-                     signal, token);
+                     signal, token, after);
   TSPH_LAUNCH_CHECK("fbm_round");
   return 0;
 }
@@ -1509,7 +1511,7 @@ int tail(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, int fbm, void*
                      (T*)f->rest_density, (const T*)f->rest_volume, (T*)f->volume_frac,
                      (const T*)f->volume_frac_tmp, f->flag, L.partial, ctrl, after);
   hipLaunchKernelGGL(k_finalize<T>, dim3(1), dim3(kBlock), 0, st, k, (int)kFinEnergy, L.partial, nb,
-                     f->n, ctrl, after);
+                     f->n, ctrl, after, fbm);
   TSPH_LAUNCH_CHECK("tail");
   return 0;
 }
@@ -1922,8 +1924,8 @@ template int solver_half<float>(const TsphParams&, TsphObject*, TsphObject*, Tsp
 template int solver_half<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, int, int, void*, void*, const void*, void*, size_t, int, hipStream_t);
 template int advect<float>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
 template int advect<double>(const TsphParams&, TsphObject*, TsphObject*, TsphControl*, void*, size_t, SolveOpen, hipStream_t);
-template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
-template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, hipStream_t);
+template int fbm_round<float>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, int, hipStream_t);
+template int fbm_round<double>(const TsphParams&, TsphObject*, TsphControl*, void*, size_t, uint64_t*, int, int, hipStream_t);
 template int tail<float>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, int, hipStream_t);
 template int tail<double>(const TsphParams&, TsphObject*, TsphControl*, int, void*, size_t, int, hipStream_t);
 

@@ -177,14 +177,14 @@ class Simulation:
         self._ctrl_host = torch.zeros(self.ctrl.numel(), dtype=torch.uint8, pin_memory=pin)
         self._stop_host = torch.zeros(16, dtype=torch.uint8, pin_memory=pin)
         # early stop signal of the Jacobi solves (tsph_solver_begin_signal):
-        # one uint64 of pinned, device-mapped, coherent host memory, and one
-        # more for tsph_step, which has both solves in flight
+        # one uint64 of pinned, device-mapped, coherent host memory, and two
+        # more for tsph_step, which has both solves and an FBM round in flight
         self._token = 0
         self._signal_host = self._signal_dev = None
         self._signal_np = np.zeros(1, dtype=np.uint64)
         if pin:
             h, d = ctypes.c_void_p(), ctypes.c_void_p()
-            _lib.check(self.lib.tsph_signal_alloc(16, ctypes.byref(h), ctypes.byref(d)), "tsph_signal_alloc")
+            _lib.check(self.lib.tsph_signal_alloc(24, ctypes.byref(h), ctypes.byref(d)), "tsph_signal_alloc")
             self._signal_host, self._signal_dev = h, d
             self._signal_np = np.ctypeslib.as_array(ctypes.cast(h, ctypes.POINTER(ctypes.c_uint64)), shape=(1,))
         self._step = _lib.TsphStep()  # tsph_step's options and results
