@@ -193,10 +193,11 @@ __device__ __forceinline__ T group_sum(T v) {
 // group holds already) and pair(record, false) leaves it out of the sums, so
 // that the loads of a trip issue back to back.  With a branch around each
 // load instead, a trip's loads went out one exec-mask change at a time: where
-// few waves are in flight (8,000 particles in 3D) psi took 12.3 us (now
-// 10.2), update 8.8 (7.2), advection 12.8 (10.5).  From 200k particles on the
-// sweeps are bound by their cache accesses and take the same time (1M: psi
-// 75.6 and 74.0 us); fewer registers hold the same loads (psi 93 -> 78).
+// few waves are in flight (8,000 particles in 3D, four rounds a block then)
+// psi took 12.3 us with it and 10.2 without, update 8.8 and 7.2, advection
+// 12.8 and 10.5.  From 200k particles on the sweeps are bound by their cache
+// accesses and take the same time (1M: psi 75.6 and 74.0 us); fewer registers
+// hold the same loads (psi 93 -> 78).
 template <int C, class Rec, int NB = kCoopNb, class Load, class Pair>
 __device__ __forceinline__ void sweep_one_list_coop(int cap, int i, int c,
                                                     const int* __restrict__ list, int n,
