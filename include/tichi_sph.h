@@ -357,7 +357,7 @@ typedef struct TsphStep {
   int32_t pred[2];       /* iterations of each solve launched before its first wait; on
                             return those that ran (at least 1), the next step's guess */
   int32_t iters[2];      /* out: iterations that ran (divergence, density) */
-  int32_t fbm_rounds;    /* out: FBM rounds launched */
+  int32_t fbm_rounds;    /* out: FBM rounds that ran, the next step's guess */
   int32_t hold;          /* steps left that launch nothing ahead (after a wrong guess) */
 } TsphStep;
 int tsph_step(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphControl* ctrl,

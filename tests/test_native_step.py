@@ -68,5 +68,6 @@ def test_native_step_is_the_call_by_call_step(name, kw, edit):
         assert (sa.div_iter, sa.incom_iter, sa.fbm_rounds) == (sb_.div_iter, sb_.incom_iter, sb_.fbm_rounds), step
         assert (sa.dt, sa.compression, sa.kinetic_energy) == (sb_.dt, sb_.compression, sb_.kinetic_energy)
         assert a.pred == b.pred
+        assert a._step.fbm_rounds == sa.fbm_rounds
         for f in ("pos", "vel", "vel_adv", "mass", "volume_frac", "sph_density", "neighb_cell_seq"):
             assert np.array_equal(a.fluid.to_numpy(f), b.fluid.to_numpy(f)), (step, f)

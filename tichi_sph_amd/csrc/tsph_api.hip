@@ -573,6 +573,9 @@ static int step_finish(const StepArgs& a, int solve, int32_t token, int k, bool*
 
 // Steps that launch nothing ahead after one whose guess fell short.
 constexpr int kStepHold = 16;
+// FBM rounds launched ahead at most.  A 4k mixture that runs two a step takes
+// 171 us with both ahead, 184 with one (the tail returns and all wait again).
+constexpr int kStepRounds = 8;
 // Particles up to which a step launches ahead.  The stop signal leaves at the
 // start of a solve's last update, so from about here (25 us an update) the
 // host's answer arrives before that kernel ends: at 1M particles the step
@@ -595,7 +598,7 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
     if (k[q] > kmax) k[q] = kmax;
   }
   if (int rc = step_iterations(a, 0, k[0])) return rc;
-  // The advection, the density solve, an FBM round and the tail are launched
+  // The advection, the density solve, the FBM rounds and the tail are launched
   // without waiting for the divergence solve's stop: they check on the device
   // that the solves stopped within the launched iterations (the tail also that
   // no further round is due), and return at once otherwise (then they are
@@ -608,6 +611,7 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
                      k[0] < TSPH_MAX_ITER_LOG && k[1] < TSPH_MAX_ITER_LOG;
   const bool tail_ahead = ahead && !s->wcsph;
   if (s->hold > 0) --s->hold;
+  const int last_rounds = s->fbm_rounds;
   s->fbm_rounds = 0;
   SolveOpen open1{s->signal + 1, 0, 1, 0};
   auto density_solve = [&](int after) -> int {
@@ -620,16 +624,21 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
     return step_iterations(a, 0, k[1], after);
   };
   int32_t round_token = 0;
+  int rounds = 0;  // launched
   auto fbm_launch = [&](int after) -> int {
     round_token = next_token(s);
-    ++s->fbm_rounds;
+    ++rounds;
     return DISPATCH(p, fbm_round, *p, f, ctrl, ws, wsb, s->signal + 2, (int)round_token, after,
                     (hipStream_t)stream);
   };
   if (ahead)
     if (int rc = density_solve(k[0])) return rc;
   if (tail_ahead) {
-    if (s->fbm)
+    // as many rounds as the last step ran; one that is not due returns at once
+    const int guess = !s->fbm ? 0
+                      : last_rounds < 1 ? 1
+                      : last_rounds > kStepRounds ? kStepRounds : last_rounds;
+    while (rounds < guess)
       if (int rc = fbm_launch(k[1])) return rc;
     if (int rc = tail_after(p, f, ctrl, s->fbm, ws, wsb, stream, k[1])) return rc;
   }
@@ -644,28 +653,27 @@ int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ct
   if (went && !s->fbm) return 0;
   if (s->wcsph)
     if (int rc = tsph_wcsph(p, f, b, ctrl, stream)) return rc;
-  if (!went) s->fbm_rounds = 0;
-  bool launched = went;  // the first round
-  while (s->fbm && f->n > 0 && (launched || s->fbm_rounds < 1000)) {
+  if (!went) rounds = 0;
+  bool launched = went;  // the first rounds, and the tail
+  while (s->fbm && f->n > 0 && (launched || rounds < 1000)) {
     if (!launched)
       if (int rc = fbm_launch(0)) return rc;
-    uint32_t flag = 0;
+    uint32_t w = 0;
     const int rc = wait_word(
-        s->signal_host + 2, round_token, (hipStream_t)stream, &flag,
-        [](uint32_t) { return true; },
+        s->signal_host + 2, round_token, (hipStream_t)stream, &w, [](uint32_t) { return true; },
         [&](uint32_t* low) -> int {
-          int32_t v;
-          const hipError_t e = hipMemcpy(&v, &ctrl->general_flag, sizeof(v), hipMemcpyDeviceToHost);
+          TsphControl c;
+          const hipError_t e = hipMemcpy(&c, ctrl, sizeof(c), hipMemcpyDeviceToHost);
           TSPH_REQUIRE(e == hipSuccess, TSPH_EHIP, "tsph_step: %s", hipGetErrorString(e));
-          *low = (uint32_t)v;
+          *low = (uint32_t)(2 * c.fbm_rounds + (c.general_flag ? 1 : 0));
           return 0;
         });
     if (rc) return rc;
-    if (!flag) {
-      if (launched) return 0;  // the tail went too
+    s->fbm_rounds = (int32_t)(w >> 1);
+    if (!(w & 1)) {
+      if (launched) return 0;
       break;
     }
-    if (launched) s->hold = kStepHold;
     launched = false;
   }
   return tsph_tail(p, f, ctrl, s->fbm, ws, wsb, stream);

@@ -1210,7 +1210,8 @@ __global__ void __launch_bounds__(kBlock)
 
 // general_flag = any particle flagged this round (sph.py:368-372); skipped,
 // like the round itself, once the flag is clear.
-// With a signal, the flag also goes to the host: (token << 32) | flag.
+// With a signal, the flag and the rounds that ran also go to the host:
+// (token << 32) | (2 rounds + flag).
 __global__ void __launch_bounds__(kBlock)
     k_fbm_check_finish(const double* __restrict__ partial, int nblk, TsphControl* ctrl,
                        uint64_t* signal, int token, int after) {
@@ -1222,7 +1223,7 @@ __global__ void __launch_bounds__(kBlock)
     if (threadIdx.x == 0) ctrl->general_flag = flag = a > 0 ? 1 : 0;
   }
   if (signal && threadIdx.x == 0)
-    __hip_atomic_store(signal, ((uint64_t)(uint32_t)token << 32) | (uint32_t)flag,
+    __hip_atomic_store(signal, ((uint64_t)(uint32_t)token << 32) | (uint32_t)(2 * ctrl->fbm_rounds + flag),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
