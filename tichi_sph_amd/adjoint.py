@@ -144,23 +144,29 @@ class DiffRunner:
         self._move(moves, m)
 
     def _clones(self, tensors):
-        """Tensors like these contiguous ones, and the moves that fill them."""
+        """Tensors like these contiguous device ones, and the moves that fill
+        them."""
         out = [torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in tensors]
         moves = (_lib.TsphCopy * len(out))(*[(d.data_ptr(), t.data_ptr(), d.numel() * d.element_size())
                                              for d, t in zip(out, tensors)])
         return out, moves
 
     def _move(self, moves, count=None):
-        rc = self.lib.tsph_copy_many(moves, len(moves) if count is None else count, self.sim.stream_ptr())
-        _lib.check(rc, "tsph_copy_many")
+        count = len(moves) if count is None else count
+        if count:
+            _lib.check(self.lib.tsph_copy_many(moves, count, self.sim.stream_ptr()), "tsph_copy_many")
 
     _STATE = ("pos", "vel", "mass", "rest_density", "rest_volume", "volume_frac", "pid")
 
     def checkpoint(self):
         f = self.sim.fluid
         n = f.part_num
-        out, moves = self._clones([f.t[name][:n] for name in self._STATE] + [self.sim.ctrl])
-        self._move(moves)
+        state = [f.t[name][:n] for name in self._STATE] + [self.sim.ctrl]
+        if self.sim.ctrl.is_cuda:
+            out, moves = self._clones(state)
+            self._move(moves)
+        else:  # a host-only scene's state
+            out = [t.clone() for t in state]
         st = dict(zip(self._STATE + ("ctrl",), out))
         st["step_index"] = self.step_index
         return st
