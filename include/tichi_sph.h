@@ -593,6 +593,9 @@ enum {
   TSPH_K_COUNT = 26
 };
 
+/* One kernel of sph.py.  The Ngrid arrays hold each cell's entries in a range of
+ * their own, [node_part_shift, node_part_shift + node_part_count); the ranges may
+ * lie in any order (tsph_ngrid_build leaves them in cell order). */
 int tsph_ref_kernel(const TsphParams* p, int32_t kernel, TsphObject* obj, const TsphObject* nobj,
                     const int32_t* node_part_count, const int32_t* node_part_shift,
                     const int32_t* part_pid_in_node, const int32_t* part_uid_in_node,

@@ -272,20 +272,44 @@ __global__ void __launch_bounds__(kBlock)
 // (W, W' and C vanish), so leaving them out changes no value.  One kernel with
 // a switch over all ids, one lane per particle and the whole pair math on each
 // of the 200 or so candidates took 130-170 us per call at 100k particles; these
-// take 36-66 us there, bound by the dependent loads of the walk (entry, then
+// take 37-69 us there, bound by the dependent loads of the walk (entry, then
 // position).  A whole reference step at 4k / 100k / 1M: 3.5 / 4.0 / 15.5 ms,
-// now 0.94 / 1.42 / 8.7.
+// now 0.94 / 1.47 / 8.7.
 // ---------------------------------------------------------------------------
 constexpr int kRefNormal = 100, kRefForce = 101;  // surface tension's two loops
 
 // The walk around cell cs[] of particle p over nuid's candidates in range, or
-// (ALL) all of them with r > 0.
+// (ALL) all of them with r > 0.  A row of cells is one range where the Ngrid
+// holds them one after the other, as tsph_ngrid_build does; where it does not
+// (the reference's mem_shift, sph_obj.py:308-314, hands the ranges out in
+// whatever order its threads reach the cells) every cell is read by itself.
+// Asking whether it does costs 1-2 us of a call's 37-69 at 100k particles.
 template <bool ALL, class T, class Load, class Term>
 __device__ __forceinline__ void ref_quad(const KP<T>& k, const RefGrid& g, const int* cs, int nuid,
                                          const V4<T>* __restrict__ npos, const V4<T>& p,
                                          WalkLds& lds, Load&& load, Term&& term) {
-  walk_quad_cells(
-      k, cs, lds, [&](int lo, int hi) { return make_int2(g.nps[lo], g.nps[hi] + g.npc[hi]); },
+  walk_quad_cells<true>(
+      k, cs, lds,
+      [&](int lo, int hi, bool* split) {
+        int s0, end;
+        if (hi - lo == 2) {  // a row of the default range (R = 1): two loads
+          int s[3], n[3];
+          __builtin_memcpy(s, g.nps + lo, sizeof(s));
+          __builtin_memcpy(n, g.npc + lo, sizeof(n));
+          s0 = s[0];
+          end = s[2] + n[2];
+          *split |= s[1] != s0 + n[0] || s[2] != s[1] + n[1];
+        } else {
+          s0 = g.nps[lo];
+          end = s0 + g.npc[lo];
+          for (int q = lo + 1; q <= hi; ++q) {
+            const int s = g.nps[q];
+            *split |= s != end;
+            end = s + g.npc[q];
+          }
+        }
+        return make_int2(s0, end);
+      },
       [&](int s) {
         Cand<T> d;
         d.j = g.uin[s] == nuid ? g.pin[s] : -1;
@@ -306,8 +330,10 @@ struct RefRec {
   T a, b, c;
 };
 
+// The FP32 update keeps 7 waves per SIMD (a spill at its entry, for the address
+// of its result, instead of 76 registers): 54 us a call at 100k with 6, 47 with 7.
 template <class T, int KID>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock, KID == TSPH_K_IPPE_update_vel_adv && sizeof(T) == 4 ? 7 : 1)
     k_ref_pair(KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no, const TsphControl* ctrl) {
   TSPH_STRICT
   __shared__ WalkLds lds;

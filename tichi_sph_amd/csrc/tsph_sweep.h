@@ -317,8 +317,10 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// The walk around cell cc[].  bounds(lo, hi) is the range of candidates of the
-// cells lo .. hi (one row run); fetch(s) is candidate s of it; take(fetched,
+// The walk around cell cc[].  bounds(lo, hi, &split) is the range of candidates
+// of the cells lo .. hi (one row run).  Where these cells' ranges do not follow
+// one another it sets split (SPLITS: it may), and the quad walks the rows from
+// there on cell by cell.  fetch(s) is candidate s of a range; take(fetched,
 // &apart) says whether it belongs to the list, and apart whether r > 0 (r = 0
 // goes to the list with a mark).  load(j) gathers what the pair terms need of
 // candidate j; term(record, j, valid, apart) adds one list slot per lane
@@ -328,31 +330,38 @@ struct Cand {
   V4<T> q;
   int j;  // negative: none
 };
-template <class T, class Bounds, class Fetch, class Take, class Load, class Term>
-__device__ __forceinline__ void walk_quad_cells(const KP<T>& k, const int* cc, WalkLds& lds,
-                                                Bounds&& bounds, Fetch&& fetch, Take&& take,
-                                                Load&& load, Term&& term) {
+// walk_quad_runs: the rows (CELLS: the cells) from run0 on; the row at which it
+// stopped for a split one, or -1 when all are done.
+template <bool CELLS, bool SPLITS, class T, class Bounds, class Fetch, class Take, class Load,
+          class Term>
+__device__ __forceinline__ int walk_quad_runs(const KP<T>& k, const int* cc, WalkLds& lds,
+                                              int run0, Bounds&& bounds, Fetch&& fetch,
+                                              Take&& take, Load&& load, Term&& term) {
   const int c = threadIdx.x & (kQuad - 1), g = threadIdx.x / kQuad;
   const unsigned below = (1u << c) - 1;
   const int R = k.R, side = 2 * R + 1, rows = k.dim == 3 ? side * side : side;
-  for (int row0 = 0; row0 < rows; row0 += kWalkRows) {
+  const int runs = CELLS ? rows * side : rows;
+  for (; run0 < runs; run0 += kWalkRows) {
     int nrun = 0;
+    bool split = false;
 #pragma unroll
     for (int q = 0; q < (kWalkRows + kQuad - 1) / kQuad; ++q) {
-      const int r = c + kQuad * q, row = row0 + r;
+      const int r = c + kQuad * q, id = run0 + r;
       int2 run = make_int2(0, 0);
-      if (r < kWalkRows && row < rows) {
+      if (r < kWalkRows && id < runs) {
+        const int row = CELLS ? id / side : id, dx = CELLS ? id - row * side - R : -R;
         const int dy = row % side - R, dz = k.dim == 3 ? row / side - R : 0;
-        const int c0 = dim_encode(k, wadd(cc[0], -R), wadd(cc[1], dy), wadd(cc[2], dz));
+        const int c0 = dim_encode(k, wadd(cc[0], dx), wadd(cc[1], dy), wadd(cc[2], dz));
         const long lo = c0 < 1 ? 1 : (long)c0;
-        long hi = (long)c0 + 2 * R;
+        long hi = CELLS ? (long)c0 : (long)c0 + 2 * R;
         if (hi > k.node_num - 1) hi = k.node_num - 1;
-        if (lo <= hi) run = bounds((int)lo, (int)hi);
+        if (lo <= hi) run = bounds((int)lo, (int)hi, &split);
       }
       const unsigned v = quad_vote(run.x < run.y);
       if (run.x < run.y) lds.run[nrun + __popc(v & below)][g] = run;
       nrun += __popc(v);
     }
+    if (SPLITS && !CELLS && quad_vote(split)) return run0;
     if (nrun == 0) continue;
     wave_lds_fence();
     int at = 0, j = lds.run[0][g].x, end = lds.run[0][g].y, cnt = 0;
@@ -412,6 +421,16 @@ __device__ __forceinline__ void walk_quad_cells(const KP<T>& k, const int* cc, W
       cnt = 0;
     }
   }
+  return -1;
+}
+template <bool SPLITS, class T, class Bounds, class Fetch, class Take, class Load, class Term>
+__device__ __forceinline__ void walk_quad_cells(const KP<T>& k, const int* cc, WalkLds& lds,
+                                                Bounds&& bounds, Fetch&& fetch, Take&& take,
+                                                Load&& load, Term&& term) {
+  const int row = walk_quad_runs<false, SPLITS>(k, cc, lds, 0, bounds, fetch, take, load, term);
+  if constexpr (SPLITS)
+    if (row >= 0)
+      walk_quad_runs<true, SPLITS>(k, cc, lds, row * (2 * k.R + 1), bounds, fetch, take, load, term);
 }
 
 // Every candidate of the cells around cc[], a quad per particle, without a
@@ -469,8 +488,8 @@ __device__ __forceinline__ void walk_quad(const KP<T>& k, const int* __restrict_
                                           WalkLds& lds, Load&& load, Term&& term) {
   int cc[3];
   node_encode(k, p.x, p.y, p.z, cc);
-  walk_quad_cells(
-      k, cc, lds, [&](int lo, int hi) { return make_int2(cstart[lo], cstart[hi + 1]); },
+  walk_quad_cells<false>(
+      k, cc, lds, [&](int lo, int hi, bool*) { return make_int2(cstart[lo], cstart[hi + 1]); },
       [&](int s) { return Cand<T>{pos[s], s}; },
       [&](const Cand<T>& d, bool* apart) {
         const T r2 = s_r2(p.x - d.q.x, p.y - d.q.y, p.z - d.q.z);
