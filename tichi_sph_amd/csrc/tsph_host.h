@@ -120,7 +120,7 @@ __host__ __device__ inline long scan_blocks(long len) { return (len + kScanTile 
 // Workspace layout used by all calls for objects of up to `cap` slots and a
 // grid of node_num cells (reference grid: node_num * 2 (cell,uid) buckets).
 struct WsLayout {
-  double* partial;     // [4 * maxblk] block partials for reductions
+  double* partial;     // [partial_doubles(cap)] block partials for reductions
   int* scan_sums;      // [scan blocks]
   int* key;            // [cap]
   int* rank;           // [cap]
@@ -134,19 +134,19 @@ struct WsLayout {
   void* a1b;           // [cap] V4: boundary part of alpha_1 (sum_b X_j grad W_ij), pass A
 };
 
+inline long partial_doubles(long cap) { return 4 * ((long)blocks_for(cap) + 8); }
+
 inline size_t ws_bytes_needed(long cap, long node_num) {
-  long maxblk = blocks_for(cap) + 8;
   long lenref = 2 * node_num + 2;
-  return seg(sizeof(double) * 4 * maxblk) + seg(sizeof(int) * (scan_blocks(lenref + 1) + 8)) +
+  return seg(sizeof(double) * partial_doubles(cap)) + seg(sizeof(int) * (scan_blocks(lenref + 1) + 8)) +
          5 * seg(sizeof(int) * cap) + seg(sizeof(int) * (lenref + 1)) +
          seg(sizeof(int) * (lenref + 2)) + 2 * seg(4 * sizeof(double) * cap) + 4096;
 }
 
 inline bool carve_ws(void* ws, size_t bytes, long cap, long node_num, WsLayout* L) {
   Carve c(ws, bytes);
-  long maxblk = blocks_for(cap) + 8;
   long lenref = 2 * node_num + 2;
-  L->partial = c.take<double>(4 * maxblk);
+  L->partial = c.take<double>(partial_doubles(cap));
   L->scan_sums = c.take<int>(scan_blocks(lenref + 1) + 8);
   L->key = c.take<int>(cap);
   L->rank = c.take<int>(cap);

@@ -6,6 +6,8 @@
 // accumulation into the existing field values.
 // These kernels are the drop-in for callers that drive the solver kernel by
 // kernel; the fused step (tsph_step.hip) is the fast path.
+#include <algorithm>
+
 #include "tsph_sweep.h"
 
 namespace tsph {
@@ -94,10 +96,112 @@ __device__ __forceinline__ T ref_norm(T x, T y, T z) {
   return s_sqrt(s_r2(x, y, z));
 }
 
+// ---------------------------------------------------------------------------
+// Candidates beyond h.  W, W' and C vanish there, so a pair's term is an exact
+// zero and leaving the pair out changes no sum, as long as what the zero is
+// multiplied with is finite: an infinity, a NaN or an overflow makes the term a
+// NaN, which the reference adds.  ref_plain_other(j) and ref_plain_own(i) hold
+// where the other's and the particle's own share of a term cannot do that:
+// magnitudes up to 1e9 and divisors from 1e-9 on, so that no product of a term
+// leaves FP32.  k_ref_plain asks it of every particle of nobj before a pair
+// kernel runs; a block of the pair kernel that meets one that is not plain, on
+// either side, takes all candidates of its walks instead of those in range.
+// ---------------------------------------------------------------------------
+constexpr int kRefNormal = 100, kRefForce = 101;  // surface tension's two loops
+
+template <class T>
+__device__ __forceinline__ bool small(T v) {
+  return fabs(v) <= T(1e9);
+}
+template <class T>
+__device__ __forceinline__ bool small(const V4<T>& v) {
+  return small(v.x) && small(v.y) && small(v.z);
+}
+template <class T>
+__device__ __forceinline__ bool divides(T v) {
+  return fabs(v) >= T(1e-9);
+}
+
+template <int KID, class T>
+__device__ __forceinline__ bool ref_plain_other(const KP<T>& k, const RefObj<T>& no, int j) {
+  bool ok = small(no.pos[j]);
+  if constexpr (KID == TSPH_K_SPH_prepare_attr)
+    ok = ok && small(no.rest_volume[j]) && small(no.mass[j]);
+  if constexpr (KID == TSPH_K_SPH_prepare_alpha_1) ok = ok && small(Xof(k, no, j));
+  if constexpr (KID == TSPH_K_SPH_prepare_alpha_2)
+    ok = ok && small(Xof(k, no, j)) && divides(no.mass[j]);
+  if constexpr (KID == TSPH_K_SPH_advection_viscosity_acc)
+    ok = ok && small(no.vel[j]) && small(Xof(k, no, j) / psiof(k, no, j));
+  if constexpr (KID == TSPH_K_WC_pressure_acce)
+    ok = ok && small(no.mass[j]) && small(no.pressure[j] / (no.dens[j] * no.dens[j]));
+  if constexpr (KID == TSPH_K_IPPE_adv_psi)
+    ok = ok && small(no.vel_adv[j]) && small(Xof(k, no, j));
+  if constexpr (KID == TSPH_K_IPPE_update_vel_adv)
+    ok = ok && small(Xof(k, no, j)) && small(no.psi_adv[j]) && divides(no.alpha[j]);
+  if constexpr (KID == kRefNormal) ok = ok && small(Xof(k, no, j) / psiof(k, no, j));
+  if constexpr (KID == kRefForce)
+    ok = ok && small(no.mass[j]) && small(no.normal[j]) && psiof(k, no, j) >= T(1e-9);
+  if constexpr (KID == TSPH_K_SPH_FBM_diffuse || KID == TSPH_K_SPH_FBM_convect) {
+    ok = ok && small(no.rest_volume[j]);
+    for (int q = 0; q < k.P; ++q) {
+      ok = ok && small(no.vf[(long)j * k.P + q]);
+      if constexpr (KID == TSPH_K_SPH_FBM_convect) ok = ok && small(no.drift[(long)j * k.P + q]);
+    }
+  }
+  return ok;
+}
+
+template <int KID, class T>
+__device__ __forceinline__ bool ref_plain_own(const KP<T>& k, const RefObj<T>& o, int i, T dt) {
+  bool ok = small(o.pos[i]) && small(dt);
+  if constexpr (KID == TSPH_K_SPH_advection_viscosity_acc)
+    ok = ok && small(o.vel[i]) && divides(o.rest_density[i]) && small(mu_of(k, o.vf, i));
+  if constexpr (KID == TSPH_K_WC_pressure_acce)
+    ok = ok && small(o.pressure[i] / (o.dens[i] * o.dens[i]));
+  if constexpr (KID == TSPH_K_IPPE_adv_psi) ok = ok && small(o.vel_adv[i]);
+  if constexpr (KID == TSPH_K_IPPE_update_vel_adv)
+    ok = ok && small(Xof(k, o, i)) && small(o.psi_adv[i]) && divides(o.alpha[i]) &&
+         divides(o.mass[i]) && divides(dt);
+  if constexpr (KID == kRefForce)
+    ok = ok && small(o.normal[i]) && small(rpsiof(k, o, i)) && psiof(k, o, i) >= T(1e-9);
+  if constexpr (KID == TSPH_K_SPH_FBM_diffuse || KID == TSPH_K_SPH_FBM_convect) {
+    ok = ok && small(KID == TSPH_K_SPH_FBM_diffuse ? dt * k.fbmD : k.fbmC * dt);
+    for (int q = 0; q < k.P; ++q) {
+      ok = ok && small(o.vf[(long)i * k.P + q]);
+      if constexpr (KID == TSPH_K_SPH_FBM_convect) ok = ok && small(o.drift[(long)i * k.P + q]);
+    }
+  }
+  return ok;
+}
+
+// flags[block]: a particle of the block's share is not plain.  At most kBlock
+// blocks, as a pair kernel's block reads one flag per thread: 4.6-5.1 us a call at
+// 100k particles.
+constexpr int kPlainThreads = 1024;
+inline int plain_blocks(int n, long room) {
+  const long want = ((long)n + kPlainThreads - 1) / kPlainThreads;
+  return (int)std::min({want, (long)kBlock, room});
+}
+template <class T, int KID>
+__global__ void __launch_bounds__(kPlainThreads) k_ref_plain(KP<T> k, RefObj<T> no, int* flags) {
+  bool ok = true;
+  for (int j = blockIdx.x * kPlainThreads + threadIdx.x; j < no.n; j += gridDim.x * kPlainThreads)
+    ok = ok && ref_plain_other<KID>(k, no, j);
+  const int odd = __syncthreads_or(!ok);
+  if (threadIdx.x == 0) flags[blockIdx.x] = odd;
+}
+// Whether this block has to take all candidates (every thread of the block asks).
+template <int KID, class T>
+__device__ __forceinline__ bool ref_take_all(const KP<T>& k, const RefObj<T>& o, int i, T dt,
+                                             const int* flags, int nflag) {
+  const bool other = (int)threadIdx.x < nflag && flags[threadIdx.x] != 0;
+  return __syncthreads_or(other || (i < o.n && !ref_plain_own<KID>(k, o, i, dt))) != 0;
+}
+
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_ref(int kid, KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no, double* partial,
-          TsphControl* ctrl) {
+          TsphControl* ctrl, const int* flags, int nflag) {
   TSPH_STRICT
   __shared__ double lds[kWaves];
   const int nblk = gridDim.x;
@@ -212,7 +316,8 @@ __global__ void __launch_bounds__(kBlock)
       if (act)
         for (int q = 0; q < P; ++q) o.vf_tmp[(long)i * P + q] = T(0);
       return;
-    case TSPH_K_SPH_FBM_diffuse:  // sph.py:308-326
+    case TSPH_K_SPH_FBM_diffuse: {  // sph.py:308-326
+      const bool all = ref_take_all<TSPH_K_SPH_FBM_diffuse>(k, o, i, dt, flags, nflag);
       if (act && o.flag[i] == 0) {
         V4<T> p = o.pos[i];
         T acc[kMaxP];
@@ -220,7 +325,7 @@ __global__ void __launch_bounds__(kBlock)
         T pre = dt * k.fbmD;
         ref_walk(k, g, cs, no.uid, [&](int j) {
           V4<T> q = no.pos[j];
-          if (!(s_r2(p.x - q.x, p.y - q.y, p.z - q.z) <= k.r2max)) return;  // exact zeros
+          if (!all && !(s_r2(p.x - q.x, p.y - q.y, p.z - q.z) <= k.r2max)) return;
           if (no.flag[j] != 0) return;
           T r = ref_norm(p.x - q.x, p.y - q.y, p.z - q.z);
           if (r > T(0)) {
@@ -235,6 +340,7 @@ __global__ void __launch_bounds__(kBlock)
         for (int q = 0; q < P; ++q) o.vf_tmp[(long)i * P + q] = acc[q];
       }
       return;
+    }
     case TSPH_K_SPH_FBM_check_tmp:  // sph.py:366-372
       if (act) {
         bool neg = false;
@@ -268,25 +374,23 @@ __global__ void __launch_bounds__(kBlock)
 // The pair kernels, one instance per kernel id, a quad of lanes per particle
 // (tsph_sweep.h: walk_quad_cells): the quad tests the candidates of the Ngrid
 // four at a time and works off those in range, and every sum takes its terms
-// in the reference's order.  Beyond h the reference's terms are exact zeros
-// (W, W' and C vanish), so leaving them out changes no value.  One kernel with
+// in the reference's order.  One kernel with
 // a switch over all ids, one lane per particle and the whole pair math on each
 // of the 200 or so candidates took 130-170 us per call at 100k particles; these
-// take 37-69 us there, bound by the dependent loads of the walk (entry, then
+// take 39-72 us there, bound by the dependent loads of the walk (entry, then
 // position).  A whole reference step at 4k / 100k / 1M: 3.5 / 4.0 / 15.5 ms,
-// now 0.94 / 1.47 / 8.7.
+// now 1.09 / 1.65 / 9.5 (0.96 / 1.46 / 8.7 without k_ref_plain's calls and the row
+// check below).
 // ---------------------------------------------------------------------------
-constexpr int kRefNormal = 100, kRefForce = 101;  // surface tension's two loops
-
-// The walk around cell cs[] of particle p over nuid's candidates in range, or
-// (ALL) all of them with r > 0.  A row of cells is one range where the Ngrid
+// The walk around cell cs[] of particle p over nuid's candidates up to r2lim
+// (those at a NaN distance among them).  A row of cells is one range where the Ngrid
 // holds them one after the other, as tsph_ngrid_build does; where it does not
 // (the reference's mem_shift, sph_obj.py:308-314, hands the ranges out in
 // whatever order its threads reach the cells) every cell is read by itself.
-// Asking whether it does costs 1-2 us of a call's 37-69 at 100k particles.
-template <bool ALL, class T, class Load, class Term>
+// Asking whether it does costs 1-2 us of a call's 39-72 at 100k particles.
+template <class T, class Load, class Term>
 __device__ __forceinline__ void ref_quad(const KP<T>& k, const RefGrid& g, const int* cs, int nuid,
-                                         const V4<T>* __restrict__ npos, const V4<T>& p,
+                                         const V4<T>* __restrict__ npos, const V4<T>& p, T r2lim,
                                          WalkLds& lds, Load&& load, Term&& term) {
   walk_quad_cells<true>(
       k, cs, lds,
@@ -319,7 +423,7 @@ __device__ __forceinline__ void ref_quad(const KP<T>& k, const RefGrid& g, const
       [&](const Cand<T>& d, bool* apart) {
         const T r2 = s_r2(p.x - d.q.x, p.y - d.q.y, p.z - d.q.z);
         *apart = r2 > T(0);  // as r > 0: the square root of a positive value is positive
-        return ALL ? *apart : r2 <= k.r2max;
+        return !(r2 > r2lim);
       },
       load, term);
 }
@@ -330,30 +434,42 @@ struct RefRec {
   T a, b, c;
 };
 
-// The FP32 update keeps 7 waves per SIMD (a spill at its entry, for the address
-// of its result, instead of 76 registers): 54 us a call at 100k with 6, 47 with 7.
+// These two keep 7 waves per SIMD in FP32 (the update by a spill at its entry, for
+// the address of its result, instead of 76 registers): 54 us a call of the update
+// at 100k with 6, 47 with 7.
+template <class T>
+constexpr int ref_waves(int kid) {
+  return sizeof(T) == 4 && (kid == TSPH_K_IPPE_update_vel_adv || kid == TSPH_K_SPH_prepare_attr) ? 7 : 1;
+}
 template <class T, int KID>
-__global__ void __launch_bounds__(kBlock, KID == TSPH_K_IPPE_update_vel_adv && sizeof(T) == 4 ? 7 : 1)
-    k_ref_pair(KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no, const TsphControl* ctrl) {
+__global__ void __launch_bounds__(kBlock, ref_waves<T>(KID))
+    k_ref_pair(KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no, const TsphControl* ctrl,
+               const int* flags, int nflag) {
   TSPH_STRICT
   __shared__ WalkLds lds;
   const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const T dt = (T)ctrl->dt;
+  bool all = ref_take_all<KID>(k, o, i, dt, flags, nflag);
+  if constexpr (KID == kRefForce) {
+    if (!all && k.gamma == T(0)) return;  // every term is an exact zero
+    all = true;                           // else (n_i - n_j) counts at any distance
+  }
+  const T r2lim = all ? T(INFINITY) : k.r2max;
   if (i >= o.n) return;
   const bool lead = coop_lane<kQuad>() == 0;
-  const T dt = (T)ctrl->dt;
   const bool d3 = k.dim == 3;
   const int* cs = o.cs + 4 * i;
   const V4<T> p = o.pos[i];
   // add(load, pair): pair(record, dx, dy, dz, r, on) with on = the lane holds
   // a candidate (r > 0, except for W(0) in prepare_attr)
   auto add = [&](auto&& load, auto&& pair) {
-    ref_quad<KID == kRefForce>(k, g, cs, no.uid, no.pos, p, lds, load,
-                               [&](const RefRec<T>& d, int, bool valid, bool apart) {
-                                 TSPH_STRICT
-                                 const T dx = p.x - d.q.x, dy = p.y - d.q.y, dz = p.z - d.q.z;
-                                 pair(d, dx, dy, dz, ref_norm(dx, dy, dz),
-                                      valid && (apart || KID == TSPH_K_SPH_prepare_attr));
-                               });
+    ref_quad(k, g, cs, no.uid, no.pos, p, r2lim, lds, load,
+             [&](const RefRec<T>& d, int, bool valid, bool apart) {
+               TSPH_STRICT
+               const T dx = p.x - d.q.x, dy = p.y - d.q.y, dz = p.z - d.q.z;
+               pair(d, dx, dy, dz, ref_norm(dx, dy, dz),
+                    valid && (apart || KID == TSPH_K_SPH_prepare_attr));
+             });
   };
   // acc + the quad's terms, component by component
   auto add3 = [&](V4<T>& acc, T x, T y, T z, bool on) {
@@ -487,11 +603,13 @@ __global__ void __launch_bounds__(kBlock, KID == TSPH_K_IPPE_update_vel_adv && s
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_ref_convect(int pass, KP<T> k, RefGrid g, RefObj<T> o, RefObj<T> no,
-                  const TsphControl* ctrl) {
+                  const TsphControl* ctrl, const int* flags, int nflag) {
   TSPH_STRICT
   int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= o.n) return;
   const T dt = (T)ctrl->dt;
+  const bool all =
+      pass == 1 && ref_take_all<TSPH_K_SPH_FBM_convect>(k, o, i, dt, flags, nflag);
+  if (i >= o.n) return;
   const int P = k.P;
   if (pass == 0) {
     V4<T> va = o.vel_adv[i], v = o.vel[i];
@@ -531,7 +649,7 @@ __global__ void __launch_bounds__(kBlock)
   ref_walk(k, g, cs, no.uid, [&](int j) {
     V4<T> q = no.pos[j];
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    if (!(s_r2(dx, dy, dz) <= k.r2max)) return;  // exact zeros
+    if (!all && !(s_r2(dx, dy, dz) <= k.r2max)) return;
     if (no.flag[j] != 0) return;
     T r = ref_norm(dx, dy, dz);
     if (r > T(0)) {
@@ -563,34 +681,49 @@ int ref_kernel(const TsphParams& prm, int kid, TsphObject* obj, const TsphObject
   RefObj<T> o = ref_obj<T>(obj);
   RefObj<T> no = ref_obj<T>(nobj ? nobj : obj);
   int nb = blocks_for(obj->n > 0 ? obj->n : 1);
-  auto pair = [&](auto kern) {
-    if (o.n > 0)
-      hipLaunchKernelGGL(kern, dim3(coop_blocks<kQuad>(o.n)), dim3(kBlock), 0, st, k, g, o, no,
-                         ctrl);
+  int* flags = (int*)L.partial;  // unused by the pair kernels otherwise
+  const int nflag = plain_blocks(no.n, partial_doubles(obj->capacity) * 2);
+  auto plain = [&](auto kern) {
+    if (nflag > 0)
+      hipLaunchKernelGGL(kern, dim3(nflag), dim3(kPlainThreads), 0, st, k, no, flags);
+  };
+  auto pair = [&](auto ask, auto kern) {
+    if (o.n <= 0) return;
+    plain(ask);
+    hipLaunchKernelGGL(kern, dim3(coop_blocks<kQuad>(o.n)), dim3(kBlock), 0, st, k, g, o, no, ctrl,
+                       flags, nflag);
   };
   if (kid == TSPH_K_SPH_prepare_attr) {
-    pair(k_ref_pair<T, TSPH_K_SPH_prepare_attr>);
+    pair(k_ref_plain<T, TSPH_K_SPH_prepare_attr>, k_ref_pair<T, TSPH_K_SPH_prepare_attr>);
   } else if (kid == TSPH_K_SPH_prepare_alpha_1) {
-    pair(k_ref_pair<T, TSPH_K_SPH_prepare_alpha_1>);
+    pair(k_ref_plain<T, TSPH_K_SPH_prepare_alpha_1>, k_ref_pair<T, TSPH_K_SPH_prepare_alpha_1>);
   } else if (kid == TSPH_K_SPH_prepare_alpha_2) {
-    pair(k_ref_pair<T, TSPH_K_SPH_prepare_alpha_2>);
+    pair(k_ref_plain<T, TSPH_K_SPH_prepare_alpha_2>, k_ref_pair<T, TSPH_K_SPH_prepare_alpha_2>);
   } else if (kid == TSPH_K_SPH_advection_viscosity_acc) {
-    pair(k_ref_pair<T, TSPH_K_SPH_advection_viscosity_acc>);
+    pair(k_ref_plain<T, TSPH_K_SPH_advection_viscosity_acc>, k_ref_pair<T, TSPH_K_SPH_advection_viscosity_acc>);
   } else if (kid == TSPH_K_WC_pressure_acce) {
-    pair(k_ref_pair<T, TSPH_K_WC_pressure_acce>);
+    pair(k_ref_plain<T, TSPH_K_WC_pressure_acce>, k_ref_pair<T, TSPH_K_WC_pressure_acce>);
   } else if (kid == TSPH_K_IPPE_adv_psi) {
-    pair(k_ref_pair<T, TSPH_K_IPPE_adv_psi>);
+    pair(k_ref_plain<T, TSPH_K_IPPE_adv_psi>, k_ref_pair<T, TSPH_K_IPPE_adv_psi>);
   } else if (kid == TSPH_K_IPPE_update_vel_adv) {
-    pair(k_ref_pair<T, TSPH_K_IPPE_update_vel_adv>);
+    pair(k_ref_plain<T, TSPH_K_IPPE_update_vel_adv>, k_ref_pair<T, TSPH_K_IPPE_update_vel_adv>);
   } else if (kid == TSPH_K_SPH_advection_surface_tension_acc) {
-    pair(k_ref_pair<T, kRefNormal>);
-    if (k.gamma != T(0)) pair(k_ref_pair<T, kRefForce>);  // else every term is an exact zero
+    pair(k_ref_plain<T, kRefNormal>, k_ref_pair<T, kRefNormal>);
+    if (k.gamma == T(0))  // whether any term can be other than zero
+      pair(k_ref_plain<T, kRefForce>, k_ref_pair<T, kRefForce>);
+    else if (o.n > 0)
+      hipLaunchKernelGGL((k_ref_pair<T, kRefForce>), dim3(coop_blocks<kQuad>(o.n)), dim3(kBlock), 0,
+                         st, k, g, o, no, ctrl, flags, 0);
   } else if (kid == TSPH_K_SPH_FBM_convect) {
-    hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 0, k, g, o, no, ctrl);
-    hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 1, k, g, o, no, ctrl);
+    hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 0, k, g, o, no, ctrl,
+                       flags, 0);
+    plain(k_ref_plain<T, TSPH_K_SPH_FBM_convect>);  // the drifts are there now
+    hipLaunchKernelGGL(k_ref_convect<T>, dim3(nb), dim3(kBlock), 0, st, 1, k, g, o, no, ctrl,
+                       flags, nflag);
   } else {
-    hipLaunchKernelGGL(k_ref<T>, dim3(nb), dim3(kBlock), 0, st, kid, k, g, o, no, L.partial,
-                       ctrl);
+    if (kid == TSPH_K_SPH_FBM_diffuse) plain(k_ref_plain<T, TSPH_K_SPH_FBM_diffuse>);
+    hipLaunchKernelGGL(k_ref<T>, dim3(nb), dim3(kBlock), 0, st, kid, k, g, o, no, L.partial, ctrl,
+                       flags, nflag);
     int mode = kid == TSPH_K_cfl_condition ? kFinCfl
                : kid == TSPH_K_SPH_update_energy ? kFinEnergy
                : kid == TSPH_K_SPH_FBM_check_tmp ? kFinFlag
