@@ -389,6 +389,7 @@ __global__ void __launch_bounds__(kBlock)
 // records of two gathers each in flight per lane.  At 200k particles, one lane
 // with 4 in flight 90 us; quads with 1 / 2 / 3 / 4 / 6 in flight 75 / 72 / 74 /
 // 92 (with a branch per candidate) / 79 us.
+// (Terms that are left out are dropped by selects: 74 us with 2 in flight.)
 constexpr int kStRevU = 2;
 template <class T>
 __global__ void __launch_bounds__(kBlock)
@@ -434,18 +435,20 @@ __global__ void __launch_bounds__(kBlock)
         }
         const V4<T>& nj = d.a;
         const V4<T>& bj = d.b;
-        const T rden = on ? f_rcp(rhoi + nj.w) : T(0);  // a factor of every term
+        const T rden = f_rcp(rhoi + nj.w);
         const T fij = T(2) * r0i * rden, r2d = T(2) * rden;
         const T dnx = ni.x - nj.x, dny = ni.y - nj.y, dnz = ni.z - nj.z;
         // e_lj = f_lj a_l - f_jl a_j
         const T ex = fij * ali_x - r2d * bj.x;
         const T ey = fij * ali_y - r2d * bj.y;
         const T ez = fij * ali_z - r2d * bj.z;
-        gs += fij * (ali_x * dnx + ali_y * dny + ali_z * dnz);
-        nbx += gam * ex;
-        nby += gam * ey;
-        nbz += gam * ez;
-        rb += -gam * rden * (dnx * ex + dny * ey + dnz * ez);
+        // (a candidate left out may hold anything: its terms are dropped, not
+        // multiplied by zero)
+        gs += on ? fij * (ali_x * dnx + ali_y * dny + ali_z * dnz) : T(0);
+        nbx += on ? gam * ex : T(0);
+        nby += on ? gam * ey : T(0);
+        nbz += on ? gam * ez : T(0);
+        rb += on ? -gam * rden * (dnx * ex + dny * ey + dnz * ez) : T(0);
       });
       // cohesion, per in-range neighbour: (x_j, X_j = m_j) as well
       auto loadc = [&](int j) { return Rec3<T>{fpos[j], tnormal[j], brec[j]}; };

@@ -882,6 +882,8 @@ __global__ void __launch_bounds__(kBlock)
 // holds about 24 candidates, one trip of six.  us, one lane with 8 in flight /
 // quads with 2, 3, 4, 6, 7, 8: 4k 29 / 14.3, 12.4, 13.4, 11.8, 12.5, 12.3; 200k
 // 50 / 52, 50, 57, 46, 49, 54; 2M 246 / 259, 244, 276, 229, 245, 266.
+// (Dropping the terms of a candidate that is left out, instead of multiplying
+// them by zero, costs 1 us at 200k and 8 at 2M.)
 constexpr int kStFwdU = 6;
 template <class T, int R = 1>
 __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, int n, int cap,
@@ -921,10 +923,13 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
       T ux = 0, uy = 0, uz = 0;  // sum of (n_i - n_j) / (psi_i + psi_j)
       walk_quad_all<kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
                              [&](int j, const V4<T>& nj, bool valid) {
-        const T w = valid && j != i && nj.w > T(0) ? f_rcp(psi_i + nj.w) : T(0);
-        ux += w * (ni.x - nj.x);
-        uy += w * (ni.y - nj.y);
-        uz += w * (ni.z - nj.z);
+        // a candidate left out may hold anything: its terms are dropped, not
+        // multiplied by zero
+        const bool on = valid && j != i && nj.w > T(0);
+        const T w = f_rcp(psi_i + nj.w);
+        ux += on ? w * (ni.x - nj.x) : T(0);
+        uy += on ? w * (ni.y - nj.y) : T(0);
+        uz += on ? w * (ni.z - nj.z) : T(0);
       });
       // per in-range neighbour: (x_j, m_j) and the normal record
       auto load = [&](int j) { return Rec2<T>{strec[j], normal[j]}; };
