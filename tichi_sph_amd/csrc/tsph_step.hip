@@ -80,7 +80,8 @@ struct PassAAcc {
     T g = qh <= T(0.5) ? k.wg_a * (T(3) * qh - T(2)) : -k.wg_b * (u * u) * f_rcp(r);
     const T Xj = q.w;
     const T xg = valid && apart ? Xj * g : T(0);
-    const T x2m = XM ? Xj : (Xj * Xj) * f_rcp(mj);
+    // both factors: a massless or infinite particle at r = 0 has no term
+    const T x2m = !(valid && apart) ? T(0) : XM ? Xj : (Xj * Xj) * f_rcp(mj);
     const T t2 = valid && apart ? (g * g) * r2 : T(0);
     add_lane<0>(xg, dx, dy, dz, t2, x2m, fluid);
     add_lane<1>(xg, dx, dy, dz, t2, x2m, fluid);
