@@ -690,8 +690,11 @@ int copy_many(const TsphCopy* c, int count, hipStream_t st) {
     if (c[q].bytes == 0) continue;
     l.c[m] = c[q];
     l.first[m++] = (int)blocks;
-    blocks += (long)((c[q].bytes + kCopyChunk - 1) / kCopyChunk);
-    TSPH_REQUIRE(blocks < (1L << 30), TSPH_EINVAL, "tsph_copy_many: too many bytes");
+    // a launch holds fewer than 2^32 threads
+    constexpr long kMaxBlocks = (1L << 32) / kBlock;
+    const bool fits = c[q].bytes < (uint64_t)kMaxBlocks * kCopyChunk;
+    if (fits) blocks += (long)((c[q].bytes + kCopyChunk - 1) / kCopyChunk);
+    TSPH_REQUIRE(fits && blocks < kMaxBlocks, TSPH_EINVAL, "tsph_copy_many: too many bytes");
   }
   if (m == 0) return 0;
   for (int q = m; q < TSPH_COPY_MAX; ++q) l.first[q] = 0x7fffffff;
