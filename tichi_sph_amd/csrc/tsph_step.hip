@@ -459,10 +459,25 @@ __device__ __forceinline__ void pass_a_quad_bound(int sub, const KP<T>& k, const
 // us per launch, one lane / quads: 3D FP32 8k 71 / 30, 64k 72 / 39, 133k 78 /
 // 67, 149k 80 / 73, 195k 82 / 85, 1M 238 / 368; FP64 8k 87 / 32, 64k 91 / 66,
 // 97k 105 / 89, 195k 130 / 156; 2D FP32 8k 24 / 17, 78k 24.8 / 23.1, 102k
-// 25.5 / 26.
+// 25.5 / 26, FP64 70k 26.8 / 25.6.
+// A boundary particle counts by a half: its walk over its own object, which the
+// sums kept from an earlier step replace (then by a sixteenth).  Fluid + boundary,
+// us, one lane / quads, sums formed and kept: 3D FP32 8k + 213k 72 / 53 and 67 /
+// 25, 8k + 283k 72 / 67, 64k + 166k 69 / 70 and 66 / 41, 64k + 283k 71 / 88 and
+// 68 / 46, 97k + 94k 69 / 66 and 69 / 51, 97k + 596k 105 / 157 and 72 / 69, 125k +
+// 283k 87 / 110 and 71 / 68; FP64 8k + 124k 83 / 64 and 84 / 28, 64k + 94k 87 / 96
+// and 86 / 67, 64k + 387k 127 / 197 and 91 / 89, 64k + 596k 167 / 268 and 92 / 104.
+// 2D FP32 8k + 134k 21.3 / 21.8 and 16.1 / 10.2, 40k + 134k 22.5 / 26.1 and 17.9 /
+// 14.4.  In 2D with FP64 the single lanes' short chain counts least: 8k + 42k
+// 20.9 / 17.2 and 18.7 / 12.0, 8k + 86k 23.6 / 26.9, 40k + 42k 26.0 / 28.6 and 21.0 /
+// 19.0, 40k + 86k 25.9 / 36.7 and 21.5 / 21.0, 40k + 134k 29 / 48 and 22.4 / 24.4.
 template <class T>
-static constexpr int pass_a_quad_max(int dim) {
-  return dim == 2 ? 80 * 1024 : sizeof(T) == 4 ? 144 * 1024 : 96 * 1024;
+static bool pass_a_by_quads(int dim, const TsphObject& f, const TsphObject& b) {
+  const bool kept = b.static_sums != nullptr && (b.flags & TSPH_OBJ_STATIC_SUMS);
+  const bool flat64 = dim == 2 && sizeof(T) == 8;
+  const long most = flat64 ? 70 * 1024 : dim == 2 ? 80 * 1024 : sizeof(T) == 4 ? 144 * 1024 : 96 * 1024;
+  const int share = kept ? (flat64 ? 4 : 16) : (flat64 ? 1 : 2);
+  return f.n > 0 && f.n + (long)b.n / share <= most;
 }
 template <class T>
 __global__ void __launch_bounds__(kBlock)
@@ -1295,8 +1310,7 @@ static int pass_a(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphContr
                   bool with_bound, const WsLayout& L, bool opened, hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   if (!opened) hipLaunchKernelGGL(k_step_reset, dim3(1), dim3(64), 0, st, ctrl);
-  if (with_bound && f->n > 0 && f->n <= pass_a_quad_max<T>(prm.dim) &&
-      b->n <= 2 * pass_a_quad_max<T>(prm.dim)) {
+  if (with_bound && pass_a_by_quads<T>(prm.dim, *f, *b)) {
     const int nbf = coop_blocks<kQuad>(f->n);
     hipLaunchKernelGGL(k_pass_a_quad<T>, dim3(nbf + (b->n > 0 ? coop_blocks<kQuad>(b->n) : 0)),
                        dim3(kBlock), 0, st, k, *f, *b, nbf, (V4<T>*)L.a1b, ctrl);
