@@ -901,7 +901,18 @@ __global__ void __launch_bounds__(kBlock)
 // (Dropping the terms of a candidate that is left out, instead of multiplying
 // them by zero, costs 1 us at 200k and 8 at 2M.)
 constexpr int kStFwdU = 6;
-template <class T, int R = 1>
+// In 2D there are three rows of half that, and large scenes take one lane per
+// particle (also with six in flight; eight of the walk and the list raise the
+// grouped kernels' registers), us, one lane / quads: FP32 9k 10.5 / 7.1, 65k 11.5 /
+// 10.4, 90k 12.3 / 13.7, 130k 12.9 / 18.2, 300k 21.6 / 32.0, 1M 54.7 / 91; FP64 9k
+// 16.4 / 8.6, 65k 17.7 / 16.1, 90k 20 / 23.2, 300k 40.0 / 60.4, 1M 120 / 202.  The
+// rule is a scene's own, also in a grouped launch, so that both sum in one order.
+__host__ __device__ __forceinline__ bool st_one_lane(int dim, int n) {
+  return dim == 2 && n > 72 * 1024;
+}
+// L lanes per particle; with one, the R sub-tiles' particles are the block's
+// first R * kBlock / kQuad threads.
+template <class T, int L, int R>
 __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, int n, int cap,
                       const V4<T>* __restrict__ fpos, const T* __restrict__ psi_rho,
                       const T* __restrict__ rdens, const T* __restrict__ vf,
@@ -910,19 +921,21 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
                       const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
                       V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
                       const TsphControl* ctrl) {
-  const int cl = coop_lane<kQuad>();
+  const int cl = coop_lane<L>();
   const T dt = (T)ctrl->dt;
+  const int own = coop_sub<R>(blk) * (kBlock / kQuad) + (int)threadIdx.x;
+  const bool has = (int)threadIdx.x < R * (kBlock / kQuad) && own < n;
   if (k.gamma == T(0)) {  // a scene without it in a grouped launch: the update alone
     TSPH_STRICT
-    const int i = coop_sub<R>(blk) * (kBlock / kQuad) + (int)threadIdx.x;
-    if ((int)threadIdx.x >= R * (kBlock / kQuad) || i >= n) return;
-    const V4<T> v = vel[i], a = acce_adv[i];
-    vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
+    if (!has) return;
+    const V4<T> v = vel[own], a = acce_adv[own];
+    vadv[own] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
     return;
   }
+  if (L == 1 && !has) return;
 #pragma unroll 1
-  for (int r = 0; r < R; ++r) {
-    const int i = coop_particle<kQuad>(coop_sub<R>(blk, r));
+  for (int r = 0; r < (L == 1 ? 1 : R); ++r) {
+    const int i = L == 1 ? own : coop_particle<kQuad>(coop_sub<R>(blk, r));
     if (i >= n) break;
     V4<T> a = acce_adv[i];
     if (vf[(long)i * k.P] > T(0.99)) {
@@ -937,8 +950,8 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
       // and reciprocals instead of the IEEE forms: the pair terms of these
       // sums are not part of the bit-exact sums.
       T ux = 0, uy = 0, uz = 0;  // sum of (n_i - n_j) / (psi_i + psi_j)
-      walk_quad_all<kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
-                             [&](int j, const V4<T>& nj, bool valid) {
+      walk_all<L, kStFwdU, kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
+                              [&](int j, const V4<T>& nj, bool valid) {
         // a candidate left out may hold anything: its terms are dropped, not
         // multiplied by zero
         const bool on = valid && j != i && nj.w > T(0);
@@ -960,12 +973,12 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
         uy -= s * dy;
         uz -= s * dz;
       };
-      sweep_lists_coop<kQuad, T, Rec2<T>>(
+      sweep_lists_coop<L, T, Rec2<T>>(
           k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, load,
           load, coh, [&](const Rec2<T>&, bool) {});
-      ux = group_sum<kQuad>(ux);
-      uy = group_sum<kQuad>(uy);
-      uz = group_sum<kQuad>(uz);
+      ux = group_sum<L>(ux);
+      uy = group_sum<L>(uy);
+      uz = group_sum<L>(uz);
       // 2 psi_0 / (psi_i + psi_j) (cohesion + curvature), cohesion =
       // -gamma m_j C(r) x_ij / r, curvature = gamma (n_i - n_j)
       const T f = T(2) * rp * k.gamma;
@@ -1001,7 +1014,7 @@ __global__ void __launch_bounds__(kBlock)
   vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
 }
 
-template <class T>
+template <class T, int L>
 __global__ void __launch_bounds__(kBlock)
     k_surface_tension(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                       const T* __restrict__ psi_rho,
@@ -1013,7 +1026,7 @@ __global__ void __launch_bounds__(kBlock)
                       TsphControl* ctrl, SolveOpen open) {
   if (open.ahead && !ctrl->go) return;
   if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
-  k_surface_tension_body<T>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
+  k_surface_tension_body<T, L, L == 1 ? kQuad : 1>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1474,12 +1487,19 @@ int advect(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphControl* ctr
     hipLaunchKernelGGL(k_vel_adv_update<T>, dim3(nb), dim3(kBlock), 0, st, k, f->n,
                        (const V4<T>*)f->vel, (const V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl,
                        open);
-  else
-    hipLaunchKernelGGL(k_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
-                       f->capacity, (const V4<T>*)f->pos, psi, (const T*)f->rest_density,
-                       (const T*)f->volume_frac, f->cell_start, (const V4<T>*)f->normal,
-                       (const V4<T>*)L.krec, f->nbr_f, f->nbr_nf, (const V4<T>*)f->vel,
-                       (V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl, open);
+  else {
+    auto tension = [&](auto kern, int blocks) {
+      hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                         (const V4<T>*)f->pos, psi, (const T*)f->rest_density,
+                         (const T*)f->volume_frac, f->cell_start, (const V4<T>*)f->normal,
+                         (const V4<T>*)L.krec, f->nbr_f, f->nbr_nf, (const V4<T>*)f->vel,
+                         (V4<T>*)f->acce_adv, (V4<T>*)f->vel_adv, ctrl, open);
+    };
+    if (st_one_lane(prm.dim, f->n))
+      tension(k_surface_tension<T, 1>, nb);
+    else
+      tension(k_surface_tension<T, kQuad>, coop_blocks<kQuad>(f->n));
+  }
   TSPH_LAUNCH_CHECK("advect");
   return 0;
 }
@@ -1810,10 +1830,14 @@ template <class T, int R>
 __global__ void __launch_bounds__(kBlock) kb_surface_tension(const char* __restrict__ tab, int ns) {
   for_coop_tiles<T, kQuad, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_surface_tension_body<T, R>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e),
-                              (const T*)f.rest_density, (const T*)f.volume_frac, f.cell_start,
-                              (const V4<T>*)f.normal, (const V4<T>*)e.L.krec, f.nbr_f, f.nbr_nf,
-                              (const V4<T>*)f.vel, (V4<T>*)f.acce_adv, (V4<T>*)f.vel_adv, e.ctrl);
+    auto scene = [&](auto lanes) {
+      k_surface_tension_body<T, decltype(lanes)::value, R>(
+          blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e), (const T*)f.rest_density,
+          (const T*)f.volume_frac, f.cell_start, (const V4<T>*)f.normal, (const V4<T>*)e.L.krec,
+          f.nbr_f, f.nbr_nf, (const V4<T>*)f.vel, (V4<T>*)f.acce_adv, (V4<T>*)f.vel_adv, e.ctrl);
+    };
+    if (st_one_lane(e.k.dim, f.n)) scene(std::integral_constant<int, 1>{});
+    else scene(std::integral_constant<int, kQuad>{});
   });
 }
 

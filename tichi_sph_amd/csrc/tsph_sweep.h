@@ -480,6 +480,17 @@ __device__ __forceinline__ void walk_quad_all(const KP<T>& k, const int* __restr
   }
 }
 
+// The same by L lanes per particle: a quad, or one lane with U1 gathers in flight.
+template <int L, int U4, int U1, class T, class Load, class F>
+__device__ __forceinline__ void walk_all(const KP<T>& k, const int* __restrict__ cstart,
+                                         const int* cc, Load&& load, F&& f) {
+  static_assert(L == kQuad || L == 1, "a quad or one lane");
+  if constexpr (L == kQuad)
+    walk_quad_all<U4>(k, cstart, cc, load, f);
+  else
+    walk_cells_prefetch<U1>(k, cstart, cc, load, [&](int j, const auto& d) { f(j, d, true); });
+}
+
 // The walk of an object in cell order around p, taking the candidates in range
 // (r^2 <= r2max).
 template <class T, class Load, class Term>
