@@ -101,13 +101,20 @@ constexpr int kBsumU = 4;  // boundary candidates in flight per lane
 // two / four lanes, the kappa half: FP32 14k 6.6 / 5.0, 98k 12.4 / 11.5, 200k
 // (compressed) 19.6 / 18.6, 405k 36.0 / 36.0, 593k 49.0 / 50.5, 1M 83.7 / 87.4;
 // FP64 14k 9.7 / 6.8, 98k 20.8 / 21.8.  The FP32 viscosity gathers four records
-// a pair and takes four lanes at every size: 14k 10.9 / 7.5, 216k 30.1 / 30.2,
+// a pair and takes four lanes at every size in 3D: 14k 10.9 / 7.5, 216k 30.1 / 30.2,
 // 405k 53.0 / 49.0, 1M 139.9 / 124.2; FP64 14k 12.6 / 10.1, 98k 27.0 / 29.6.
+// In 2D, with some 20 neighbours to a particle, a trip of four lanes is half empty
+// at the list's end: two lanes from 96k on in FP32 (us, four / two: kappa 130k 10.5 /
+// 9.1, viscosity 130k 14.5 / 12.6, 300k 26.4 / 22.0, 1.2M 96 / 77), and in FP64 in pass
+// A's reverse too.  The surface tension's and the boundary sums' walks (rows of 12
+// candidates) then take one lane, us, quads / one: tension FP32 65k 13.0 / 18, 130k
+// 22.1 / 19.8, 1.2M 148 / 113, FP64 65k 19.2 / 23, 300k 76 / 62; sums 1.2M 14.7 / 9.6.
 constexpr int kCoopR = 2;
 template <class T>
-static constexpr int adj_quad_max() {
-  return sizeof(T) == 4 ? 256 * 1024 : 48 * 1024;
+static constexpr int adj_quad_max(int dim) {
+  return sizeof(T) == 8 ? 48 * 1024 : dim == 3 ? 256 * 1024 : 96 * 1024;
 }
+static constexpr bool adj_one_lane(int dim, int n) { return dim == 2 && n > 96 * 1024; }
 // Gathers in flight per lane in the reverse viscosity sweep.  Its four-vector
 // records take 152 VGPRs at four in flight (3 waves per SIMD); two keep it at
 // 110 (4 waves) and run faster.  The Jacobi sweeps keep four: at two they
@@ -118,15 +125,15 @@ constexpr int kNbVis = 2;
 // the latency of the walks of the few particles near a wall.  One lane with 8
 // in flight 21.0 us at 200k particles and 38.0 at 1M, quads with 2 / 4 in
 // flight 15.4 / 15.8 and 40.8 / 39.2.
-template <class T>
+template <class T, int L>
 __global__ void __launch_bounds__(kBlock)
     k_adj_bound_sums(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                      const int* __restrict__ nbr_nb, const V4<T>* __restrict__ bpos,
                      const int* __restrict__ bstart, V4<T>* __restrict__ bmom,
                      int* __restrict__ bflag) {
-  const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int i = coop_particle<L>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
-  const bool first = coop_lane<kQuad>() == 0;
+  const bool first = coop_lane<L>() == 0;
   if (nbr_nb[i] == 0) {  // the step found no boundary neighbour: nothing to walk
     if (first) bflag[i] = 0;
     return;
@@ -136,7 +143,7 @@ __global__ void __launch_bounds__(kBlock)
   node_encode(k, p.x, p.y, p.z, c);
   T ax = 0, ay = 0, az = 0, G = 0, hxx = 0, hyy = 0, hzz = 0, hxy = 0, hxz = 0, hyz = 0;
   int any = 0;
-  walk_quad_all<kBsumU>(k, bstart, c, [&](int j) { return bpos[j]; },
+  walk_all<L, kBsumU, 8>(k, bstart, c, [&](int j) { return bpos[j]; },
                         [&](int, const V4<T>& q, bool valid) {
     const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const T r2 = s_r2(dx, dy, dz);
@@ -155,10 +162,10 @@ __global__ void __launch_bounds__(kBlock)
     hyz += xh * dy * dz;
     any = 1;
   });
-  any = group_sum<kQuad>(any);
-  const V4<T> A = v4(group_sum<kQuad>(ax), group_sum<kQuad>(ay), group_sum<kQuad>(az), group_sum<kQuad>(G));
-  const V4<T> H = v4(group_sum<kQuad>(hxx), group_sum<kQuad>(hyy), group_sum<kQuad>(hzz), group_sum<kQuad>(hxy));
-  const V4<T> O = v4(group_sum<kQuad>(hxz), group_sum<kQuad>(hyz), T(0), T(0));
+  any = group_sum<L>(any);
+  const V4<T> A = v4(group_sum<L>(ax), group_sum<L>(ay), group_sum<L>(az), group_sum<L>(G));
+  const V4<T> H = v4(group_sum<L>(hxx), group_sum<L>(hyy), group_sum<L>(hzz), group_sum<L>(hxy));
+  const V4<T> O = v4(group_sum<L>(hxz), group_sum<L>(hyz), T(0), T(0));
   if (!first) return;
   bflag[i] = any != 0;
   if (any) {
@@ -391,7 +398,7 @@ __global__ void __launch_bounds__(kBlock)
 // 92 (with a branch per candidate) / 79 us.
 // (Terms that are left out are dropped by selects: 74 us with 2 in flight.)
 constexpr int kStRevU = 2;
-template <class T>
+template <class T, int L>
 __global__ void __launch_bounds__(kBlock)
     k_adj_surface_tension(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                           const T* __restrict__ fmass, const T* __restrict__ dens,
@@ -403,8 +410,8 @@ __global__ void __launch_bounds__(kBlock)
                           V4<T>* __restrict__ xbar, double* __restrict__ partial,
                           const TsphControl* ctrl) {
   __shared__ double lds[kWaves];
-  const int i = coop_particle<kQuad>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
-  const int cl = coop_lane<kQuad>();
+  const int i = coop_particle<L>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int cl = coop_lane<L>();
   double gsum = 0;
   if (i < n) {
     const T dt = (T)ctrl->dt;
@@ -427,7 +434,7 @@ __global__ void __launch_bounds__(kBlock)
       // spare lane (negative where j's 0.99 gate fails; the forward advection
       // writes it) and b_j
       auto loadn = [&](int j) { return Rec2<T>{tnormal[j], brec[j]}; };
-      walk_quad_all<kStRevU>(k, fstart, c, loadn, [&](int j, const Rec2<T>& d, bool valid) {
+      walk_all<L, kStRevU, 4>(k, fstart, c, loadn, [&](int j, const Rec2<T>& d, bool valid) {
         bool on = valid && j != i && d.a.w > T(0);
         if (on && j >= own0 && j < own1) {
           const V4<T> q = fpos[j];
@@ -479,17 +486,17 @@ __global__ void __launch_bounds__(kBlock)
         az += -gam * (cr * wz + s * dz);
         rb += -gam * rden * (r2d * mi * cr * bd - fij * mj * cr * ad);
       };
-      sweep_lists_coop<kQuad, T, Rec3<T>, 2>(
+      sweep_lists_coop<L, T, Rec3<T>, 2>(
           k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, loadc,
           loadc, coh, [&](const Rec3<T>&, bool) {});
-      nbx = group_sum<kQuad>(nbx);
-      nby = group_sum<kQuad>(nby);
-      nbz = group_sum<kQuad>(nbz);
-      ax = group_sum<kQuad>(ax);
-      ay = group_sum<kQuad>(ay);
-      az = group_sum<kQuad>(az);
-      rb = group_sum<kQuad>(rb);
-      gs = group_sum<kQuad>(gs);
+      nbx = group_sum<L>(nbx);
+      nby = group_sum<L>(nby);
+      nbz = group_sum<L>(nbz);
+      ax = group_sum<L>(ax);
+      ay = group_sum<L>(ay);
+      az = group_sum<L>(az);
+      rb = group_sum<L>(rb);
+      gs = group_sum<L>(gs);
     }
     if (cl == 0) {
       nbar[i] = v4(nbx, nby, nbz);
@@ -734,7 +741,7 @@ __global__ void __launch_bounds__(kBlock)
 // alpha_2_l = sum_j W'^2 X_j^2 / m_j -> x_bar_l += 2 g W'' (a2b_l X_j^2/m_j + a2b_j X_l^2/m_l) x
 // (boundary neighbours: density and alpha_1 terms of l's equation only;
 // alpha_2 of the fluid is (f,f) only, sph.py:194).
-template <class T>
+template <class T, int C>
 __global__ void __launch_bounds__(kBlock)
     k_adj_pass_a(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                  const T* __restrict__ fmass, const T* __restrict__ rhobar,
@@ -742,9 +749,9 @@ __global__ void __launch_bounds__(kBlock)
                  const int* __restrict__ nbr_f, const int* __restrict__ nbr_nf,
                  const V4<T>* __restrict__ bmom, const int* __restrict__ bflag,
                  V4<T>* __restrict__ xbar) {
-  const int i = coop_particle<kCoop>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
+  const int i = coop_particle<C>(coop_sub(Blk{(int)blockIdx.x, (int)gridDim.x}));
   if (i >= n) return;
-  const int cl = coop_lane<kCoop>();
+  const int cl = coop_lane<C>();
   const V4<T> p = fpos[i];
   const T Xi = p.w, mi = fmass[i];
   const T rbi = rhobar[i];
@@ -758,7 +765,7 @@ __global__ void __launch_bounds__(kBlock)
   // (f,f) pairs.  Record: a = position (w = X_j), b = a1bar_j (w = a2bar_j),
   // c = (rho_bar_j, m_j).  The (f,b) pairs (rho_bar_b = 0, no alpha_2 term,
   // DFSPH: m_b = X_b) are rho_bar_l A_l + M_l a1bar_l from the boundary sums.
-  sweep_lists_coop<kCoop, T, Rec4<T>>(
+  sweep_lists_coop<C, T, Rec4<T>>(
       k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0,
       [&](int j) {
         V4<T> q = fpos[j];
@@ -784,9 +791,9 @@ __global__ void __launch_bounds__(kBlock)
               q.w * abi.z - Xi * abj.z);
       },
       [&](const Rec4<T>&, bool) {});
-  ax = group_sum<kCoop>(ax);
-  ay = group_sum<kCoop>(ay);
-  az = group_sum<kCoop>(az);
+  ax = group_sum<C>(ax);
+  ay = group_sum<C>(ay);
+  az = group_sum<C>(az);
   if (cl != 0) return;
   if (hb) {
     ax += rbi * bs.m0.x;
@@ -843,7 +850,7 @@ int adj_solver_iteration(const TsphParams& prm, TsphObject* f, TsphObject* b, Ts
                        f->nbr_nf, (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->vbar_out,
                        (V4<T>*)a->xbar, ctrl);
   };
-  if (f->n <= adj_quad_max<T>())
+  if (f->n <= adj_quad_max<T>(prm.dim))
     iteration(k_adj_kappa<T, kQuad>, k_adj_vel<T, kQuad>, coop_blocks<kQuad>(f->n));
   else
     iteration(k_adj_kappa<T, kCoopR>, k_adj_vel<T, kCoopR>, coop_blocks<kCoopR>(f->n));
@@ -871,15 +878,19 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
                      (const T*)f->rest_density, (const V4<T>*)a->vbar, (V4<T>*)L.a1b,
                      a->nbar ? (V4<T>*)L.krec : (V4<T>*)nullptr, ctrl);
   if (a->nbar) {
-    hipLaunchKernelGGL(k_adj_surface_tension<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
-                       f->capacity, (const V4<T>*)f->pos, (const T*)f->mass,
-                       (const T*)f->sph_density, (const T*)f->rest_density,
-                       (const T*)f->volume_frac, f->cell_start, f->nbr_f, f->nbr_nf,
-                       (const V4<T>*)a->tape_normal, (const V4<T>*)a->vbar,
-                       (const V4<T>*)L.krec, (V4<T>*)a->nbar,
-                       (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
-    hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial,
-                       coop_blocks<kQuad>(f->n), a->grad, 1);
+    auto tension = [&](auto kern, int blocks) {
+      hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                         (const V4<T>*)f->pos, (const T*)f->mass, (const T*)f->sph_density,
+                         (const T*)f->rest_density, (const T*)f->volume_frac, f->cell_start,
+                         f->nbr_f, f->nbr_nf, (const V4<T>*)a->tape_normal, (const V4<T>*)a->vbar,
+                         (const V4<T>*)L.krec, (V4<T>*)a->nbar, (T*)a->rhobar, (V4<T>*)a->xbar,
+                         L.partial, ctrl);
+      hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial, blocks, a->grad, 1);
+    };
+    if (adj_one_lane(prm.dim, f->n))
+      tension(k_adj_surface_tension<T, 1>, nb);
+    else
+      tension(k_adj_surface_tension<T, kQuad>, coop_blocks<kQuad>(f->n));
   }
   auto viscosity = [&](auto kern, int nbk) {
     hipLaunchKernelGGL(kern, dim3(nbk), dim3(kBlock), 0, st, k, f->n, f->capacity,
@@ -890,7 +901,7 @@ int adj_advect(const TsphParams& prm, TsphObject* f, TsphControl* ctrl, TsphAdjo
                        (V4<T>*)a->vbar_out, (T*)a->rhobar, (V4<T>*)a->xbar, L.partial, ctrl);
     hipLaunchKernelGGL(k_adj_grad_add, dim3(1), dim3(kBlock), 0, st, L.partial, nbk, a->grad, 0);
   };
-  if (sizeof(T) == 4 || f->n <= adj_quad_max<T>())
+  if ((sizeof(T) == 4 && prm.dim == 3) || f->n <= adj_quad_max<T>(prm.dim))
     viscosity(k_adj_viscosity<T, kQuad>, coop_blocks<kQuad>(f->n));
   else
     viscosity(k_adj_viscosity<T, kCoopR>, coop_blocks<kCoopR>(f->n));
@@ -907,11 +918,16 @@ int adj_density_alpha(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphA
   hipLaunchKernelGGL(k_adj_alpha_prep<T>, dim3(nb), dim3(kBlock), 0, st, f->n, (const T*)f->alpha,
                      (const V4<T>*)f->alpha_1, (const T*)f->mass, (const T*)a->alphabar,
                      (V4<T>*)a->a1bar);
-  hipLaunchKernelGGL(k_adj_pass_a<T>, dim3(coop_blocks<kCoop>(f->n)), dim3(kBlock), 0, st, k,
-                     f->n, f->capacity,
-                     (const V4<T>*)f->pos, (const T*)f->mass, (const T*)a->rhobar,
-                     (const V4<T>*)a->a1bar, f->cell_start, f->nbr_f, f->nbr_nf,
-                     (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->xbar);
+  auto pass_a = [&](auto kern, int blocks) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                       (const V4<T>*)f->pos, (const T*)f->mass, (const T*)a->rhobar,
+                       (const V4<T>*)a->a1bar, f->cell_start, f->nbr_f, f->nbr_nf,
+                       (const V4<T>*)a->bmom, a->bflag, (V4<T>*)a->xbar);
+  };
+  if (sizeof(T) == 8 && adj_one_lane(prm.dim, f->n))
+    pass_a(k_adj_pass_a<T, kCoopR>, coop_blocks<kCoopR>(f->n));
+  else
+    pass_a(k_adj_pass_a<T, kCoop>, coop_blocks<kCoop>(f->n));
   TSPH_LAUNCH_CHECK("adj_density_alpha");
   return 0;
 }
@@ -921,9 +937,15 @@ int adj_bound_sums(const TsphParams& prm, TsphObject* f, TsphObject* b, TsphAdjo
                    hipStream_t st) {
   KP<T> k = make_kp<T>(prm);
   if (f->n == 0) return 0;
-  hipLaunchKernelGGL(k_adj_bound_sums<T>, dim3(coop_blocks<kQuad>(f->n)), dim3(kBlock), 0, st, k, f->n,
-                     f->capacity, (const V4<T>*)f->pos, f->nbr_nb, (const V4<T>*)b->pos,
-                     b->cell_start, (V4<T>*)a->bmom, a->bflag);
+  auto sums = [&](auto kern, int blocks) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, st, k, f->n, f->capacity,
+                       (const V4<T>*)f->pos, f->nbr_nb, (const V4<T>*)b->pos, b->cell_start,
+                       (V4<T>*)a->bmom, a->bflag);
+  };
+  if (adj_one_lane(prm.dim, f->n))
+    sums(k_adj_bound_sums<T, 1>, blocks_for(f->n));
+  else
+    sums(k_adj_bound_sums<T, kQuad>, coop_blocks<kQuad>(f->n));
   TSPH_LAUNCH_CHECK("adj_bound_sums");
   return 0;
 }
