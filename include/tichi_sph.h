@@ -342,12 +342,17 @@ int tsph_wcsph(const TsphParams* p, TsphObject* fluid, TsphObject* bound, TsphCo
  * is set, main.py:348): tsph_sort_object(fluid), tsph_density_alpha, the two
  * solves to their stop rule around tsph_advect, [tsph_wcsph], [tsph_fbm_round
  * while any particle was flagged, at most 1000 times], tsph_tail, on sorted
- * boundaries, with the same results.  Between launches the calling thread
- * waits where the next launch depends on the device: for each solve's
- * decision and each FBM round's flag, through the early stop signal
- * (tsph_solver_begin_signal) without draining the stream.  It returns with
- * the tail enqueued.  As after tsph_sort_object, *fluid's front and back
- * state pointers are swapped, also when a later part fails.
+ * boundaries, with the same results.  In scenes of up to 512k particles the
+ * advection, the density solve, the FBM rounds and the tail are enqueued with
+ * the divergence solve, on the guess that the solves and rounds take as many
+ * iterations as the last step's; the device checks the guess, and what it
+ * turned away is enqueued again.  The calling thread waits for each solve's
+ * decision and the last FBM round's flag through the early stop signal
+ * (tsph_solver_begin_signal) without draining the stream, where nothing is
+ * enqueued ahead (larger scenes, after a wrong guess, the parts after
+ * tsph_wcsph) before it enqueues what follows.  It returns with the tail
+ * enqueued.  As after tsph_sort_object, *fluid's front and back state pointers
+ * are swapped, also when a later part fails.
  */
 typedef struct TsphStep {
   int32_t cfl, wcsph, fbm;

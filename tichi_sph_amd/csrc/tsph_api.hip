@@ -578,8 +578,10 @@ constexpr int kStepHold = 16;
 constexpr int kStepRounds = 8;
 // Particles up to which a step launches ahead.  The stop signal leaves at the
 // start of a solve's last update, so from about here (25 us an update) the
-// host's answer arrives before that kernel ends: at 1M particles the step
-// takes 872 us either way (874 ahead).
+// host's answer arrives before that kernel ends.  us a step, waiting / ahead: 3D
+// FP32 27k 120 / 113, 97k 167 / 158, 216k 265 / 255, 314k 317 / 315, 439k 411 / 408,
+// 512k 448 / 447, 593k 516 / 516, 729k 608 / 610, 1M 835 / 836; FP64 97k 253 / 243,
+// 262k 448 / 447, 512k 834 / 835.
 constexpr int kStepAheadMax = 512 * 1024;
 
 int tsph_step(const TsphParams* p, TsphObject* f, TsphObject* b, TsphControl* ctrl, TsphStep* s,

@@ -374,18 +374,18 @@ __global__ void __launch_bounds__(kBlock)
 // The pair kernels, one instance per kernel id, a quad of lanes per particle
 // (tsph_sweep.h: walk_quad_cells): the quad tests the candidates of the Ngrid
 // four at a time and works off those in range, and every sum takes its terms
-// in the reference's order.  One kernel with
-// a switch over all ids, one lane per particle and the whole pair math on each
-// of the 200 or so candidates took 130-170 us per call at 100k particles; these
-// take 39-72 us there, bound by the dependent loads of the walk (entry, then
-// position).  A whole reference step at 4k / 100k / 1M: 3.5 / 4.0 / 15.5 ms,
-// now 1.09 / 1.65 / 9.5 (0.96 / 1.46 / 8.7 without k_ref_plain's calls and the row
-// check below).
+// in the reference's order.  One kernel with a switch over all ids, one lane per
+// particle and the whole pair math on each of the 200 or so candidates took
+// 130-170 us per call at 100k particles; these take 39-72 us there, bound by the
+// dependent loads of the walk (entry, then position).  A whole reference step at
+// 4k / 100k / 1M: 3.5 / 4.0 / 15.5 ms, now 1.09 / 1.65 / 9.5 (0.96 / 1.46 / 8.7
+// without k_ref_plain's calls and the row check below).
 // ---------------------------------------------------------------------------
+
 // The walk around cell cs[] of particle p over nuid's candidates up to r2lim
-// (those at a NaN distance among them).  A row of cells is one range where the Ngrid
-// holds them one after the other, as tsph_ngrid_build does; where it does not
-// (the reference's mem_shift, sph_obj.py:308-314, hands the ranges out in
+// (those at a NaN distance among them).  A row of cells is one range where the
+// Ngrid holds them one after the other, as tsph_ngrid_build does; where it does
+// not (the reference's mem_shift, sph_obj.py:308-314, hands the ranges out in
 // whatever order its threads reach the cells) every cell is read by itself.
 // Asking whether it does costs 1-2 us of a call's 39-72 at 100k particles.
 template <class T, class Load, class Term>

@@ -162,9 +162,16 @@ __device__ __forceinline__ int coop_particle(int sub) {
 }
 // Every scene's sweep in a grouped launch; f(entry, blk).  A block takes R of
 // a fluid tile's C sub-tiles: finding a tile's scene and its constants is a
-// chain of dependent loads, which R = C pays once per tile where the tiles
-// alone fill the chip (24 scenes, 2,700 tiles: psi 45.4 us, split 52.3);
-// fewer tiles are split (coop_split), as a single scene's launch is.
+// chain of dependent loads, which R = C pays once per tile, while split tiles
+// leave no block waiting for its last round.  us of psi and surface tension,
+// split / whole, FP32 by tiles: 96 6.0 / 11.4 and 15 / 37, 500 13.6 / 15.6 and 39 /
+// 53, 1000 22.6 / 24.5 and 65 / 75, 2000 40.1 / 43.4 and 121 / 144, 2304 46.2 / 45.5
+// and 138 / 151, 3000 57.5 / 62.6 and 175 / 201; FP64 1060 48 / 55, 2544 108 / 104.
+// Where no scene has surface tension its launch is the update alone, 10.8 / 7.6 at
+// 2275 tiles, and whole steps from 700 tiles on take the same time either way (24
+// scenes 2275 tiles 782 / 782, 48 scenes 3584 tiles 1000 / 1003, 64 scenes 15734
+// tiles 4091 / 4094).  Tiles up to coop_split's line are split, as a single scene's
+// launch is; above it whole ones take fewer blocks for the same time.
 template <class T, int C, int R, class F>
 __device__ __forceinline__ void for_coop_tiles(const char* __restrict__ tab, int ns, F&& f) {
   constexpr int split = C / R;
@@ -187,8 +194,9 @@ __device__ __forceinline__ T group_sum(T v) {
   return v;
 }
 
-// One list, lane c's share, software-pipelined like sweep_one_list, NB
-// gathers in flight per lane.  Every trip gathers NB records without a
+// One list, lane c's share of it, NB gathers in flight per lane; the next trip's
+// list entries are loaded right after this one's records are requested, so that a
+// trip costs one round trip to memory instead of two (index, then record).  Every trip gathers NB records without a
 // branch: a slot past the list's end reads the last slot again (a line the
 // group holds already) and pair(record, false) leaves it out of the sums, so
 // that the loads of a trip issue back to back.  With a branch around each
@@ -223,8 +231,9 @@ __device__ __forceinline__ void sweep_one_list_coop(int cap, int i, int c,
   }
 }
 
-// sweep_lists for lane c of a particle's group.  A particle whose list
-// overflowed is swept by lane 0 alone, walking the cells.
+// A particle's fluid list, then its boundary list, for lane c of its group.  A
+// particle whose list overflowed is swept by lane 0 alone, walking the cells with
+// the lists' in-range test.
 template <int C, class T, class Rec, int NB = kCoopNb, class LoadF, class LoadB, class PairF,
           class PairB>
 __device__ __forceinline__ void sweep_lists_coop(const KP<T>& k, int cap, int i, int c, V4<T> p,
