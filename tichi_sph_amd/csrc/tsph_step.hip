@@ -71,10 +71,12 @@ struct PassAAcc {
       r2 = s_r2(dx, dy, dz);
       r = pa_sqrt<FQ>(r2);
       qh = pa_quot<FQ>(k, r);
-      const T Wr = valid ? s_W_q_sel(k, qh) : T(0);
-      w = quad_add(w, Wr);
-      cp = quad_add(cp, Wr * vj);
-      dn = quad_add(dn, Wr * mj);
+      // (a lane without a slot holds another's: its products are dropped, since
+      // zero times an infinite mass is a NaN)
+      const T Wr = s_W_q_sel(k, qh);
+      w = quad_add(w, valid ? Wr : T(0));
+      cp = quad_add(cp, valid ? Wr * vj : T(0));
+      dn = quad_add(dn, valid ? Wr * mj : T(0));
     }
     const T u = T(1) - qh;
     T g = qh <= T(0.5) ? k.wg_a * (T(3) * qh - T(2)) : -k.wg_b * (u * u) * f_rcp(r);
@@ -412,10 +414,10 @@ __device__ __forceinline__ void pass_a_quad_bound(int sub, const KP<T>& k, const
               [&](const BoundRec<T>& r, int, bool valid, bool) {
                 TSPH_STRICT
                 const T d = s_sqrt(s_r2(p.x - r.q.x, p.y - r.q.y, p.z - r.q.z));
-                const T Wr = valid ? s_W_q_sel(k, d / k.h) : T(0);
-                w = quad_add(w, Wr);
-                cp = quad_add(cp, Wr * r.v);
-                dn = quad_add(dn, Wr * r.m);
+                const T Wr = s_W_q_sel(k, d / k.h);
+                w = quad_add(w, valid ? Wr : T(0));
+                cp = quad_add(cp, valid ? Wr * r.v : T(0));
+                dn = quad_add(dn, valid ? Wr * r.m : T(0));
               });
     if (ss != nullptr && c == 0) ss[i] = V4<T>{w, cp, dn, T(0)};
   }
@@ -428,10 +430,10 @@ __device__ __forceinline__ void pass_a_quad_bound(int sub, const KP<T>& k, const
                 TSPH_STRICT
                 const T d = s_sqrt(s_r2(p.x - r.q.x, p.y - r.q.y, p.z - r.q.z));
                 const T qh = d / k.h;
-                const T Wr = valid ? s_W_q_sel(k, qh) : T(0);
-                w = quad_add(w, Wr);
-                cp = quad_add(cp, Wr * r.v);
-                dn = quad_add(dn, Wr * r.m);
+                const T Wr = s_W_q_sel(k, qh);
+                w = quad_add(w, valid ? Wr : T(0));
+                cp = quad_add(cp, valid ? Wr * r.v : T(0));
+                dn = quad_add(dn, valid ? Wr * r.m : T(0));
                 const T wg = s_Wg_q(k, qh);
                 const T Xj = r.q.w;
                 const T wg2 = wg * wg;
@@ -637,7 +639,8 @@ __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n
         T r2 = dx * dx + dy * dy + dz * dz, r;
         T g = f_grad(k, r2, &r);
         T dot = (dx * (va.x - vj.x) + dy * (va.y - vj.y) + dz * (va.z - vj.z)) * g;
-        sum += (ok ? dot : T(0)) * q.w;
+        const T with = sum + dot * q.w;
+        sum = ok ? with : sum;  // (no zero times X_j: it may be infinite)
       };
       // (f,f) pairs from the list; the (f,b) pairs have v_j = 0 (boundary
       // vel_adv is never written), so their sum is v_i . sum_b X_j grad W_ij,
