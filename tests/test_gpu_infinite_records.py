@@ -2,12 +2,13 @@
 list reads its last neighbour again for the lanes and slots that are left over,
 and what those bring must be left out, not multiplied by zero (0 * inf is a NaN).
 Pass A by quads of lanes against single lanes (a grouped step) bit for bit, and
-one pair whose second particle is infinite in one quantity: the psi of the first
-is infinite, as the one term of its sum is."""
+one pair whose second particle is infinite in one quantity: the psi sweep and the
+gradient of the first are infinite, as the one term of their sums is."""
 import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +78,16 @@ def test_psi_of_an_infinite_neighbour(precision):
     _lib.check(lib.tsph_solver_begin(P, c, 0, st), "solver_begin")
     _lib.check(lib.tsph_solver_psi(P, f, b, c, 0, ws, wsb, st), "solver_psi")
     assert sim.fluid.to_numpy("psi_adv")[0] == np.inf
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+def test_gradient_of_an_infinite_neighbour(precision):
+    from tichi_sph_amd.adjoint import DiffRunner, rollout
+    sim = pair(precision)
+    dt = sim.fluid.dtype
+    away = torch.tensor([[-0.6, -0.64, -0.48], [0.6, 0.64, 0.48]], dtype=dt, device="cuda", requires_grad=True)
+    x, v = rollout(DiffRunner(sim), away, 0.05, 0.0, 1)
+    weight = torch.ones_like(v)
+    weight[1, 0] = np.inf
+    torch.autograd.backward((x, v), (torch.zeros_like(x), weight))
+    assert torch.isinf(away.grad[0]).all(), away.grad

@@ -266,17 +266,22 @@ __global__ void __launch_bounds__(kBlock)
   if (hb) bs = load_bound_sums(bmom, cap, i);
   T kb = 0, ax = 0, ay = 0, az = 0;
   auto term = [&](const Rec2<T>& d, bool ok) {  // a fluid neighbour j
+    const T kb0 = kb, ax0 = ax, ay0 = ay, az0 = az;
     const V4<T>& q = d.a;   // q.w = X_j = m_j
     const V4<T>& uj = d.b;  // xyz = u_j, w = kappa_j
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
-    e.g = ok ? e.g : T(0);
-    e.hq = ok ? e.hq : T(0);
     T rmj = f_rcp(q.w);  // hardware reciprocal in FP32 (the reverse is not a bit-exact sum)
     T mx = wx - uj.x * rmj, my = wy - uj.y * rmj, mz = wz - uj.z * rmj;
     kb += q.w * e.g * (dx * mx + dy * my + dz * mz);
     T c = ki * q.w + uj.w * Xi;
     add_J(ax, ay, az, e, dx, dy, dz, c * mx, c * my, c * mz);
+    // a slot past the list's end: the sums as they were, since a zero factor
+    // would make an infinite record a NaN
+    kb = ok ? kb : kb0;
+    ax = ok ? ax : ax0;
+    ay = ok ? ay : ay0;
+    az = ok ? az : az0;
   };
   // (f,f) pairs; the (f,b) pairs (u_b = kappa_b = 0) are w_l . A_l and
   // kappa_l M_l w_l from the boundary sums
@@ -335,18 +340,23 @@ __global__ void __launch_bounds__(kBlock)
   if (hb) bs = load_bound_sums(bmom, cap, i);
   T vx = 0, vy = 0, vz = 0, ax = 0, ay = 0, az = 0;
   auto term = [&](const Rec2<T>& d, bool ok) {
+    const T vx0 = vx, vy0 = vy, vz0 = vz, ax0 = ax, ay0 = ay, az0 = az;
     const V4<T>& q = d.a;   // q.w = X_j
     const V4<T>& vj = d.b;  // xyz = vel_adv_j, w = psib_j
     T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
-    e.g = ok ? e.g : T(0);
-    e.hq = ok ? e.hq : T(0);
     T c = pbi * q.w + vj.w * Xi;
     T cg = c * e.g;
     vx += cg * dx;
     vy += cg * dy;
     vz += cg * dz;
     add_J(ax, ay, az, e, dx, dy, dz, c * (vi.x - vj.x), c * (vi.y - vj.y), c * (vi.z - vj.z));
+    vx = ok ? vx : vx0;
+    vy = ok ? vy : vy0;
+    vz = ok ? vz : vz0;
+    ax = ok ? ax : ax0;
+    ay = ok ? ay : ay0;
+    az = ok ? az : az0;
   };
   // (f,f) pairs; the (f,b) pairs (v_b = psib_b = 0) are psib_l A_l and
   // psib_l M_l v_l from the boundary sums
@@ -578,6 +588,8 @@ __global__ void __launch_bounds__(kBlock)
     const V4<T> xb = xbar[i];
     T vbx = 0, vby = 0, vbz = 0, xbx = 0, xby = 0, xbz = 0, Vb = 0, ms = 0;
     auto term = [&](const Rec4<T>& d, bool ok) {
+      const T vbx0 = vbx, vby0 = vby, vbz0 = vbz, xbx0 = xbx, xby0 = xby, xbz0 = xbz;
+      const T Vb0 = Vb, ms0 = ms;
       const V4<T>& q = d.a;   // position
       const V4<T>& vj = d.b;  // velocity, w = V_j
       const V4<T>& aj = d.c;  // a_bar_j, w = fv_j
@@ -585,8 +597,6 @@ __global__ void __launch_bounds__(kBlock)
       T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       T r2 = dx * dx + dy * dy + dz * dz;
       D2<T> e = kern_d2(k, r2);
-      e.g = ok ? e.g : T(0);
-      e.hq = ok ? e.hq : T(0);
       T den = k.eps + r2;
       T rden = f_rcp(den);
       T w = e.g * rden;
@@ -614,6 +624,14 @@ __global__ void __launch_bounds__(kBlock)
       xbx += -k.h * (e.g * cx + s * dx);
       xby += -k.h * (e.g * cy + s * dy);
       xbz += -k.h * (e.g * cz + s * dz);
+      vbx = ok ? vbx : vbx0;
+      vby = ok ? vby : vby0;
+      vbz = ok ? vbz : vbz0;
+      xbx = ok ? xbx : xbx0;
+      xby = ok ? xby : xby0;
+      xbz = ok ? xbz : xbz0;
+      Vb = ok ? Vb : Vb0;
+      ms = ok ? ms : ms0;
     };
     sweep_lists_coop<C, T, Rec4<T>, kNbVis>(
         k, cap, i, cl, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
@@ -779,8 +797,7 @@ __global__ void __launch_bounds__(kBlock)
         const T rbj = d.c.x, mj = d.c.y;
         T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         D2<T> e = kern_d2(k, dx * dx + dy * dy + dz * dz);
-        e.g = ok ? e.g : T(0);
-        e.hq = ok ? e.hq : T(0);
+        const T ax0 = ax, ay0 = ay, az0 = az;
         T cd = (rbi * mj + rbj * mi) * e.g;
         T c2 = T(2) * e.g * e.w2 * (abi.w * q.w * q.w * f_rcp(mj) + abj.w * xm_i);
         T s1 = cd + c2;
@@ -789,6 +806,9 @@ __global__ void __launch_bounds__(kBlock)
         az += s1 * dz;
         add_J(ax, ay, az, e, dx, dy, dz, q.w * abi.x - Xi * abj.x, q.w * abi.y - Xi * abj.y,
               q.w * abi.z - Xi * abj.z);
+        ax = ok ? ax : ax0;
+        ay = ok ? ay : ay0;
+        az = ok ? az : az0;
       },
       [&](const Rec4<T>&, bool) {});
   ax = group_sum<C>(ax);
