@@ -1,4 +1,6 @@
 // extern "C" entry points declared in include/tichi_sph.h.
+#include <algorithm>
+#include <climits>
 #include <cstdarg>
 
 #include <cstring>
@@ -68,7 +70,10 @@ int batch_prepare(const TsphParams* p, const TsphObject* f, const TsphObject* b,
   std::memset(host, 0, batch_table_bytes<T>(ns));
   SceneEntry<T>* E = (SceneEntry<T>*)host;
   int* first = (int*)((char*)host + batch_entries_bytes<T>(ns));
-  int tot[kTileKinds] = {0, 0, 0, 0};
+  int tot[kTileKinds] = {};
+  long tiles = 0;
+  for (int s = 0; s < ns; ++s) tiles += f[s].n > 0 ? blocks_for(f[s].n) : 0;
+  const bool one_lane_2d = st_one_lane(2, (int)std::min(tiles * kBlock, (long)INT_MAX));
   for (int s = 0; s < ns; ++s) {
     TSPH_REQUIRE(p[s].precision == p[0].precision, TSPH_EINVAL,
                  "tsph_batch_prepare: scene %d has another precision", s);
@@ -81,8 +86,10 @@ int batch_prepare(const TsphParams* p, const TsphObject* f, const TsphObject* b,
     E[s].ctrl = ctrl[s];
     TSPH_REQUIRE(carve_ws(ws[s], wsb[s], f[s].capacity, p[s].node_num, &E[s].L), TSPH_ECAPACITY,
                  "tsph_batch_prepare: workspace of scene %d too small", s);
-    const int t[kTileKinds] = {blocks_for(f[s].n), blocks_for(b[s].n),
-                               (int)cell_tiles(p[s].node_num), 1};
+    const bool whole = E[s].k.gamma == T(0) || (p[s].dim == 2 && one_lane_2d);
+    const int nf = blocks_for(f[s].n);
+    const int t[kTileKinds] = {nf, blocks_for(b[s].n), (int)cell_tiles(p[s].node_num), 1,
+                               whole ? nf : 0, whole ? 0 : nf};
     for (int q = 0; q < kTileKinds; ++q) {
       first[q * (ns + 1) + s] = tot[q];
       tot[q] += t[q];
@@ -90,7 +97,7 @@ int batch_prepare(const TsphParams* p, const TsphObject* f, const TsphObject* b,
   }
   for (int q = 0; q < kTileKinds; ++q) {
     first[q * (ns + 1) + ns] = tot[q];
-    info->tiles[q] = tot[q];
+    if (q < kTileCounts) info->tiles[q] = tot[q];
   }
   info->nscenes = ns;
   info->precision = p[0].precision;

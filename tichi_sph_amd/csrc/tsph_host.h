@@ -176,7 +176,24 @@ struct SceneEntry {
   WsLayout L;
 };
 
-enum TileKind { kTileFluid = 0, kTileBound = 1, kTileCell = 2, kTileScene = 3, kTileKinds = 4 };
+// Surface tension takes the fluid tiles of a scene whole or by quads (kTileWhole,
+// kTileQuads: st_one_lane); the launch counts are those of the first four kinds.
+enum TileKind {
+  kTileFluid = 0, kTileBound = 1, kTileCell = 2, kTileScene = 3, kTileCounts = 4,
+  kTileWhole = 4, kTileQuads = 5, kTileKinds = 6
+};
+
+// Surface tension of a 2D scene of n particles by one lane per particle instead of four
+// (in four partial sums, a quad's bit for bit); a grouped launch goes by its scenes'
+// particles together.  In 2D there are three rows of half the candidates, so that a
+// quad's lanes do less each than the look-up of the rows.  us, one lane / quads: 9k 10.5
+// / 7.1, 65k 11.5 / 10.4, 90k 12.3 / 13.7, 300k 21.6 / 32.0, 1M 54.7 / 91, FP64 65k 17.7
+// / 16.1, 90k 20 / 23.2, 1M 120 / 202; grouped, 49k 12.0 / 10.2, 98k 14.6 / 14.3, 190k
+// 19.2 / 26.1, 737k 48.3 / 84.5, FP64 98k 22.6 / 25.9, 737k 94 / 158.  In 3D quads stay:
+// grouped, 737k 194 / 171, FP64 1.2M 553 / 534.
+__host__ __device__ __forceinline__ bool st_one_lane(int dim, int n) {
+  return dim == 2 && n > 72 * 1024;
+}
 
 template <class T>
 __host__ __device__ inline size_t batch_entries_bytes(int ns) {

@@ -904,18 +904,97 @@ __global__ void __launch_bounds__(kBlock)
 // (Dropping the terms of a candidate that is left out, instead of multiplying
 // them by zero, costs 1 us at 200k and 8 at 2M.)
 constexpr int kStFwdU = 6;
-// In 2D there are three rows of half that, and large scenes take one lane per
-// particle (also with six in flight; eight of the walk and the list raise the
-// grouped kernels' registers), us, one lane / quads: FP32 9k 10.5 / 7.1, 65k 11.5 /
-// 10.4, 90k 12.3 / 13.7, 130k 12.9 / 18.2, 300k 21.6 / 32.0, 1M 54.7 / 91; FP64 9k
-// 16.4 / 8.6, 65k 17.7 / 16.1, 90k 20 / 23.2, 300k 40.0 / 60.4, 1M 120 / 202.  The
-// rule is a scene's own, also in a grouped launch, so that both sum in one order.
-__host__ __device__ __forceinline__ bool st_one_lane(int dim, int n) {
-  return dim == 2 && n > 72 * 1024;
+// One lane per particle (st_one_lane) has kStOneU in flight; eight of the walk and the
+// list raise the registers of the grouped kernel.
+constexpr int kStOneU = 4;
+// One particle, by L lanes: a quad, or one lane in a quad's order (the same sums
+// bit for bit, so that a scene's own launch and a grouped one may differ in it).
+template <class T, int L>
+__device__ __forceinline__ void st_particle(int i, const KP<T>& k, int cap,
+                      const V4<T>* __restrict__ fpos, const T* __restrict__ psi_rho,
+                      const T* __restrict__ rdens, const T* __restrict__ vf,
+                      const int* __restrict__ fstart, const V4<T>* __restrict__ normal,
+                      const V4<T>* __restrict__ strec, const int* __restrict__ nbr_f,
+                      const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
+                      V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv, T dt) {
+  const int cl = coop_lane<L>();
+  V4<T> a = acce_adv[i];
+  if (vf[(long)i * k.P] > T(0.99)) {
+    V4<T> p = fpos[i];
+    V4<T> ni = normal[i];
+    T rp = rest_psi_of(k, rdens, i);
+    T psi_i = psi_rho[i];
+    int c[3];
+    node_encode(k, p.x, p.y, p.z, c);
+    // the normal record's spare lane holds +-psi_j, negative where j's 0.99
+    // gate fails (the advection sweep writes it).  Reciprocal square root
+    // and reciprocals instead of the IEEE forms: the pair terms of these
+    // sums are not part of the bit-exact sums.
+    constexpr int S = L == 1 ? kQuad : 1;  // partial sums per lane
+    T ux[S], uy[S], uz[S];                 // sums of (n_i - n_j) / (psi_i + psi_j)
+#pragma unroll
+    for (int u = 0; u < S; ++u) ux[u] = uy[u] = uz[u] = T(0);
+    auto curv = [&](int u, int j, const V4<T>& nj, bool valid) {
+      // a candidate left out may hold anything: its terms are dropped, not
+      // multiplied by zero
+      const bool on = valid && j != i && nj.w > T(0);
+      const T w = f_rcp(psi_i + nj.w);
+      ux[u] += on ? w * (ni.x - nj.x) : T(0);
+      uy[u] += on ? w * (ni.y - nj.y) : T(0);
+      uz[u] += on ? w * (ni.z - nj.z) : T(0);
+    };
+    auto loadn = [&](int j) { return normal[j]; };
+    // per in-range neighbour: (x_j, m_j) and the normal record
+    auto load = [&](int j) { return Rec2<T>{strec[j], normal[j]}; };
+    auto coh = [&](int u, const Rec2<T>& d, bool ok) {  // - m_j C(r) x_ij / r / (psi_i + psi_j)
+      const V4<T>& q = d.a;
+      const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+      const T r2 = dx * dx + dy * dy + dz * dz;
+      const T rinv = f_rsqrt(r2);
+      T s = q.w * f_coh(k, r2 * rinv * k.inv_h) * rinv * f_rcp(psi_i + d.b.w);
+      s = ok && d.b.w > T(0) ? s : T(0);
+      ux[u] -= s * dx;
+      uy[u] -= s * dy;
+      uz[u] -= s * dz;
+    };
+    T sx, sy, sz;
+    if constexpr (L == 1) {
+      walk_as_quad<kStOneU>(k, fstart, c, loadn, curv);
+      sweep_list_as_quad<Rec2<T>, kQuad>(k, cap, i, p, c, fstart, fpos, nbr_f, nbr_nf[i], load,
+                                         coh);
+      sx = (ux[0] + ux[1]) + (ux[2] + ux[3]);
+      sy = (uy[0] + uy[1]) + (uy[2] + uy[3]);
+      sz = (uz[0] + uz[1]) + (uz[2] + uz[3]);
+    } else {
+      walk_quad_all<kStFwdU>(k, fstart, c, loadn, [&](int j, const V4<T>& nj, bool valid) {
+        curv(0, j, nj, valid);
+      });
+      sweep_lists_coop<kQuad, T, Rec2<T>>(
+          k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, load,
+          load, [&](const Rec2<T>& d, bool ok) { coh(0, d, ok); }, [&](const Rec2<T>&, bool) {});
+      sx = group_sum<kQuad>(ux[0]);
+      sy = group_sum<kQuad>(uy[0]);
+      sz = group_sum<kQuad>(uz[0]);
+    }
+    // 2 psi_0 / (psi_i + psi_j) (cohesion + curvature), cohesion =
+    // -gamma m_j C(r) x_ij / r, curvature = gamma (n_i - n_j)
+    const T f = T(2) * rp * k.gamma;
+    a.x += f * sx;
+    a.y += f * sy;
+    a.z += f * sz;
+    if (cl == 0) acce_adv[i] = a;
+  }
+  if (cl != 0) return;
+  {
+    TSPH_STRICT  // SPH_advection_update_vel_adv, sph.py:247-250
+    const V4<T> v = vel[i];
+    vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
+  }
 }
-// L lanes per particle; with one, the R sub-tiles' particles are the block's
-// first R * kBlock / kQuad threads.
-template <class T, int L, int R>
+
+// A block's particles: with a quad each the sub-tile of 64 (blk counts sub-tiles),
+// with one lane each the tile of 256 (blk counts tiles).
+template <class T, int L>
 __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, int n, int cap,
                       const V4<T>* __restrict__ fpos, const T* __restrict__ psi_rho,
                       const T* __restrict__ rdens, const T* __restrict__ vf,
@@ -924,79 +1003,24 @@ __device__ __forceinline__ void k_surface_tension_body(Blk blk, const KP<T>& k, 
                       const int* __restrict__ nbr_nf, const V4<T>* __restrict__ vel,
                       V4<T>* __restrict__ acce_adv, V4<T>* __restrict__ vadv,
                       const TsphControl* ctrl) {
-  const int cl = coop_lane<L>();
   const T dt = (T)ctrl->dt;
-  const int own = coop_sub<R>(blk) * (kBlock / kQuad) + (int)threadIdx.x;
-  const bool has = (int)threadIdx.x < R * (kBlock / kQuad) && own < n;
-  if (k.gamma == T(0)) {  // a scene without it in a grouped launch: the update alone
-    TSPH_STRICT
-    if (!has) return;
-    const V4<T> v = vel[own], a = acce_adv[own];
-    vadv[own] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
-    return;
-  }
-  if (L == 1 && !has) return;
-#pragma unroll 1
-  for (int r = 0; r < (L == 1 ? 1 : R); ++r) {
-    const int i = L == 1 ? own : coop_particle<kQuad>(coop_sub<R>(blk, r));
-    if (i >= n) break;
-    V4<T> a = acce_adv[i];
-    if (vf[(long)i * k.P] > T(0.99)) {
-      V4<T> p = fpos[i];
-      V4<T> ni = normal[i];
-      T rp = rest_psi_of(k, rdens, i);
-      T psi_i = psi_rho[i];
-      int c[3];
-      node_encode(k, p.x, p.y, p.z, c);
-      // the normal record's spare lane holds +-psi_j, negative where j's 0.99
-      // gate fails (the advection sweep writes it).  Reciprocal square root
-      // and reciprocals instead of the IEEE forms: the pair terms of these
-      // sums are not part of the bit-exact sums.
-      T ux = 0, uy = 0, uz = 0;  // sum of (n_i - n_j) / (psi_i + psi_j)
-      walk_all<L, kStFwdU, kStFwdU>(k, fstart, c, [&](int j) { return normal[j]; },
-                              [&](int j, const V4<T>& nj, bool valid) {
-        // a candidate left out may hold anything: its terms are dropped, not
-        // multiplied by zero
-        const bool on = valid && j != i && nj.w > T(0);
-        const T w = f_rcp(psi_i + nj.w);
-        ux += on ? w * (ni.x - nj.x) : T(0);
-        uy += on ? w * (ni.y - nj.y) : T(0);
-        uz += on ? w * (ni.z - nj.z) : T(0);
-      });
-      // per in-range neighbour: (x_j, m_j) and the normal record
-      auto load = [&](int j) { return Rec2<T>{strec[j], normal[j]}; };
-      auto coh = [&](const Rec2<T>& d, bool ok) {  // - m_j C(r) x_ij / r / (psi_i + psi_j)
-        const V4<T>& q = d.a;
-        const T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        const T rinv = f_rsqrt(r2);
-        T s = q.w * f_coh(k, r2 * rinv * k.inv_h) * rinv * f_rcp(psi_i + d.b.w);
-        s = ok && d.b.w > T(0) ? s : T(0);
-        ux -= s * dx;
-        uy -= s * dy;
-        uz -= s * dz;
-      };
-      sweep_lists_coop<L, T, Rec2<T>>(
-          k, cap, i, cl, p, fstart, nullptr, fpos, nullptr, nbr_f, nullptr, nbr_nf[i], 0, load,
-          load, coh, [&](const Rec2<T>&, bool) {});
-      ux = group_sum<L>(ux);
-      uy = group_sum<L>(uy);
-      uz = group_sum<L>(uz);
-      // 2 psi_0 / (psi_i + psi_j) (cohesion + curvature), cohesion =
-      // -gamma m_j C(r) x_ij / r, curvature = gamma (n_i - n_j)
-      const T f = T(2) * rp * k.gamma;
-      a.x += f * ux;
-      a.y += f * uy;
-      a.z += f * uz;
-      if (cl == 0) acce_adv[i] = a;
-    }
-    if (cl != 0) continue;
-    {
-      TSPH_STRICT  // SPH_advection_update_vel_adv, sph.py:247-250
-      const V4<T> v = vel[i];
-      vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
-    }
-  }
+  const int i = coop_particle<L>(coop_sub(blk));
+  if (i < n)
+    st_particle<T, L>(i, k, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf,
+                      vel, acce_adv, vadv, dt);
+}
+// vel_adv = vel + dt acce_adv alone, of a scene without surface tension in a grouped
+// launch: a tile of 256 particles.
+template <class T>
+__device__ __forceinline__ void st_update_only(Blk blk, int n, const V4<T>* __restrict__ vel,
+                                               const V4<T>* __restrict__ acce_adv,
+                                               V4<T>* __restrict__ vadv, const TsphControl* ctrl) {
+  TSPH_STRICT
+  const int i = xcd_block(blk.b, blk.nb) * kBlock + (int)threadIdx.x;
+  if (i >= n) return;
+  const T dt = (T)ctrl->dt;
+  const V4<T> v = vel[i], a = acce_adv[i];
+  vadv[i] = V4<T>{v.x + a.x * dt, v.y + a.y * dt, v.z + a.z * dt, T(0)};
 }
 
 // SPH_advection_update_vel_adv alone (sph.py:247-250), for gamma = 0: a
@@ -1018,7 +1042,7 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 template <class T, int L>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 7 : 1)  // 72 registers, not 75
     k_surface_tension(KP<T> k, int n, int cap, const V4<T>* __restrict__ fpos,
                       const T* __restrict__ psi_rho,
                       const T* __restrict__ rdens, const T* __restrict__ vf,
@@ -1029,7 +1053,7 @@ __global__ void __launch_bounds__(kBlock)
                       TsphControl* ctrl, SolveOpen open) {
   if (open.ahead && !ctrl->go) return;
   if (open.on && blockIdx.x == 0) solver_begin_body(k, ctrl, 1, (int*)open.signal, open.token);
-  k_surface_tension_body<T, L, L == 1 ? kQuad : 1>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
+  k_surface_tension_body<T, L>(Blk{(int)blockIdx.x, (int)gridDim.x}, k, n, cap, fpos, psi_rho, rdens, vf, fstart, normal, strec, nbr_f, nbr_nf, vel, acce_adv, vadv, ctrl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1829,19 +1853,39 @@ __global__ void __launch_bounds__(kBlock) kb_advect(const char* __restrict__ tab
   });
 }
 
-template <class T, int R>
-__global__ void __launch_bounds__(kBlock) kb_surface_tension(const char* __restrict__ tab, int ns) {
-  for_coop_tiles<T, kQuad, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
+// Tiles [0, whole tiles) are whole ones (one lane per particle, or the update alone),
+// the rest sub-tiles of a quad each.  Each kind has its own tiles: blocks of a scene's
+// sub-tiles that leave its work to every fourth one fill a quarter of the shader engines
+// (2D, 2880 tiles: 146 us, and 48).  FP64 is held to 128 registers for four waves per
+// SIMD: 3D, 768 tiles 94 us, with 132 registers and three 103; 4608 tiles 531 and 592.
+template <class T>
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 6 : 4)
+    kb_surface_tension(const char* __restrict__ tab, int ns) {
+  const int tw = tile_prefix<T, kTileWhole>(tab, ns)[ns];
+  const int total = tw + tile_prefix<T, kTileQuads>(tab, ns)[ns] * kQuad;
+  auto scene = [&](const SceneEntry<T>& e, Blk blk, auto lanes) {
     const TsphObject& f = e.f;
-    auto scene = [&](auto lanes) {
-      k_surface_tension_body<T, decltype(lanes)::value, R>(
-          blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e), (const T*)f.rest_density,
-          (const T*)f.volume_frac, f.cell_start, (const V4<T>*)f.normal, (const V4<T>*)e.L.krec,
-          f.nbr_f, f.nbr_nf, (const V4<T>*)f.vel, (V4<T>*)f.acce_adv, (V4<T>*)f.vel_adv, e.ctrl);
-    };
-    if (st_one_lane(e.k.dim, f.n)) scene(std::integral_constant<int, 1>{});
-    else scene(std::integral_constant<int, kQuad>{});
-  });
+    k_surface_tension_body<T, decltype(lanes)::value>(
+        blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, psi_of(e), (const T*)f.rest_density,
+        (const T*)f.volume_frac, f.cell_start, (const V4<T>*)f.normal, (const V4<T>*)e.L.krec,
+        f.nbr_f, f.nbr_nf, (const V4<T>*)f.vel, (V4<T>*)f.acce_adv, (V4<T>*)f.vel_adv, e.ctrl);
+  };
+  for (int t = blockIdx.x; t < total; t += gridDim.x) {
+    if (t < tw)
+      on_tile<T, kTileWhole>(tab, ns, t, [&](const SceneEntry<T>& e, int, Blk tile) {
+        const TsphObject& f = e.f;
+        if (e.k.gamma == T(0))
+          st_update_only<T>(tile, f.n, (const V4<T>*)f.vel, (const V4<T>*)f.acce_adv,
+                            (V4<T>*)f.vel_adv, e.ctrl);
+        else
+          scene(e, tile, std::integral_constant<int, 1>{});
+      });
+    else
+      on_tile<T, kTileQuads>(tab, ns, (t - tw) / kQuad, [&](const SceneEntry<T>& e, int, Blk tile) {
+        scene(e, Blk{tile.b * kQuad + (t - tw) % kQuad, tile.nb * kQuad},
+              std::integral_constant<int, kQuad>{});
+      });
+  }
 }
 
 template <class T>
@@ -1924,12 +1968,8 @@ int batch_advect(const TsphBatchInfo& bi, char* tab, int grid, hipStream_t st) {
                        tab, bi.nscenes);
   else
     hipLaunchKernelGGL((kb_advect<T, kCoop>), dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
-  if (coop_split(tiles))
-    hipLaunchKernelGGL((kb_surface_tension<T, 1>), dim3(grid_for(tiles * kQuad, grid)),
-                       dim3(kBlock), 0, st, tab, bi.nscenes);
-  else
-    hipLaunchKernelGGL((kb_surface_tension<T, kQuad>), dim3(g), dim3(kBlock), 0, st, tab,
-                       bi.nscenes);
+  hipLaunchKernelGGL(kb_surface_tension<T>, dim3(grid_for(tiles * kQuad, grid)), dim3(kBlock), 0, st,
+                     tab, bi.nscenes);
   TSPH_LAUNCH_CHECK("batch_advect");
   return 0;
 }

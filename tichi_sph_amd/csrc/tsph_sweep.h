@@ -500,6 +500,51 @@ __device__ __forceinline__ void walk_all(const KP<T>& k, const int* __restrict__
     walk_cells_prefetch<U1>(k, cstart, cc, load, [&](int j, const auto& d) { f(j, d, true); });
 }
 
+// The same candidates, and a list's slots, by one lane in the order of a quad: f and
+// pair also get the lane of the quad that would take each, so that sums kept apart
+// by it and added as group_sum does are a quad's bit for bit.
+template <int U, class T, class Load, class F>
+__device__ __forceinline__ void walk_as_quad(const KP<T>& k, const int* __restrict__ cstart,
+                                             const int* cc, Load&& load, F&& f) {
+  static_assert(U % kQuad == 0, "a trip is whole rounds of a quad");
+  walk_runs(k, cstart, cc, [&](int j0, int j1) {
+    for (int j = j0; j < j1; j += U) {
+      decltype(load(0)) rec[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) rec[u] = load(min(j + u, j1 - 1));
+#pragma unroll
+      for (int u = 0; u < U; ++u) f(u % kQuad, j + u, rec[u], j + u < j1);
+    }
+  });
+}
+template <class Rec, int NB, class T, class Load, class Pair>
+__device__ __forceinline__ void sweep_list_as_quad(const KP<T>& k, int cap, int i, const V4<T>& p,
+                                                   const int* cc, const int* __restrict__ fstart,
+                                                   const V4<T>* __restrict__ fpos,
+                                                   const int* __restrict__ list, int n,
+                                                   Load&& load, Pair&& pair) {
+  static_assert(NB % kQuad == 0, "a trip is whole rounds of a quad");
+  if (n > k.list_cap_f) {  // overflowed: the quad's first lane walks the cells
+    walk_cells(k, fstart, cc, [&](int j) {
+      const V4<T> q = fpos[j];
+      const T r2 = s_r2(p.x - q.x, p.y - q.y, p.z - q.z);
+      if (r2 > T(0) && r2 <= k.r2max) pair(0, load(j), true);
+    });
+    return;
+  }
+  for (int s = 0; s < n; s += NB) {
+    int j[NB];
+    Rec d[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) j[u] = list[(long)min(s + u, n - 1) * cap + i];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) d[u] = load(j[u]);
+#pragma unroll
+    for (int u = 0; u < NB; ++u) pair(u % kQuad, d[u], s + u < n);
+  }
+}
+
+
 // The walk of an object in cell order around p, taking the candidates in range
 // (r^2 <= r2max).
 template <class T, class Load, class Term>
