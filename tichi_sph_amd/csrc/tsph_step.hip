@@ -602,7 +602,7 @@ __global__ void k_solver_begin(KP<T> k, TsphControl* ctrl, int solve, int* signa
 
 // Jacobi half-step P: IPPE_adv_psi_init + IPPE_adv_psi (f,f)(f,b) +
 // IPPE_psi_adv_non_negative (sph.py:196-226) for iteration kk of the solve.
-template <class T, int R = 1>
+template <class T, int R = 1, bool GROUP = false>
 __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n, int cap, int kk, const V4<T>* __restrict__ fpos,
                  const V4<T>* __restrict__ vadv, const T* __restrict__ psi_rho,
                  const T* __restrict__ rdens, const T* __restrict__ alpha,
@@ -645,7 +645,8 @@ __device__ __forceinline__ void k_solver_psi_body(Blk blk, const KP<T>& k, int n
       // (f,f) pairs from the list; the (f,b) pairs have v_j = 0 (boundary
       // vel_adv is never written), so their sum is v_i . sum_b X_j grad W_ij,
       // the boundary share of alpha_1 that pass A recorded
-      sweep_lists_coop<kCoop, T, Rec2<T>>(
+      sweep_lists_coop<kCoop, T, Rec2<T>, GROUP ? group_nb<T, Rec2<T>, R>(3) : kCoopNb,
+                     GROUP ? group_nb<T, Rec2<T>, R>(2) : kCoopNb>(
           k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
           [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
           [&](int) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
@@ -709,7 +710,7 @@ __global__ void __launch_bounds__(kBlock)
 // alpha_1 = sum_j X_j grad W_ij of pass A (positions and X do not change
 // within the step), so the sweep only visits the fluid list, gathering the
 // one record (x_j, kappa_j) that the psi half-step wrote.
-template <class T, int R = 1>
+template <class T, int R = 1, bool GROUP = false>
 __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, int n, int cap, int kk, const V4<T>* __restrict__ fpos,
                     const T* __restrict__ fmass, const T* __restrict__ kappa,
                     const V4<T>* __restrict__ krec, const V4<T>* __restrict__ alpha_1,
@@ -765,7 +766,8 @@ __device__ __forceinline__ void k_solver_update_body(Blk blk, const KP<T>& k, in
       sy += s * dy;
       sz += s * dz;
     };
-    sweep_lists_coop<kCoopU, T, V4<T>>(
+    sweep_lists_coop<kCoopU, T, V4<T>, GROUP ? group_nb<T, V4<T>, R>(3) : kCoopNb,
+                     GROUP ? group_nb<T, V4<T>, R>(2) : kCoopNb>(
         k, cap, i, cl, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
         [&](int j) { return krec[j]; }, [&](int) { return V4<T>{}; }, term,
         [&](const V4<T>&, bool) {});
@@ -806,7 +808,7 @@ __global__ void __launch_bounds__(kBlock)
 // must not write vel_adv: the update vel_adv = vel + dt * acce_adv happens in
 // the next kernel (k_surface_tension).
 // ---------------------------------------------------------------------------
-template <class T, int R = 1>
+template <class T, bool GROUP = false>
 __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, int cap, const V4<T>* __restrict__ fpos, const T* __restrict__ vf,
              const T* __restrict__ rdens, const int* __restrict__ fstart,
              const int* __restrict__ bstart, const V4<T>* __restrict__ bpos,
@@ -815,60 +817,58 @@ __device__ __forceinline__ void k_advect_body(Blk blk, const KP<T>& k, int n, in
              V4<T>* __restrict__ normal, const T* __restrict__ fmass,
              const T* __restrict__ psi_rho, V4<T>* __restrict__ strec) {
   const int c = coop_lane<kCoop>();
-#pragma unroll 1
-  for (int r = 0; r < R; ++r) {
-    const int i = coop_particle<kCoop>(coop_sub<R>(blk, r));
-    if (i >= n) break;
-    const V4<T> p = fpos[i];
-    const V4<T> vi = vadv[i];
-    const T fvis = k.two_d2 * mu_of(k, vf, i) / rdens[i];
-    T ax = 0, ay = 0, az = 0, nx = 0, ny = 0, nz = 0;  // this lane's share
-    auto term = [&](const Rec2<T>& d, bool ok) {
-      const V4<T>& q = d.a;
-      const V4<T>& vj = d.b;
-      T Vj = vj.w;  // V_j = X_j / sph_psi_j rides in vel_adv's 4th lane (pass A)
-      T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-      T r2 = dx * dx + dy * dy + dz * dz, r;
-      T g = f_grad(k, r2, &r);
-      T Ax = (vi.x - vj.x) * dx + (vi.y - vj.y) * dy + (vi.z - vj.z) * dz;
-      T s = fvis * Vj * g * Ax * f_rcp(k.eps + r2);  // W_lap, sph_util.py:40-43 (fast quotient)
-      s = ok ? s : T(0);
-      ax += s * dx;
-      ay += s * dy;
-      az += s * dz;
-      T t = ok ? -Vj * g : T(0);  // normal, sph.py:149
-      nx += t * dx;
-      ny += t * dy;
-      nz += t * dz;
-    };
-    // viscosity and normals are (f,f) only: the boundary list is not visited
-    sweep_lists_coop<kCoop, T, Rec2<T>>(
-        k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
-        [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
-        [&](int j) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
-    ax = group_sum<kCoop>(ax);
-    ay = group_sum<kCoop>(ay);
-    az = group_sum<kCoop>(az);
-    nx = group_sum<kCoop>(nx);
-    ny = group_sum<kCoop>(ny);
-    nz = group_sum<kCoop>(nz);
-    if (c != 0) continue;
-    // SPH_vel_adv_2_vel; the spare lane keeps V_i until the tail writes 0:
-    // the adjoint's tape of this velocity carries it to the reverse sweep
-    vel[i] = vi;
-    acce_adv[i] = V4<T>{k.g[0] + ax, k.g[1] + ay, k.g[2] + az, T(0)};
-    if (k.gamma != T(0) || k.st_rec) {
-      // the records the surface-tension walks gather per candidate j: the
-      // normal's spare lane carries +-psi_j, negative where j's 0.99 gate
-      // fails (psi_j > 0 for every particle in a cell: its own W(0) term),
-      // and the forward walk's (x_j, m_j) goes to strec, so that it loads two
-      // records instead of five
-      const T psi = psi_rho[i];
-      normal[i] = V4<T>{nx * k.h, ny * k.h, nz * k.h, vf[(long)i * k.P] > T(0.99) ? psi : -psi};
-      strec[i] = V4<T>{p.x, p.y, p.z, fmass[i]};
-    } else {
-      normal[i] = V4<T>{nx * k.h, ny * k.h, nz * k.h, T(0)};
-    }
+  const int i = coop_particle<kCoop>(coop_sub(blk));
+  if (i >= n) return;
+  const V4<T> p = fpos[i];
+  const V4<T> vi = vadv[i];
+  const T fvis = k.two_d2 * mu_of(k, vf, i) / rdens[i];
+  T ax = 0, ay = 0, az = 0, nx = 0, ny = 0, nz = 0;  // this lane's share
+  auto term = [&](const Rec2<T>& d, bool ok) {
+    const V4<T>& q = d.a;
+    const V4<T>& vj = d.b;
+    T Vj = vj.w;  // V_j = X_j / sph_psi_j rides in vel_adv's 4th lane (pass A)
+    T dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+    T r2 = dx * dx + dy * dy + dz * dz, r;
+    T g = f_grad(k, r2, &r);
+    T Ax = (vi.x - vj.x) * dx + (vi.y - vj.y) * dy + (vi.z - vj.z) * dz;
+    T s = fvis * Vj * g * Ax * f_rcp(k.eps + r2);  // W_lap, sph_util.py:40-43 (fast quotient)
+    s = ok ? s : T(0);
+    ax += s * dx;
+    ay += s * dy;
+    az += s * dz;
+    T t = ok ? -Vj * g : T(0);  // normal, sph.py:149
+    nx += t * dx;
+    ny += t * dy;
+    nz += t * dz;
+  };
+  // viscosity and normals are (f,f) only: the boundary list is not visited
+  sweep_lists_coop<kCoop, T, Rec2<T>, GROUP ? group_nb<T, Rec2<T>, 1>(3) : kCoopNb,
+                     GROUP ? group_nb<T, Rec2<T>, 1>(2) : kCoopNb>(
+      k, cap, i, c, p, fstart, bstart, fpos, bpos, nbr_f, nullptr, nbr_nf[i], 0,
+      [&](int j) { return Rec2<T>{fpos[j], vadv[j]}; },
+      [&](int j) { return Rec2<T>{}; }, term, [&](const Rec2<T>&, bool) {});
+  ax = group_sum<kCoop>(ax);
+  ay = group_sum<kCoop>(ay);
+  az = group_sum<kCoop>(az);
+  nx = group_sum<kCoop>(nx);
+  ny = group_sum<kCoop>(ny);
+  nz = group_sum<kCoop>(nz);
+  if (c != 0) return;
+  // SPH_vel_adv_2_vel; the spare lane keeps V_i until the tail writes 0:
+  // the adjoint's tape of this velocity carries it to the reverse sweep
+  vel[i] = vi;
+  acce_adv[i] = V4<T>{k.g[0] + ax, k.g[1] + ay, k.g[2] + az, T(0)};
+  if (k.gamma != T(0) || k.st_rec) {
+    // the records the surface-tension walks gather per candidate j: the
+    // normal's spare lane carries +-psi_j, negative where j's 0.99 gate
+    // fails (psi_j > 0 for every particle in a cell: its own W(0) term),
+    // and the forward walk's (x_j, m_j) goes to strec, so that it loads two
+    // records instead of five
+    const T psi = psi_rho[i];
+    normal[i] = V4<T>{nx * k.h, ny * k.h, nz * k.h, vf[(long)i * k.P] > T(0.99) ? psi : -psi};
+    strec[i] = V4<T>{p.x, p.y, p.z, fmass[i]};
+  } else {
+    normal[i] = V4<T>{nx * k.h, ny * k.h, nz * k.h, T(0)};
   }
 }
 
@@ -1815,11 +1815,11 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 template <class T, int R>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 5 : 1)  // R = 4: 96 registers, not 99
     kb_solver_psi(const char* __restrict__ tab, int ns, int kk) {
   for_coop_tiles<T, kCoop, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_solver_psi_body<T, R>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
+    k_solver_psi_body<T, R, true>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
                          (const V4<T>*)f.vel_adv, psi_of(e), (const T*)f.rest_density,
                          (const T*)f.alpha, f.cell_start, (const V4<T>*)e.b.pos, e.b.cell_start,
                          f.nbr_f, f.nbr_b, f.nbr_nf, f.nbr_nb, (T*)f.psi_adv, (T*)f.kappa,
@@ -1833,7 +1833,7 @@ __global__ void __launch_bounds__(kBlock)
     kb_solver_update(const char* __restrict__ tab, int ns, int kk) {
   for_coop_tiles<T, kCoopU, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_solver_update_body<T, R>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
+    k_solver_update_body<T, R, true>(blk, e.k, f.n, f.capacity, kk, (const V4<T>*)f.pos,
                             (const T*)f.mass, (const T*)f.kappa, (const V4<T>*)e.L.krec,
                             (const V4<T>*)f.alpha_1, f.cell_start,
                             (const V4<T>*)e.b.pos, e.b.cell_start, f.nbr_f, f.nbr_b, f.nbr_nf,
@@ -1841,11 +1841,11 @@ __global__ void __launch_bounds__(kBlock)
   });
 }
 
-template <class T, int R>
+template <class T>
 __global__ void __launch_bounds__(kBlock) kb_advect(const char* __restrict__ tab, int ns) {
-  for_coop_tiles<T, kCoop, R>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
+  for_coop_tiles<T, kCoop, 1>(tab, ns, [&](const SceneEntry<T>& e, Blk blk) {
     const TsphObject& f = e.f;
-    k_advect_body<T, R>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, (const T*)f.volume_frac,
+    k_advect_body<T, true>(blk, e.k, f.n, f.capacity, (const V4<T>*)f.pos, (const T*)f.volume_frac,
                      (const T*)f.rest_density, f.cell_start, e.b.cell_start,
                      (const V4<T>*)e.b.pos, f.nbr_f, f.nbr_nf, (V4<T>*)f.vel_adv, (V4<T>*)f.vel,
                      (V4<T>*)f.acce_adv, (V4<T>*)f.normal, (const T*)f.mass, psi_of(e),
@@ -1945,13 +1945,12 @@ int batch_solver_half(const TsphBatchInfo& bi, char* tab, int kk, int half, int 
   auto launch = [&](auto kern, int blocks) {
     hipLaunchKernelGGL(kern, dim3(grid_for(blocks, grid)), dim3(kBlock), 0, st, tab, bi.nscenes, kk);
   };
-  const bool split = coop_split(tiles);
   if (half & 1) {
-    if (split) launch(kb_solver_psi<T, 1>, tiles * kCoop);
+    if (psi_split<T>(tiles)) launch(kb_solver_psi<T, 1>, tiles * kCoop);
     else launch(kb_solver_psi<T, kCoop>, tiles);
   }
   if (half & 2) {
-    if (split) launch(kb_solver_update<T, 1>, tiles * kCoopU);
+    if (update_split<T>(tiles)) launch(kb_solver_update<T, 1>, tiles * kCoopU);
     else launch(kb_solver_update<T, kCoopU>, tiles);
   }
   TSPH_LAUNCH_CHECK("batch_solver_iteration");
@@ -1960,14 +1959,10 @@ int batch_solver_half(const TsphBatchInfo& bi, char* tab, int kk, int half, int 
 
 template <class T>
 int batch_advect(const TsphBatchInfo& bi, char* tab, int grid, hipStream_t st) {
-  const int g = grid_for(bi.tiles[kTileFluid], grid);
-  if (!g) return 0;
   const int tiles = bi.tiles[kTileFluid];
-  if (coop_split(tiles))
-    hipLaunchKernelGGL((kb_advect<T, 1>), dim3(grid_for(tiles * kCoop, grid)), dim3(kBlock), 0, st,
-                       tab, bi.nscenes);
-  else
-    hipLaunchKernelGGL((kb_advect<T, kCoop>), dim3(g), dim3(kBlock), 0, st, tab, bi.nscenes);
+  if (tiles <= 0) return 0;
+  hipLaunchKernelGGL(kb_advect<T>, dim3(grid_for(tiles * kCoop, grid)), dim3(kBlock), 0, st, tab,
+                     bi.nscenes);
   hipLaunchKernelGGL(kb_surface_tension<T>, dim3(grid_for(tiles * kQuad, grid)), dim3(kBlock), 0, st,
                      tab, bi.nscenes);
   TSPH_LAUNCH_CHECK("batch_advect");

@@ -135,6 +135,20 @@ struct Rec3 {
 constexpr int kCoop = 4;    // lanes per particle of the gather-heavy sweeps
 constexpr int kCoopU = 2;   // lanes per particle of the update sweep (one gather per pair)
 constexpr int kCoopNb = 4;  // gathers in flight per lane
+// In a grouped launch the scenes' constants take registers besides: fewer in flight in
+// FP64, for the waves, and in 2D, where the 12 neighbours (32 in 3D) take three slots
+// of each of four lanes.  (How many does not change a sum.)
+// us with 4 / 3 in flight, 24 2D scenes of 25-35k: psi 35.3 / 33.5, update 23.9 / 23.2,
+// advection (and velocity update) 43.6 / 41.2; 3D FP32 psi, 3 x 180k, 43.7 / 47.5.  FP64
+// with 4 / 3 / 2: psi 2D 901 tiles 27.1 / 23.8 / 23.0, 3D 908 tiles 40.8 / 38.2 / 35.1,
+// 2024 80.6 / 76.0 / 69.7, 19404 (R = 4) 742 / 787 / 784; advection 3D 908 44.5 / 46.0 /
+// 42.0, 2799 118 / 122 / 113, 19404 842 / 885 / 874; update with 4 / 3 2D 2798 36.7 / 34.9,
+// 3D 2799 66.9 / 62.1, 19404 472 / 491.
+template <class T, class Rec, int R>
+constexpr int group_nb(int dim) {
+  const bool two = sizeof(Rec) > sizeof(V4<T>);  // psi, advection; the update: one vector
+  return dim == 2 ? 3 : sizeof(T) == 4 ? 4 : !two ? 3 : R == 1 ? 2 : 4;
+}
 
 // A block covers kBlock / C particles, one per group: C rounds of as many
 // particles in a C-th of the blocks leave a small launch short of blocks and
@@ -163,15 +177,21 @@ __device__ __forceinline__ int coop_particle(int sub) {
 // Every scene's sweep in a grouped launch; f(entry, blk).  A block takes R of
 // a fluid tile's C sub-tiles: finding a tile's scene and its constants is a
 // chain of dependent loads, which R = C pays once per tile, while split tiles
-// leave no block waiting for its last round.  us of psi and surface tension,
-// split / whole, FP32 by tiles: 96 6.0 / 11.4 and 15 / 37, 500 13.6 / 15.6 and 39 /
-// 53, 1000 22.6 / 24.5 and 65 / 75, 2000 40.1 / 43.4 and 121 / 144, 2304 46.2 / 45.5
-// and 138 / 151, 3000 57.5 / 62.6 and 175 / 201; FP64 1060 48 / 55, 2544 108 / 104.
-// Where no scene has surface tension its launch is the update alone, 10.8 / 7.6 at
-// 2275 tiles, and whole steps from 700 tiles on take the same time either way (24
-// scenes 2275 tiles 782 / 782, 48 scenes 3584 tiles 1000 / 1003, 64 scenes 15734
-// tiles 4091 / 4094).  Tiles up to coop_split's line are split, as a single scene's
-// launch is; above it whole ones take fewer blocks for the same time.
+// (R = 1, as in a single scene's launch) leave no block waiting for its last round.
+//   Advection is split always, us with the velocity update, split / whole: 2D 2798
+// tiles 40.9 / 41.7, FP64 72.0 / 78.0, 19150 tiles FP64 531 / 579; 3D 2799 tiles 58.1 /
+// 61.3, FP64 117 / 126.
+//   Psi up to 2048 tiles, us split / whole: 3D 56 tiles 5.3 / 10.9, 908 20.8 / 21.5, 1440
+// 29.2 / 32.6, 2024 38.5 / 38.6, 2799 50.3 / 51.6, 19404 394 / 403; but 2D 1135 17.4 /
+// 15.8, 1428 21.0 / 22.3, 2026 27.6 / 25.5, 2360 31.1 / 27.3, 19150 256 / 228.  In FP64 up
+// to 3072: 3D 2338 83.6 / 92.1, 2799 99.6 / 104, 5555 223 / 220, 19404 767 / 740; 2D 2360
+// 52.7 / 54.5, 2798 61.0 / 61.2, 3471 76.0 / 75.0, 19150 455 / 428.
+//   The update while its blocks are about all on the chip at once: a scene's first block
+// sends the host the stop signal, and a block that waits for a place sends it late, so
+// that the next kernel comes late.  Steps, us split / whole: 3D 449 tiles 269 / 285, 602
+// 298 / 322, 908 358 / 348, 1440 445 / 437; FP64 218 291 / 294, 449 371 / 372, 676 445 /
+// 438, 760 462 / 449, 908 556 / 539, 2D 598 263 / 262, 671 274 / 271, 756 286 / 283 (the
+// kernel alone is the faster for being split: 760 tiles 20.2 / 20.5, 602 17.6 / 20.1).
 template <class T, int C, int R, class F>
 __device__ __forceinline__ void for_coop_tiles(const char* __restrict__ tab, int ns, F&& f) {
   constexpr int split = C / R;
@@ -181,8 +201,10 @@ __device__ __forceinline__ void for_coop_tiles(const char* __restrict__ tab, int
       f(e, Blk{tile.b * split + t % split, tile.nb * split});
     });
 }
-constexpr int kCoopTilesFull = 2048;  // fluid tiles that fill the 256 CUs eight times
-inline bool coop_split(int tiles) { return tiles < kCoopTilesFull; }
+template <class T>
+inline bool psi_split(int tiles) { return tiles < (sizeof(T) == 8 ? 3072 : 2048); }
+template <class T>
+inline bool update_split(int tiles) { return tiles < (sizeof(T) == 8 ? 512 : 896); }
 template <int C>
 __device__ __forceinline__ int coop_lane() {
   return threadIdx.x & (C - 1);
@@ -196,8 +218,8 @@ __device__ __forceinline__ T group_sum(T v) {
 
 // One list, lane c's share of it, NB gathers in flight per lane; the next trip's
 // list entries are loaded right after this one's records are requested, so that a
-// trip costs one round trip to memory instead of two (index, then record).  Every trip gathers NB records without a
-// branch: a slot past the list's end reads the last slot again (a line the
+// trip costs one round trip to memory instead of two (index, then record).  Every
+// trip gathers NB records without a branch: a slot past the list's end reads the last slot again (a line the
 // group holds already) and pair(record, false) leaves it out of the sums, so
 // that the loads of a trip issue back to back.  With a branch around each
 // load instead, a trip's loads went out one exec-mask change at a time: where
@@ -234,8 +256,8 @@ __device__ __forceinline__ void sweep_one_list_coop(int cap, int i, int c,
 // A particle's fluid list, then its boundary list, for lane c of its group.  A
 // particle whose list overflowed is swept by lane 0 alone, walking the cells with
 // the lists' in-range test.
-template <int C, class T, class Rec, int NB = kCoopNb, class LoadF, class LoadB, class PairF,
-          class PairB>
+template <int C, class T, class Rec, int NB = kCoopNb, int NB2D = NB, class LoadF, class LoadB,
+          class PairF, class PairB>
 __device__ __forceinline__ void sweep_lists_coop(const KP<T>& k, int cap, int i, int c, V4<T> p,
                                                  const int* __restrict__ fstart,
                                                  const int* __restrict__ bstart,
@@ -246,7 +268,10 @@ __device__ __forceinline__ void sweep_lists_coop(const KP<T>& k, int cap, int i,
                                                  LoadF&& load_f, LoadB&& load_b, PairF&& pair_f,
                                                  PairB&& pair_b) {
   if (nf <= k.list_cap_f && nbb <= k.list_cap_b) {
-    sweep_one_list_coop<C, Rec, NB>(cap, i, c, nbr_f, nf, load_f, pair_f);
+    if (NB2D != NB && k.dim == 2)
+      sweep_one_list_coop<C, Rec, NB2D>(cap, i, c, nbr_f, nf, load_f, pair_f);
+    else
+      sweep_one_list_coop<C, Rec, NB>(cap, i, c, nbr_f, nf, load_f, pair_f);
     if (nbb > 0) sweep_one_list_coop<C, Rec, NB>(cap, i, c, nbr_b, nbb, load_b, pair_b);
     return;
   }
@@ -543,7 +568,6 @@ __device__ __forceinline__ void sweep_list_as_quad(const KP<T>& k, int cap, int 
     for (int u = 0; u < NB; ++u) pair(u % kQuad, d[u], s + u < n);
   }
 }
-
 
 // The walk of an object in cell order around p, taking the candidates in range
 // (r^2 <= r2max).
