@@ -103,8 +103,8 @@ constexpr int kBsumU = 4;  // boundary candidates in flight per lane
 // FP64 14k 9.7 / 6.8, 98k 20.8 / 21.8.  The FP32 viscosity gathers four records
 // a pair and takes four lanes at every size in 3D: 14k 10.9 / 7.5, 216k 30.1 / 30.2,
 // 405k 53.0 / 49.0, 1M 139.9 / 124.2; FP64 14k 12.6 / 10.1, 98k 27.0 / 29.6.
-// In 2D, with some 20 neighbours to a particle, a trip of four lanes is half empty
-// at the list's end: two lanes from 96k on in FP32 (us, four / two: kappa 130k 10.5 /
+// In 2D, with 12 neighbours to a particle, a trip of four lanes is a quarter empty
+// (32 in 3D: none): two lanes from 96k on in FP32 (us, four / two: kappa 130k 10.5 /
 // 9.1, viscosity 130k 14.5 / 12.6, 300k 26.4 / 22.0, 1.2M 96 / 77), and in FP64 in pass
 // A's reverse too.  The surface tension's and the boundary sums' walks (rows of 12
 // candidates) then take one lane, us, quads / one: tension FP32 65k 13.0 / 18, 130k
